@@ -9,6 +9,7 @@
 // addressing and clamp-to-edge stencils.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <new>
 
@@ -81,167 +82,237 @@ __device__ __forceinline__ float d5(float m2, float m1, float p1, float p2)
     return t;
 }
 
-__global__ __launch_bounds__(256) void k_hs_warp(const float* __restrict__ I1, int w, int h, int s,
-                                                 const float* __restrict__ u,
-                                                 const float* __restrict__ v,
-                                                 float* __restrict__ out)
-{
-    const int ix = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int iy = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (ix >= w || iy >= h) return;
-    const size_t pos = (size_t)ix + (size_t)iy * s;
-    out[pos] = bilinear_at(I1, w, h, s, (float)ix + u[pos], (float)iy + v[pos]);
-}
+// Tile of the fused warp + derivatives kernel: kWdX x kWdY output pixels per
+// workgroup, the warped frame staged in LDS with the stencil's 2-pixel halo.
+constexpr int kWdX = 64, kWdY = 8, kWdH = 2;
 
-__global__ __launch_bounds__(256) void k_hs_derivatives(const float* __restrict__ I0,
-                                                        const float* __restrict__ I1w, int w,
-                                                        int h, int s, float* __restrict__ Ix,
+// Warp and derivatives in one launch: the workgroup warps its tile plus halo
+// into LDS (a halo position takes the clamped pixel's warp, which is what the
+// clamped stencil reads), then every thread forms the derivatives of two
+// pixels from LDS and I0.  A launch costs about as much as its memory traffic
+// at these sizes; one launch instead of two also drops the round trip of the
+// warped plane (1280x720: 3.2 + 3.5 us before).
+__global__ __launch_bounds__(256) void k_hs_warp_derivs(const float* __restrict__ I0,
+                                                        const float* __restrict__ I1, int w, int h,
+                                                        int s, const float* __restrict__ u,
+                                                        const float* __restrict__ v,
+                                                        float* __restrict__ Ix,
                                                         float* __restrict__ Iy,
-                                                        float* __restrict__ Iz)
+                                                        float* __restrict__ Iz,
+                                                        float* __restrict__ I1w_out)
 {
-    const int ix = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int iy = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (ix >= w || iy >= h) return;
-    const size_t pos = (size_t)ix + (size_t)iy * s;
-    const size_t row = (size_t)iy * s;
+    constexpr int PX = kWdX + 2 * kWdH, PY = kWdY + 2 * kWdH;
+    __shared__ float sw[PY][PX];
+    const int x0 = blockIdx.x * kWdX, y0 = blockIdx.y * kWdY;
+    for (int e = threadIdx.x; e < PX * PY; e += 256) {
+        const int py = e / PX, px = e - py * PX;
+        const int ix = clampi(x0 + px - kWdH, 0, w - 1), iy = clampi(y0 + py - kWdH, 0, h - 1);
+        const size_t pos = (size_t)ix + (size_t)iy * s;
+        sw[py][px] = bilinear_at(I1, w, h, s, (float)ix + u[pos], (float)iy + v[pos]);
+    }
+    __syncthreads();
+    const int lx = threadIdx.x & 63;
+    const int ix = x0 + lx;
+    if (ix >= w) return;
     const int xm2 = clampi(ix - 2, 0, w - 1), xm1 = clampi(ix - 1, 0, w - 1);
     const int xp1 = clampi(ix + 1, 0, w - 1), xp2 = clampi(ix + 2, 0, w - 1);
-    const size_t ym2 = (size_t)clampi(iy - 2, 0, h - 1) * s, ym1 = (size_t)clampi(iy - 1, 0, h - 1) * s;
-    const size_t yp1 = (size_t)clampi(iy + 1, 0, h - 1) * s, yp2 = (size_t)clampi(iy + 2, 0, h - 1) * s;
-    float t0 = d5(I0[row + xm2], I0[row + xm1], I0[row + xp1], I0[row + xp2]);
-    float t1 = d5(I1w[row + xm2], I1w[row + xm1], I1w[row + xp1], I1w[row + xp2]);
-    Ix[pos] = (t0 + t1) * 0.5f;
-    Iz[pos] = I1w[pos] - I0[pos];
-    t0 = d5(I0[ym2 + ix], I0[ym1 + ix], I0[yp1 + ix], I0[yp2 + ix]);
-    t1 = d5(I1w[ym2 + ix], I1w[ym1 + ix], I1w[yp1 + ix], I1w[yp2 + ix]);
-    Iy[pos] = (t0 + t1) * 0.5f;
+#pragma unroll
+    for (int k = 0; k < kWdY / 4; k++) {
+        const int ly = (threadIdx.x >> 6) + 4 * k;
+        const int iy = y0 + ly;
+        if (iy >= h) return;
+        const size_t row = (size_t)iy * s, pos = row + ix;
+        const size_t ym2 = (size_t)clampi(iy - 2, 0, h - 1) * s, ym1 = (size_t)clampi(iy - 1, 0, h - 1) * s;
+        const size_t yp1 = (size_t)clampi(iy + 1, 0, h - 1) * s, yp2 = (size_t)clampi(iy + 2, 0, h - 1) * s;
+        const float* c = &sw[ly + kWdH][lx + kWdH];
+        const float t0 = d5(I0[row + xm2], I0[row + xm1], I0[row + xp1], I0[row + xp2]);
+        const float t1 = d5(c[-2], c[-1], c[1], c[2]);
+        Ix[pos] = (t0 + t1) * 0.5f;
+        Iz[pos] = c[0] - I0[pos];
+        const float r0 = d5(I0[ym2 + ix], I0[ym1 + ix], I0[yp1 + ix], I0[yp2 + ix]);
+        const float r1 = d5(c[-2 * PX], c[-PX], c[PX], c[2 * PX]);
+        Iy[pos] = (r0 + r1) * 0.5f;
+        if (I1w_out) I1w_out[pos] = c[0];
+    }
 }
 
-// Waves per workgroup of the Jacobi kernel.  Eight waves of R rows hide the
-// latency of a sweep better than four of 2R: at 640x480 with 4 sweeps per
-// launch, 8 waves x 4 rows took 0.174 ms for 100 sweeps, 4 waves x 8 rows
-// 0.198 ms and 4 waves x 4 rows 0.217 ms.
-constexpr int kHsWaves = 8;
+// One launch of Jacobi sweeps (solverKernel.cuh:39-153): `kk` sweeps (at most
+// the halo K) of every pixel.
+struct JacobiArgs {
+    const float *du0, *dv0;        // input increments
+    const float *Ix, *Iy, *Iz;
+    float *du1, *dv1;              // output increments; unused with `u` set
+    float *u, *v;                  // set on a warping's last launch: u += du, v += dv
+    int w, h, s;
+    float alpha;
+    int K, kk;
+    int zero_in;                   // the input increments are all zero
+};
 
-// K Jacobi sweeps (solverKernel.cuh:39-153) per launch.  Layout as in the
-// TV-L1 iteration kernel, with kHsWaves waves: each lane a column of R rows
-// held in registers, horizontal neighbours by lane shuffles, vertical ones
-// from registers or one LDS row per wave (double-buffered: one barrier per
-// sweep).  Values within K pixels of the tile edge go stale one pixel per
-// sweep; the central (64-2K) x (8R-2K) pixels are stored.  `zero_in`: the
-// input increments are all zero (first launch of a warping).
-
-template <int K, int R>
-__global__ __launch_bounds__(64 * kHsWaves) void k_hs_jacobi(const float* __restrict__ du0,
-                                                   const float* __restrict__ dv0,
-                                                   const float* __restrict__ Ix,
-                                                   const float* __restrict__ Iy,
-                                                   const float* __restrict__ Iz, int w, int h,
-                                                   int s, float alpha, int kk, int zero_in,
-                                                   float* __restrict__ du1,
-                                                   float* __restrict__ dv1)
+// Lane shifts with zero in the lane that has no source (its pixel is never
+// stored): without a value to keep, the shift folds into the addition.
+__device__ __forceinline__ float lane_left(float v)
 {
-    constexpr int NW = kHsWaves;
-    constexpr int TW = 64 - 2 * K;
-    constexpr int TH = NW * R - 2 * K;
-    __shared__ float sh_first[2][2][NW][64];   // [buf][u/v][wave][lane]: row 0 of each wave
-    __shared__ float sh_last[2][2][NW][64];    // row R-1 of each wave
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138 /* wave_shr:1 */, 0xf, 0xf, true));
+}
 
+__device__ __forceinline__ float lane_right(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
+}
+
+// 1/d of a float in double, to about an ulp: the hardware reciprocal and two
+// Newton steps.  0, infinite and NaN divisors give garbage (div_by fixes it).
+__device__ __forceinline__ double recip_f64(double d)
+{
+    double y = __builtin_amdgcn_rcp(d);
+    y = __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+    return __builtin_fma(__builtin_fma(-d, y, 1.0), y, y);
+}
+
+// The IEEE float quotient n / d from d's double reciprocal y = recip_f64(d),
+// for a divisor that stays while the numerators change: 6 instructions
+// instead of the 11 of the division sequence.  The corrected double quotient
+// is exact where n / d has at most 53 bits (so also on every float rounding
+// boundary, subnormal ones included) and otherwise within 2^-52 of n / d,
+// which is never within 2^-49 of a boundary: rounding it gives the IEEE
+// quotient.  v_div_fixup supplies the special values.
+__device__ __forceinline__ float div_by(float n, float d, double dd, double y)
+{
+    const double nd = (double)n;
+    double q = nd * y;
+    q = __builtin_fma(__builtin_fma(-q, dd, nd), y, q);
+    return __builtin_amdgcn_div_fixupf((float)q, d, n);
+}
+
+// K sweeps per launch (the halo) on tiles of 64 columns (one per lane) by
+// NW*R rows (R consecutive rows per wave, in registers); horizontal
+// neighbours by lane shifts, vertical ones from registers or one LDS row per
+// wave (double-buffered: one barrier per sweep).  Values within K pixels of
+// the tile edge go stale one pixel per sweep; the central (64-2K) x (NW*R-2K)
+// pixels are stored.
+// Left and right of the image the tile holds the mirrored columns.  They stay
+// the mirror image sweep after sweep (left + right commutes bit for bit), so
+// the neighbour across the border is the clamped one without a select.  Up
+// and down do not commute in the sum: tiles that reach the first or last row
+// (EDGE) take selects there.
+template <int R, int NW, bool EDGE>
+__device__ __forceinline__ void jacobi_tile(const JacobiArgs& a, float (*sh)[4][NW][64])
+{
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int w = a.w, h = a.h, K = a.K;
+    const int TW = 64 - 2 * K, TH = NW * R - 2 * K;
     const int x = (int)blockIdx.x * TW - K + lane;
-    const int ybase = (int)blockIdx.y * TH - K + wave * R;
     const int oy0 = (int)blockIdx.y * TH;
-    const bool xin = x >= 0 && x < w;
-    const bool xout = xin && lane >= K && lane < K + TW;
-    const bool fc = x <= 0, lc = x >= w - 1;
+    const int ybase = oy0 - K + wave * R;
+    int xm = x;
+    if (xm < 0 || xm >= w) {
+        xm %= 2 * w;
+        if (xm < 0) xm += 2 * w;
+        if (xm >= w) xm = 2 * w - 1 - xm;
+    }
 
     float u[R], v[R], gx[R], gy[R], gz[R], den[R];
+    double dd[R], rd[R];
 #pragma unroll
     for (int r = 0; r < R; r++) {
         const int y = ybase + r;
-        if (xin && y >= 0 && y < h) {
-            const size_t p = (size_t)y * s + x;
-            u[r] = zero_in ? 0.0f : du0[p];
-            v[r] = zero_in ? 0.0f : dv0[p];
-            gx[r] = Ix[p];
-            gy[r] = Iy[p];
-            gz[r] = Iz[p];
-        } else {
-            u[r] = v[r] = gx[r] = gy[r] = gz[r] = 0.0f;
+        u[r] = v[r] = gx[r] = gy[r] = gz[r] = 0.0f;
+        if (!EDGE || (y >= 0 && y < h)) {
+            const size_t p = (size_t)y * a.s + xm;
+            gx[r] = a.Ix[p];
+            gy[r] = a.Iy[p];
+            gz[r] = a.Iz[p];
+            if (!a.zero_in) {
+                u[r] = a.du0[p];
+                v[r] = a.dv0[p];
+            }
         }
-        den[r] = (gx[r] * gx[r] + gy[r] * gy[r]) + alpha;
+    }
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        den[r] = (gx[r] * gx[r] + gy[r] * gy[r]) + a.alpha;
+        dd[r] = (double)den[r];
+        rd[r] = recip_f64(dd[r]);
     }
 
-#pragma unroll 1
-    for (int t = 0; t < kk; t++) {
-        const int b = t & 1;
-        sh_first[b][0][wave][lane] = u[0];
-        sh_first[b][1][wave][lane] = v[0];
-        sh_last[b][0][wave][lane] = u[R - 1];
-        sh_last[b][1][wave][lane] = v[R - 1];
+    // the outermost waves read their own rows: stale, never stored
+    const int wu = wave < NW - 1 ? wave + 1 : wave, wd = wave ? wave - 1 : wave;
+    auto sweep = [&](float(*b)[NW][64]) {
+        b[0][wave][lane] = u[0];
+        b[1][wave][lane] = v[0];
+        b[2][wave][lane] = u[R - 1];
+        b[3][wave][lane] = v[R - 1];
+        // left + right of every row while the LDS rows travel
+        float hu[R], hv[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            hu[r] = lane_left(u[r]) + lane_right(u[r]);
+            hv[r] = lane_left(v[r]) + lane_right(v[r]);
+        }
         __syncthreads();
-        const float upU = wave < NW - 1 ? sh_first[b][0][wave + 1][lane] : u[R - 1];
-        const float upV = wave < NW - 1 ? sh_first[b][1][wave + 1][lane] : v[R - 1];
-        const float dnU = wave ? sh_last[b][0][wave - 1][lane] : u[0];
-        const float dnV = wave ? sh_last[b][1][wave - 1][lane] : v[0];
-        float nu[R], nv[R];
+        const float upU = b[0][wu][lane], upV = b[1][wu][lane];
+        float du = b[2][wd][lane], dv = b[3][wd][lane];
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int y = ybase + r;
-            const float lu = from_left(u[r]), lv = from_left(v[r]);
-            const float ru = from_right(u[r]), rv = from_right(v[r]);
-            const float left_u = fc ? u[r] : lu, left_v = fc ? v[r] : lv;
-            const float right_u = lc ? u[r] : ru, right_v = lc ? v[r] : rv;
+            const bool top = EDGE && y <= 0, bottom = EDGE && y >= h - 1;
+            const float cu = u[r], cv = v[r];
+            const float uu = r < R - 1 ? u[r + 1] : upU, uv = r < R - 1 ? v[r + 1] : upV;
             // "up" is row y+1 and "down" row y-1, clamped at the image edge
-            const float up_u = (y >= h - 1) ? u[r] : (r < R - 1 ? u[r + 1] : upU);
-            const float up_v = (y >= h - 1) ? v[r] : (r < R - 1 ? v[r + 1] : upV);
-            const float dn_u = (y <= 0) ? u[r] : (r > 0 ? u[r - 1] : dnU);
-            const float dn_v = (y <= 0) ? v[r] : (r > 0 ? v[r - 1] : dnV);
-            const float sumU = (((left_u + right_u) + up_u) + dn_u) * 0.25f;
-            const float sumV = (((left_v + right_v) + up_v) + dn_v) * 0.25f;
-            const float frac = ((gx[r] * sumU + gy[r] * sumV) + gz[r]) / den[r];
-            nu[r] = sumU - gx[r] * frac;
-            nv[r] = sumV - gy[r] * frac;
+            const float sumU = ((hu[r] + (bottom ? cu : uu)) + (top ? cu : du)) * 0.25f;
+            const float sumV = ((hv[r] + (bottom ? cv : uv)) + (top ? cv : dv)) * 0.25f;
+            const float frac = div_by((gx[r] * sumU + gy[r] * sumV) + gz[r], den[r], dd[r], rd[r]);
+            u[r] = sumU - gx[r] * frac;
+            v[r] = sumV - gy[r] * frac;
+            du = cu;
+            dv = cv;
         }
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            u[r] = nu[r];
-            v[r] = nv[r];
-        }
+    };
+    // two sweeps per trip: the LDS buffer of each is known at compile time
+#pragma unroll 1
+    for (int t = 0; t < a.kk; t += 2) {
+        sweep(sh[0]);
+        if (t + 1 < a.kk) sweep(sh[1]);
     }
-    if (xout) {
+    if (!(x >= 0 && x < w && lane >= K && lane < K + TW)) return;
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int y = ybase + r;
-            if (y >= oy0 && y < oy0 + TH && y < h) {
-                const size_t p = (size_t)y * s + x;
-                du1[p] = u[r];
-                dv1[p] = v[r];
+    for (int r = 0; r < R; r++) {
+        const int y = ybase + r;
+        if (y >= oy0 && y < oy0 + TH && (!EDGE || y < h)) {
+            const size_t p = (size_t)y * a.s + x;
+            if (a.u) {
+                a.u[p] = a.u[p] + u[r];
+                a.v[p] = a.v[p] + v[r];
+            } else {
+                a.du1[p] = u[r];
+                a.dv1[p] = v[r];
             }
         }
     }
 }
 
-__global__ __launch_bounds__(256) void k_hs_add(float* __restrict__ u, const float* __restrict__ du,
-                                                float* __restrict__ v, const float* __restrict__ dv,
-                                                int w, int h, int s)
+template <int R, int NW>
+__global__ __launch_bounds__(64 * NW) void k_hs_jacobi(JacobiArgs a)
 {
-    const int ix = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int iy = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (ix >= w || iy >= h) return;
-    const size_t p = (size_t)ix + (size_t)iy * s;
-    u[p] = u[p] + du[p];
-    v[p] = v[p] + dv[p];
+    __shared__ float sh[2][4][NW][64];   // [buffer][first u, first v, last u, last v][wave][lane]
+    const int y0 = (int)blockIdx.y * (NW * R - 2 * a.K) - a.K;
+    if (y0 >= 1 && y0 + NW * R - 1 <= a.h - 2) jacobi_tile<R, NW, false>(a, sh);
+    else jacobi_tile<R, NW, true>(a, sh);
 }
 
-__global__ __launch_bounds__(256) void k_hs_zero(float* __restrict__ a, float* __restrict__ b,
-                                                 size_t n)
+// Frames in and flow cleared, or flow out: two planes copied (a1 may be
+// null: that pair is not copied) and two cleared, in one launch.
+__global__ __launch_bounds__(256) void k_hs_copy2(const float* a0, float* a1, const float* b0, float* b1,
+                                                  float* z0, float* z1, size_t n)
 {
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
          i += (size_t)gridDim.x * blockDim.x) {
-        a[i] = 0.0f;
-        b[i] = 0.0f;
+        if (a1) a1[i] = a0[i];
+        if (b1) b1[i] = b0[i];
+        if (z0) z0[i] = 0.0f;
+        if (z1) z1[i] = 0.0f;
     }
 }
 
@@ -256,6 +327,10 @@ inline dim3 grid2d(int w, int h) { return dim3(cdiv(w, 64), cdiv(h, 4)); }
         }                                                   \
     } while (0)
 
+// Waves per workgroup of the shapes set by of_hs_set_jacobi_shape: 64 x 8R
+// pixel tiles.
+constexpr int kHsWaves = 8;
+
 bool jacobi_shape_ok(int K, int R)
 {
     if (!(K == 1 || K == 2 || K == 4 || K == 8)) return false;
@@ -263,48 +338,51 @@ bool jacobi_shape_ok(int K, int R)
     return kHsWaves * R - 2 * K >= 4;
 }
 
-template <int K, int R>
-int launch_jacobi_kr(const float* du0, const float* dv0, const float* Ix, const float* Iy,
-                     const float* Iz, int w, int h, int s, float alpha, int kk, int zero_in,
-                     float* du1, float* dv1, hipStream_t st)
+// A launch shape: sweeps per launch (the halo), rows per wave, waves.
+struct JacobiShape {
+    int K, R, NW;
+};
+
+template <int R, int NW>
+int launch_jacobi_rn(const JacobiArgs& a, hipStream_t st)
 {
-    const dim3 g(cdiv(w, 64 - 2 * K), cdiv(h, kHsWaves * R - 2 * K));
-    hipLaunchKernelGGL((k_hs_jacobi<K, R>), g, dim3(64 * kHsWaves), 0, st, du0, dv0, Ix, Iy, Iz, w, h, s,
-                       alpha, kk, zero_in, du1, dv1);
+    const dim3 g(cdiv(a.w, 64 - 2 * a.K), cdiv(a.h, NW * R - 2 * a.K));
+    hipLaunchKernelGGL((k_hs_jacobi<R, NW>), g, dim3(64 * NW), 0, st, a);
     HS_CHECK("k_hs_jacobi");
     return OF_OK;
 }
 
-int launch_jacobi(int K, int R, const float* du0, const float* dv0, const float* Ix,
-                  const float* Iy, const float* Iz, int w, int h, int s, float alpha, int kk,
-                  int zero_in, float* du1, float* dv1, hipStream_t st)
+int launch_jacobi(const JacobiShape& t, const JacobiArgs& a, hipStream_t st)
 {
-#define HS_CASE(k, r)                                                                           \
-    if (K == k && R == r)                                                                       \
-        return launch_jacobi_kr<k, r>(du0, dv0, Ix, Iy, Iz, w, h, s, alpha, kk, zero_in, du1, \
-                                      dv1, st);
-    HS_CASE(1, 2) HS_CASE(2, 2) HS_CASE(1, 4) HS_CASE(2, 4) HS_CASE(4, 4)
-    HS_CASE(1, 8) HS_CASE(2, 8) HS_CASE(4, 8) HS_CASE(8, 8)
+    if (t.K < 1 || 2 * t.K >= 64 || 2 * t.K >= t.R * t.NW || a.kk > t.K) return OF_ERR_ARG;
+#define HS_CASE(r, n) \
+    if (t.R == r && t.NW == n) return launch_jacobi_rn<r, n>(a, st);
+    HS_CASE(2, 8) HS_CASE(4, 8) HS_CASE(8, 8) HS_CASE(2, 16) HS_CASE(3, 16)
 #undef HS_CASE
     return OF_ERR_UNSUPPORTED;
 }
 
-// n Jacobi sweeps from (du0,dv0) (or from zero) with launches of K sweeps;
-// returns the buffer index (0: du0/dv0, 1: du1/dv1) holding the result.
-int run_jacobi(int K, int R, float* du[2], float* dv[2], const float* Ix, const float* Iy,
-               const float* Iz, int w, int h, int s, float alpha, int n, bool zero_first,
-               int* result, hipStream_t st)
+// n Jacobi sweeps from (du0,dv0) (or from zero).  With u/v the last launch
+// adds the increments to them; otherwise *result names the buffer holding
+// the result (0: du[0]/dv[0], 1: du[1]/dv[1]).
+int run_jacobi(const JacobiShape& t, JacobiArgs a, float* du[2], float* dv[2], int n, bool zero_first,
+               float* u, float* v, int* result, hipStream_t st)
 {
     int cur = 0;
-    bool zero = zero_first;
-    int done = 0;
-    while (done < n) {
-        const int kk = (n - done) < K ? (n - done) : K;
-        OF_TRY(launch_jacobi(K, R, du[cur], dv[cur], Ix, Iy, Iz, w, h, s, alpha, kk, zero ? 1 : 0,
-                             du[cur ^ 1], dv[cur ^ 1], st));
-        zero = false;
+    a.K = t.K;
+    a.zero_in = zero_first ? 1 : 0;
+    for (int done = 0; done < n;) {
+        a.kk = (n - done) < t.K ? (n - done) : t.K;
+        done += a.kk;
+        a.du0 = du[cur];
+        a.dv0 = dv[cur];
+        a.du1 = du[cur ^ 1];
+        a.dv1 = dv[cur ^ 1];
+        a.u = done == n ? u : nullptr;
+        a.v = done == n ? v : nullptr;
+        OF_TRY(launch_jacobi(t, a, st));
+        a.zero_in = 0;
         cur ^= 1;
-        done += kk;
     }
     *result = cur;
     return OF_OK;
@@ -323,9 +401,9 @@ struct of_hs {
     int pW[32]{}, pH[32]{}, pS[32]{};
     float *u = nullptr, *v = nullptr, *nu = nullptr, *nv = nullptr;
     float *du[2]{}, *dv[2]{};
-    float *Ix = nullptr, *Iy = nullptr, *Iz = nullptr, *tmp = nullptr;
+    float *Ix = nullptr, *Iy = nullptr, *Iz = nullptr;
     float *hin0 = nullptr, *hin1 = nullptr;   // device staging of host inputs
-    int K = 4, R = 4;                         // Jacobi launch shape
+    int K = 0, R = 0;                         // Jacobi launch shape set by the caller; 0: by frame size
 };
 
 namespace {
@@ -341,10 +419,39 @@ void hs_release(of_hs* h)
     delete[] h->pI1;
     dev_free(h->u); dev_free(h->v); dev_free(h->nu); dev_free(h->nv);
     dev_free(h->du[0]); dev_free(h->du[1]); dev_free(h->dv[0]); dev_free(h->dv[1]);
-    dev_free(h->Ix); dev_free(h->Iy); dev_free(h->Iz); dev_free(h->tmp);
+    dev_free(h->Ix); dev_free(h->Iy); dev_free(h->Iz);
     dev_free(h->hin0); dev_free(h->hin1);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
+}
+
+// The launch shape of a level: the caller's, or the cheapest of 64x32 and
+// 64x48 tiles with 1..14 sweeps per launch.  A sweep is bound by VALU issue
+// (26 instructions per pixel of the tile, halo included), a launch adds its ramp and, per round of 256 workgroups, the loads and
+// stores; deep blocks amortise those, small halos save work, and the grid
+// quantises to rounds of the 256 CUs.  The model (us): 1.5 per launch, per
+// round 1.5 + 0.010 per tile row and sweep.  Over 79x44 .. 1920x1080 it
+// picks within 8% of the fastest of 46 measured shapes (64x64 and 8-wave
+// tiles among them), e.g. 120 sweeps (us; 64x32 tiles with 4 sweeps per
+// launch in parentheses): 79x44 83 (152), 638x359 127 (185), 640x480 151
+// (190), 1277x719 282 (331), 1920x1080 490 (607).
+JacobiShape pick_shape(const of_hs* h, int w, int hh, int sweeps)
+{
+    if (h->K) return JacobiShape{h->K, h->R, kHsWaves};
+    JacobiShape best{4, 2, 16};
+    double best_us = 0.0;
+    for (int R = 2; R <= 3; R++)
+        for (int K = 1; K <= 14 && K <= std::max(sweeps, 1); K++) {
+            const int rows = 16 * R;
+            const double launches = (sweeps + K - 1) / K;
+            const double rounds = cdiv((size_t)cdiv(w, 64 - 2 * K) * cdiv(hh, rows - 2 * K), 256);
+            const double us = launches * (1.5 + 1.5 * rounds) + 0.010 * rows * rounds * sweeps;
+            if (best_us == 0.0 || us < best_us) {
+                best_us = us;
+                best = JacobiShape{K, R, 16};
+            }
+        }
+    return best;
 }
 
 // ComputeFlow, src/hs/cuda/flow.cu:112-208, from device frames (stride s).
@@ -357,8 +464,10 @@ int hs_solve(of_hs* h, const float* dI0, const float* dI1, int width, int height
     if (nWarpIters < 0 || nSolverIters < 0) return OF_ERR_ARG;
     const size_t fsize = (size_t)stride * height;
     int L = nLevels - 1;
-    OF_HIP(hipMemcpyAsync(h->pI0[L], dI0, fsize * sizeof(float), hipMemcpyDeviceToDevice, st));
-    OF_HIP(hipMemcpyAsync(h->pI1[L], dI1, fsize * sizeof(float), hipMemcpyDeviceToDevice, st));
+    const unsigned blocks = cdiv(fsize, 256) > 2048 ? 2048 : cdiv(fsize, 256);
+    hipLaunchKernelGGL(k_hs_copy2, dim3(blocks), dim3(256), 0, st, dI0, h->pI0[L], dI1, h->pI1[L], h->u,
+                       h->v, fsize);
+    HS_CHECK("k_hs_copy2");
     for (; L > 0; --L) {
         hipLaunchKernelGGL(k_hs_downscale, grid2d(h->pW[L - 1], h->pH[L - 1]), dim3(256), 0, st,
                            h->pI0[L], h->pS[L], h->pI0[L - 1], h->pW[L - 1], h->pH[L - 1], h->pS[L - 1]);
@@ -367,26 +476,24 @@ int hs_solve(of_hs* h, const float* dI0, const float* dI1, int width, int height
                            h->pI1[L], h->pS[L], h->pI1[L - 1], h->pW[L - 1], h->pH[L - 1], h->pS[L - 1]);
         HS_CHECK("k_hs_downscale");
     }
-    hipLaunchKernelGGL(k_hs_zero, dim3(cdiv(fsize, 256) > 2048 ? 2048 : cdiv(fsize, 256)), dim3(256),
-                       0, st, h->u, h->v, fsize);
-    HS_CHECK("k_hs_zero");
     for (L = 0; L < nLevels; ++L) {
         const int w = h->pW[L], hh = h->pH[L], s = h->pS[L];
         for (int wi = 0; wi < nWarpIters; ++wi) {
-            hipLaunchKernelGGL(k_hs_warp, grid2d(w, hh), dim3(256), 0, st, h->pI1[L], w, hh, s, h->u,
-                               h->v, h->tmp);
-            HS_CHECK("k_hs_warp");
-            hipLaunchKernelGGL(k_hs_derivatives, grid2d(w, hh), dim3(256), 0, st, h->pI0[L], h->tmp,
-                               w, hh, s, h->Ix, h->Iy, h->Iz);
-            HS_CHECK("k_hs_derivatives");
+            hipLaunchKernelGGL(k_hs_warp_derivs, dim3(cdiv(w, kWdX), cdiv(hh, kWdY)), dim3(256), 0, st,
+                               h->pI0[L], h->pI1[L], w, hh, s, h->u, h->v, h->Ix, h->Iy, h->Iz,
+                               (float*)nullptr);
+            HS_CHECK("k_hs_warp_derivs");
             int res = 0;
-            if (nSolverIters > 0) {
-                OF_TRY(run_jacobi(h->K, h->R, h->du, h->dv, h->Ix, h->Iy, h->Iz, w, hh, s, alpha,
-                                  nSolverIters, true, &res, st));
-                hipLaunchKernelGGL(k_hs_add, grid2d(w, hh), dim3(256), 0, st, h->u, h->du[res],
-                                   h->v, h->dv[res], w, hh, s);
-                HS_CHECK("k_hs_add");
-            }
+            JacobiArgs a{};
+            a.Ix = h->Ix;
+            a.Iy = h->Iy;
+            a.Iz = h->Iz;
+            a.w = w;
+            a.h = hh;
+            a.s = s;
+            a.alpha = alpha;
+            OF_TRY(run_jacobi(pick_shape(h, w, hh, nSolverIters), a, h->du, h->dv, nSolverIters, true,
+                              h->u, h->v, &res, st));
         }
         if (L != nLevels - 1) {
             const float scaleX = (float)h->pW[L + 1] / (float)h->pW[L];
@@ -402,8 +509,11 @@ int hs_solve(of_hs* h, const float* dI0, const float* dI1, int width, int height
         }
     }
     // the result is in h->u/h->v, which the level loop swaps with nu/nv
-    if (du_out) OF_HIP(hipMemcpyAsync(du_out, h->u, fsize * sizeof(float), hipMemcpyDeviceToDevice, st));
-    if (dv_out) OF_HIP(hipMemcpyAsync(dv_out, h->v, fsize * sizeof(float), hipMemcpyDeviceToDevice, st));
+    if (du_out && dv_out) {
+        hipLaunchKernelGGL(k_hs_copy2, dim3(blocks), dim3(256), 0, st, h->u, du_out, h->v, dv_out,
+                           (float*)nullptr, (float*)nullptr, fsize);
+        HS_CHECK("k_hs_copy2");
+    }
     OF_HIP(hipStreamSynchronize(st));
     return OF_OK;
 }
@@ -448,7 +558,7 @@ int of_hs_create(int nLevels, int stride, int width, int height, of_hs** out)
         if (!st) st = dev_alloc(&h->pI1[L], n);
     }
     float** bufs[] = {&h->u, &h->v, &h->nu, &h->nv, &h->du[0], &h->du[1], &h->dv[0], &h->dv[1],
-                      &h->Ix, &h->Iy, &h->Iz, &h->tmp, &h->hin0, &h->hin1};
+                      &h->Ix, &h->Iy, &h->Iz, &h->hin0, &h->hin1};
     for (float** b : bufs)
         if (!st) st = dev_alloc(b, fsize);
     if (st) { hs_release(h); return st; }
@@ -530,7 +640,15 @@ int of_dbg_hs_jacobi(const float* du, const float* dv, const float* Ix, const fl
     int res = 0;
     float* dus[2] = {b[0], b[5]};
     float* dvs[2] = {b[1], b[6]};
-    if (!st) st = run_jacobi(K, R, dus, dvs, b[2], b[3], b[4], w, h, w, alpha, iters, false, &res, nullptr);
+    JacobiArgs a{};
+    a.Ix = b[2];
+    a.Iy = b[3];
+    a.Iz = b[4];
+    a.w = w;
+    a.h = h;
+    a.s = w;
+    a.alpha = alpha;
+    if (!st) st = run_jacobi(JacobiShape{K, R, kHsWaves}, a, dus, dvs, iters, false, nullptr, nullptr, &res, nullptr);
     if (!st && hipMemcpy(du_out, dus[res], n * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess) st = OF_ERR_HIP;
     if (!st && hipMemcpy(dv_out, dvs[res], n * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess) st = OF_ERR_HIP;
     for (float*& p : b) dev_free(p);
@@ -550,9 +668,8 @@ int of_dbg_hs_warp_derivatives(const float* I0, const float* I1, const float* u,
     for (int i = 0; i < 4 && !st; i++)
         if (hipMemcpy(b[i], src[i], n * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) st = OF_ERR_HIP;
     if (!st) {
-        hipLaunchKernelGGL(k_hs_warp, grid2d(w, h), dim3(256), 0, nullptr, b[1], w, h, w, b[2], b[3], b[4]);
-        hipLaunchKernelGGL(k_hs_derivatives, grid2d(w, h), dim3(256), 0, nullptr, b[0], b[4], w, h, w,
-                           b[5], b[6], b[7]);
+        hipLaunchKernelGGL(k_hs_warp_derivs, dim3(cdiv(w, kWdX), cdiv(h, kWdY)), dim3(256), 0, nullptr, b[0],
+                           b[1], w, h, w, b[2], b[3], b[5], b[6], b[7], b[4]);
         if (hipGetLastError() != hipSuccess) st = OF_ERR_HIP;
     }
     float* dst[4] = {I1w, Ix, Iy, Iz};

@@ -95,6 +95,40 @@ def test_hs_multilevel_strided_matches_oracle(shape):
     assert np.array_equal(u[:, :w], ou[:, :w]) and np.array_equal(v[:, :w], ov[:, :w])
 
 
+@pytest.mark.parametrize("w,h,sweeps", [(1, 1, 5), (2, 3, 14), (5, 200, 15), (36, 4, 29), (63, 31, 1),
+                                        (65, 49, 16), (129, 97, 3), (641, 359, 43), (900, 701, 13)])
+def test_hs_shape_by_size_matches_oracle(w, h, sweeps):
+    """The launch shape follows the level's size and the sweep count: frames
+    narrower than a halo (mirrored columns wrap around), one tile, ragged
+    tiles, both tile heights, a short last launch."""
+    rng = np.random.default_rng(w + h)
+    I0 = (rng.random((h, w)) * 255).astype(np.float32)
+    I1 = (rng.random((h, w)) * 255).astype(np.float32)
+    with HornSchunck(1, w, w, h) as hs:
+        u, v = hs.ComputeFlow(I0, I1, w, h, w, 15.0, 1, 2, sweeps)
+    ou, ov = O.hs_compute(I0, I1, alpha=15.0, nLevels=1, nWarpIters=2, nSolverIters=sweeps)
+    assert np.array_equal(u, ou) and np.array_equal(v, ov)
+
+
+@pytest.mark.parametrize("scale", [1e-37, 1e-41, 3e-45])
+def test_hs_jacobi_subnormal_increments_bitexact(scale):
+    """Quotients that land on and between subnormal floats (a diffusion front
+    in a static region), with divisors that have short mantissas: the exact
+    quotient is often halfway between two subnormals."""
+    rng = np.random.default_rng(9)
+    h, w = 40, 70
+    du = (rng.integers(-9, 10, (h, w)) * scale).astype(np.float32)
+    dv = (rng.integers(-9, 10, (h, w)) * scale).astype(np.float32)
+    Ix = rng.integers(-6, 7, (h, w)).astype(np.float32)
+    Iy = rng.integers(-6, 7, (h, w)).astype(np.float32)
+    Iz = np.zeros((h, w), np.float32)
+    gu, gv = D.hs_jacobi(du, dv, Ix, Iy, Iz, 1.0, 2, 2, 2)
+    ou, ov = du, dv
+    for _ in range(2):
+        ou, ov = O.hs_jacobi(ou, ov, Ix, Iy, Iz, 1.0)
+    assert np.array_equal(gu, ou) and np.array_equal(gv, ov)
+
+
 @pytest.mark.parametrize("spac,temp,win", [(3, 2, 5), (5, 2, 7), (7, 3, 3), (9, 5, 9), (1, 2, 5)])
 def test_lk_single_scale_matches_oracle(spac, temp, win):
     rng = np.random.default_rng(spac * 10 + temp)
