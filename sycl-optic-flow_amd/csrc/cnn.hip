@@ -49,7 +49,7 @@ __host__ __device__ __forceinline__ short to_bf16(float f)
 // gfx950 16x16x32 MFMA: lane l supplies row (l % 16) of A and column
 // (l % 16) of B for k = 8*(l/16) .. +7, and receives column (l % 16), rows
 // 4*(l/16) .. +3 of the 16x16 product (of_dbg_cnn_mfma checks this through
-// k_conv).
+// k_conv_lds).
 __device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
@@ -58,299 +58,337 @@ __device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c)
 // fp32 -> bf16, round to nearest even (v_cvt_pk_bf16_f32 on gfx950).
 __device__ __forceinline__ bf16x8 to_bf16x8(f32x8 v) { return __builtin_convertvector(v, bf16x8); }
 
-struct Pix {
-    int b, y, x;
-};
+// GEMM-k layout of the packed weights: tap t, channel c at k = t*CP + c, with
+// the channel count padded to CP (a multiple of 8, so that the 8 consecutive
+// k of one MFMA lane are channels of one tap: one 16-byte LDS read), the
+// whole padded to a multiple of 32.
+__host__ __device__ constexpr int pad_channels(int c) { return (c + 7) / 8 * 8; }
+__host__ __device__ constexpr int pad_k(int c) { return (9 * pad_channels(c) + 31) / 32 * 32; }
 
-__device__ __forceinline__ Pix pix_of(long long m, int H, int W)
-{
-    Pix p;
-    const int hw = H * W;
-    const int mi = (int)m;   // pixel counts stay below 2^31
-    p.b = mi / hw;
-    const int r = mi - p.b * hw;
-    p.y = r / W;
-    p.x = r - p.y * W;
-    return p;
-}
-
-__device__ __forceinline__ void pix_next(Pix& p, int H, int W)
-{
-    if (++p.x == W) {
-        p.x = 0;
-        if (++p.y == H) {
-            p.y = 0;
-            p.b++;
-        }
-    }
-}
-
-// Eight consecutive GEMM-k entries k .. k+7 of pixel p's im2col row
-// (k = t*CX + c), gathered from an NHWC tensor with CX channels; `sgn` = -1
-// mirrors the tap offsets (data gradient).
+// Eight consecutive channels c8 .. c8+7 (zero past CX) of an NHWC pixel.
 template <int CX>
-__device__ __forceinline__ bf16x8 gather8(const float* __restrict__ X, const Pix& p, bool valid,
-                                          int k, int K, int H, int W, int sgn)
+__device__ __forceinline__ f32x8 load_channels(const float* __restrict__ X, long long pix, int c8)
 {
-    f32x8 r;
+    f32x8 v;
+#pragma unroll
+    for (int j = 0; j < 8; j++) v[j] = 0.0f;
     if constexpr (CX % 8 == 0) {
-        // the eight entries share a tap: two 16-byte loads
-        const int t = k / CX, c = k - t * CX;
-        const int yy = p.y + sgn * (t / 3 - 1), xx = p.x + sgn * (t % 3 - 1);
-        float4 v0 = make_float4(0.f, 0.f, 0.f, 0.f), v1 = v0;
-        if (valid && k < K && yy >= 0 && yy < H && xx >= 0 && xx < W) {
-            const float4* q = reinterpret_cast<const float4*>(X + (((long long)p.b * H + yy) * W + xx) * CX + c);
-            v0 = q[0];
-            v1 = q[1];
-        }
-        r[0] = v0.x; r[1] = v0.y; r[2] = v0.z; r[3] = v0.w;
-        r[4] = v1.x; r[5] = v1.y; r[6] = v1.z; r[7] = v1.w;
+        const float4* q = reinterpret_cast<const float4*>(X + pix * CX + c8);
+        const float4 v0 = q[0], v1 = q[1];
+        v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
+        v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
     } else {
+        static_assert(CX <= 8, "one group of 8 channels");
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int kk = k + j;
-            const int t = kk / CX, c = kk - t * CX;
-            const int yy = p.y + sgn * (t / 3 - 1), xx = p.x + sgn * (t % 3 - 1);
-            float v = 0.0f;
-            if (valid && kk < K && yy >= 0 && yy < H && xx >= 0 && xx < W)
-                v = X[(((long long)p.b * H + yy) * W + xx) * CX + c];
-            r[j] = v;
-        }
+        for (int j = 0; j < CX; j++) v[j] = X[pix * CX + j];
     }
-    return to_bf16x8(r);
+    return v;
 }
 
-// Implicit-GEMM 3x3 convolution.  A block is 4 waves; a wave owns 16
-// pixels and NT 16-wide tiles of output channels.  Wp: bf16 [NT*16][Kpad]
-// (Kpad a multiple of 32), row n = output channel, zero beyond K and N.
-// Epilogue: + bias, ReLU, and/or zero where mask[m][n] <= 0 (the ReLU
+// Implicit-GEMM 3x3 convolution on the MFMA, 16-wide output tiles of NT*16
+// channels.  A block (4 waves) computes a tile of 16 x TR pixels of one
+// image, each wave TR/4 rows of 16 pixels (one MFMA row block each), from a
+// (16+2) x (TR+2) bf16 input patch and the bf16 weights, both staged in LDS
+// once.  Epilogue: + bias, ReLU, and/or zero where mask[m][n] <= 0 (the ReLU
 // derivative of the layer below).
-template <int CX, int NT>
-__global__ __launch_bounds__(256) void k_conv(const float* __restrict__ X, int B, int H, int W,
-                                              const short* __restrict__ Wp, int Kpad, int N,
-                                              const float* __restrict__ bias, int sgn, int relu,
-                                              const float* __restrict__ mask,
-                                              float* __restrict__ Y)
-{
-    const int K = 9 * CX;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long long M = (long long)B * H * W;
-    const long long m0 = ((long long)blockIdx.x * 4 + wave) * 16;
-    if (m0 >= M) return;
-    const int row = lane & 15, kg = lane >> 4;
-    const long long ma = m0 + row;
-    const bool valid = ma < M;
-    const Pix p = pix_of(valid ? ma : 0, H, W);
-    f32x4 acc[NT];
-#pragma unroll
-    for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
-    constexpr int KP = (9 * CX + 31) / 32 * 32;   // == Kpad (checked by the launcher)
-#pragma unroll
-    for (int k0 = 0; k0 < KP; k0 += 32) {
-        const bf16x8 a = gather8<CX>(X, p, valid, k0 + 8 * kg, K, H, W, sgn);
-#pragma unroll
-        for (int t = 0; t < NT; t++) {
-            const bf16x8 b = __builtin_bit_cast(
-                bf16x8, *reinterpret_cast<const s16x8*>(Wp + (size_t)(t * 16 + row) * KP + k0 + 8 * kg));
-            acc[t] = mfma32(a, b, acc[t]);
-        }
-    }
-#pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const int n = t * 16 + row;
-        if (n >= N) continue;
-        const float bn = bias ? bias[n] : 0.0f;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const long long m = m0 + 4 * kg + j;
-            if (m >= M) continue;
-            float v = acc[t][j] + bn;
-            if (relu) v = v > 0.0f ? v : 0.0f;
-            if (mask && !(mask[m * N + n] > 0.0f)) v = 0.0f;
-            Y[m * N + n] = v;
-        }
-    }
-}
-
-// The same convolution for CX % 32 == 0 with the operands staged in LDS:
-// a block computes an 8x8-pixel tile of one image (waves take 2 rows each)
-// from a 10x10xCX bf16 input patch and the bf16 weights, both loaded once,
-// so each input pixel and each weight leaves HBM / L2 once per block
-// instead of once per tap and per wave.  MFMA operands come from LDS with
-// 16-byte reads; accumulation, epilogue and results equal k_conv's.
-template <int CX, int NT>
+//
+// Bound by the fp32 activations (each read once plus the halo, written
+// once; 32 images of 68x120x32: 67 MB, 17.9 us, 3.7 TB/s) and at small
+// batches by the latency of one tile, so every load of a tile is issued before
+// the first is used: with branches around the loads they had gone out one by
+// one (26.7 us; one image 9 us, now 3.8).  LDS rows are padded by 16 B so that
+// 8 lanes' 16-byte reads fall on distinct banks.
+template <int CX, int NT, int TR>
 __global__ __launch_bounds__(256) void k_conv_lds(const float* __restrict__ X, int B, int H, int W,
                                                   const short* __restrict__ Wp, int N,
                                                   const float* __restrict__ bias, int sgn, int relu,
                                                   const float* __restrict__ mask,
                                                   float* __restrict__ Y)
 {
-    static_assert(CX % 32 == 0, "one 32-wide k-step must stay inside one tap");
-    constexpr int KP = 9 * CX;           // a multiple of 32
-    constexpr int PW = 10, PP = PW * PW;
-    __shared__ __align__(16) short patch[PP * CX];
-    __shared__ __align__(16) short wts[NT * 16 * KP];
-    const int tiles_x = (W + 7) / 8, tiles_y = (H + 7) / 8;
+    constexpr int CP = pad_channels(CX), KP = pad_k(CX), MB = TR / 4;
+    constexpr int PW = 18, PP = PW * (TR + 2), PS = CP + 8, WS = KP + 8;
+    __shared__ __align__(16) short patch[PP * PS];
+    __shared__ __align__(16) short wts[NT * 16 * WS];
+    const int tiles_x = (W + 15) / 16, tiles_y = (H + TR - 1) / TR;
     const int tile = blockIdx.x;
     const int b = tile / (tiles_x * tiles_y);
     const int r = tile - b * tiles_x * tiles_y;
-    const int y0 = (r / tiles_x) * 8, x0 = (r % tiles_x) * 8;
-    // input patch rows y0-1 .. y0+8, columns x0-1 .. x0+8, zero outside
-    for (int e = threadIdx.x; e < PP * (CX / 8); e += 256) {
-        const int pix = e / (CX / 8), c8 = (e - pix * (CX / 8)) * 8;
-        const int yy = y0 - 1 + pix / PW, xx = x0 - 1 + pix % PW;
-        f32x8 v;
+    const int y0 = (r / tiles_x) * TR, x0 = (r % tiles_x) * 16;
+    // input patch rows y0-1 .. y0+TR, columns x0-1 .. x0+16, zero outside; all
+    // of a thread's loads are issued before its first LDS write
+    constexpr int ITEMS = PP * (CP / 8), NI = (ITEMS + 255) / 256;
+    // (positions outside read pixel 0 instead of branching around the load)
+    f32x8 v[NI];
+    bool in[NI];
 #pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = 0.0f;
-        if (yy >= 0 && yy < H && xx >= 0 && xx < W) {
-            const float4* q = reinterpret_cast<const float4*>(X + (((long long)b * H + yy) * W + xx) * CX + c8);
-            const float4 v0 = q[0], v1 = q[1];
-            v[0] = v0.x; v[1] = v0.y; v[2] = v0.z; v[3] = v0.w;
-            v[4] = v1.x; v[5] = v1.y; v[6] = v1.z; v[7] = v1.w;
-        }
-        *reinterpret_cast<bf16x8*>(patch + pix * CX + c8) = to_bf16x8(v);
+    for (int i = 0; i < NI; i++) {
+        const int e = (int)threadIdx.x + 256 * i;
+        const int pix = e / (CP / 8), c8 = (e - pix * (CP / 8)) * 8;
+        const int yy = y0 - 1 + pix / PW, xx = x0 - 1 + pix % PW;
+        in[i] = e < ITEMS && yy >= 0 && yy < H && xx >= 0 && xx < W;
+        v[i] = load_channels<CX>(X, in[i] ? ((long long)b * H + yy) * W + xx : 0, c8);
     }
-    for (int e = threadIdx.x; e < NT * 16 * KP / 8; e += 256)
-        reinterpret_cast<s16x8*>(wts)[e] = reinterpret_cast<const s16x8*>(Wp)[e];
+    for (int e = threadIdx.x; e < NT * 16 * (KP / 8); e += 256) {
+        const int n = e / (KP / 8), k8 = e - n * (KP / 8);
+        *reinterpret_cast<s16x8*>(wts + n * WS + 8 * k8) = reinterpret_cast<const s16x8*>(Wp)[e];
+    }
+#pragma unroll
+    for (int i = 0; i < NI; i++) {
+        const int e = (int)threadIdx.x + 256 * i;
+        const int pix = e / (CP / 8), c8 = (e - pix * (CP / 8)) * 8;
+        if (e < ITEMS) *reinterpret_cast<bf16x8*>(patch + pix * PS + c8) = in[i] ? to_bf16x8(v[i]) : bf16x8{};
+    }
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = lane & 15, kg = lane >> 4;
-    const int py = wave * 2 + (row >> 3), px = row & 7;   // this lane's A pixel in the tile
-    f32x4 acc[NT];
+    f32x4 acc[MB][NT];
 #pragma unroll
-    for (int t = 0; t < NT; t++) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int m = 0; m < MB; m++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[m][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const short* pbase = patch + ((wave * MB + 1) * PW + row + 1) * PS;
 #pragma unroll
     for (int k0 = 0; k0 < KP; k0 += 32) {
-        const int tap = k0 / CX, c = k0 - tap * CX + 8 * kg;
-        const int dy = sgn * (tap / 3 - 1), dx = sgn * (tap % 3 - 1);
-        const bf16x8 a = *reinterpret_cast<const bf16x8*>(patch + ((py + 1 + dy) * PW + (px + 1 + dx)) * CX + c);
+        const int k = k0 + 8 * kg;
+        const int tap = CP % 32 == 0 ? k0 / CP : (k / CP < 9 ? k / CP : 8);   // past 9: zero weights
+        const int c = CP % 32 == 0 ? k0 % CP + 8 * kg : k % CP;
+        const int off = sgn * ((tap / 3 - 1) * PW + (tap % 3 - 1)) * PS + c;
+        bf16x8 w[NT];
+#pragma unroll
+        for (int t = 0; t < NT; t++) w[t] = *reinterpret_cast<const bf16x8*>(wts + (t * 16 + row) * WS + k);
+#pragma unroll
+        for (int m = 0; m < MB; m++) {
+            const bf16x8 a = *reinterpret_cast<const bf16x8*>(pbase + m * PW * PS + off);
+#pragma unroll
+            for (int t = 0; t < NT; t++) acc[m][t] = mfma32(a, w[t], acc[m][t]);
+        }
+    }
+    // accumulator: column n = t*16 + row, rows (pixels) x0 + 4*kg + j of image row
+    if (relu || bias) {
 #pragma unroll
         for (int t = 0; t < NT; t++) {
-            const bf16x8 bv = *reinterpret_cast<const bf16x8*>(wts + (t * 16 + row) * KP + k0 + 8 * kg);
-            acc[t] = mfma32(a, bv, acc[t]);
+            const float bn = bias && t * 16 + row < N ? bias[t * 16 + row] : 0.0f;
+#pragma unroll
+            for (int m = 0; m < MB; m++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float q = acc[m][t][j] + bn;
+                    acc[m][t][j] = relu && !(q > 0.0f) ? 0.0f : q;
+                }
         }
     }
-    // accumulator: column n = t*16 + row, rows (pixels) 4*kg + j of the wave's 16
 #pragma unroll
-    for (int t = 0; t < NT; t++) {
-        const int n = t * 16 + row;
-        if (n >= N) continue;
-        const float bn = bias ? bias[n] : 0.0f;
+    for (int m = 0; m < MB; m++) {
+        const int yy = y0 + wave * MB + m;
+        if (yy >= H) break;
+        const long long o0 = (((long long)b * H + yy) * W + x0 + 4 * kg) * N + row;
+        bool ok[4][NT];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int q = 4 * kg + j;
-            const int yy = y0 + wave * 2 + (q >> 3), xx = x0 + (q & 7);
-            if (yy >= H || xx >= W) continue;
-            const long long m = ((long long)b * H + yy) * W + xx;
-            float v = acc[t][j] + bn;
-            if (relu) v = v > 0.0f ? v : 0.0f;
-            if (mask && !(mask[m * N + n] > 0.0f)) v = 0.0f;
-            Y[m * N + n] = v;
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int t = 0; t < NT; t++) ok[j][t] = x0 + 4 * kg + j < W && t * 16 + row < N;
+        if (mask) {
+            float mk[4][NT];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int t = 0; t < NT; t++) mk[j][t] = mask[ok[j][t] ? o0 + j * N + t * 16 : 0];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int t = 0; t < NT; t++)
+                    if (!(mk[j][t] > 0.0f)) acc[m][t][j] = 0.0f;
         }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+#pragma unroll
+            for (int t = 0; t < NT; t++)
+                if (ok[j][t]) Y[o0 + j * N + t * 16] = acc[m][t][j];
     }
 }
 
-// Weight-gradient partials.  Block (kt, nt, z) forms the 16x16 tile
-// dW[16*nt ..][16*kt ..] over the pixels [z*chunk, (z+1)*chunk): the four
-// waves take interleaved 32-pixel steps (A = dY^T, B = im2col(X), GEMM-k =
-// pixels) and are then added in wave order.  part: [splits][Npad][Kpad].
-template <int CX>
-__global__ __launch_bounds__(256) void k_wgrad(const float* __restrict__ dY, int N,
+// Weight- and bias-gradient partials of one layer.  dW[n][t][c] is a GEMM over
+// pixels: a block walks tiles of 8 x 16 pixels (blockIdx.x, + gridDim.x, ..)
+// and keeps its whole dW in MFMA accumulators, the NT*16 x 16 column tiles
+// dealt to its 4 waves.  Per tile dY^T and X^T are staged in LDS as bf16 with
+// 8 consecutive pixels of a channel per 16 bytes, which is what one lane of
+// an MFMA operand holds; X^T three times, shifted by the taps' dx, so that
+// every tap reads aligned.  part: [blocks][NT*16][Kpad] with k = t*CX + c.
+// The bias gradient is the fp32 sum of dY, taken on the way to LDS.
+//
+// Bound by reading dY and X once (fp32; 67 MB per 32->32 layer at 32 x 68 x
+// 120 pixels).  The earlier kernel formed one 16x16
+// tile per block and so read both once per column tile: 139 us per 32->32
+// layer of 32 x 68 x 120 pixels, and 122 us for the bias sums.
+constexpr int kWgRows = 16;          // tile height in pixels
+constexpr int kWgMaxBlocks = 768;    // three per CU; bounds the partials
+
+template <int CX, int N>
+__global__ __launch_bounds__(256) void k_wgrad(const float* __restrict__ dY,
                                                const float* __restrict__ X, int B, int H, int W,
-                                               int Kpad, long long chunk, float* __restrict__ part)
+                                               int ntiles, int Kpad, float* __restrict__ part,
+                                               float* __restrict__ bpart)
 {
-    __shared__ float sh[4][16][17];
-    const int K = 9 * CX;
+    constexpr int NT = (N + 15) / 16;
+    constexpr int T = kWgRows, XR = T + 2, YR = T + 1;   // YR: one row of padding against bank conflicts
+    constexpr int COLS = (9 * CX + 15) / 16, CW = (COLS + 3) / 4;
+    __shared__ __align__(16) short xs[3][CX][XR][8];
+    __shared__ __align__(16) short ys[NT * 16][YR][8];
+    __shared__ float sb[256];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int k0 = blockIdx.x * 16, n0 = blockIdx.y * 16;
-    const long long M = (long long)B * H * W;
-    const long long p_begin = (long long)blockIdx.z * chunk;
-    const long long p_end = p_begin + chunk < M ? p_begin + chunk : M;
     const int row = lane & 15, kg = lane >> 4;
-    const int k = k0 + row;   // B column
-    const bool kvalid = k < K;
-    int dy = 0, dx = 0, c = 0;
-    if (kvalid) {
-        const int t = k / CX;
-        c = k - t * CX;
-        dy = t / 3 - 1;
-        dx = t % 3 - 1;
-    }
-    const int n = n0 + row;   // A row
-    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (long long q0 = p_begin + wave * 32; q0 < p_end; q0 += 128) {
-        f32x8 a, b;
-        const long long qf = q0 + 8 * kg;
-        Pix p = pix_of(qf < M ? qf : 0, H, W);
+    const int tiles_x = (W + 7) / 8, tiles_y = (H + T - 1) / T;
+    // LDS offset of this lane's column of each of the wave's column tiles
+    int xoff[CW];
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const long long q = qf + j;
-            float va = 0.0f, vb = 0.0f;
-            if (q < p_end) {
-                if (n < N) va = dY[q * N + n];
-                if (kvalid) {
-                    const int y = p.y + dy, x = p.x + dx;
-                    if (y >= 0 && y < H && x >= 0 && x < W)
-                        vb = X[(((long long)p.b * H + y) * W + x) * CX + c];
+    for (int i = 0; i < CW; i++) {
+        const int k = min((wave + 4 * i) * 16 + row, 9 * CX - 1);   // past the end: computed, not read back
+        const int t = k / CX, c = k - t * CX;
+        xoff[i] = ((t % 3) * CX + c) * XR * 8 + (t / 3) * 8;
+    }
+    f32x4 acc[CW][NT];
+#pragma unroll
+    for (int i = 0; i < CW; i++)
+#pragma unroll
+        for (int t = 0; t < NT; t++) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // rows past N stay zero
+    for (int e = threadIdx.x; e < NT * 16 * YR; e += 256)
+        *reinterpret_cast<bf16x8*>(&ys[0][0][0] + 8 * e) = bf16x8{};
+    float bsum = 0.0f;
+    const int yn = (int)threadIdx.x % N;   // 256 % N == 0: a thread's dY items share the channel
+    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int b = tile / (tiles_x * tiles_y);
+        const int r = tile - b * tiles_x * tiles_y;
+        const int y0 = (r / tiles_x) * T, x0 = (r % tiles_x) * 8;
+        // positions outside the image load a pixel inside instead of branching
+        // around the load, and are zeroed afterwards
+        const bool xedge = x0 == 0 || x0 + 9 > W;   // uniform
+        constexpr int XI = (XR * CX + 255) / 256;
+        float xv[XI][10];
+        bool xin[XI];
+#pragma unroll
+        for (int i = 0; i < XI; i++) {
+            const int e = (int)threadIdx.x + 256 * i;
+            const int pr = e / CX, c = e - pr * CX;
+            const int yy = y0 - 1 + pr;
+            xin[i] = e < XR * CX && yy >= 0 && yy < H;
+            const float* p = X + (xin[i] ? ((long long)b * H + yy) * W * CX : 0) + c;
+#pragma unroll
+            for (int j = 0; j < 10; j++) xv[i][j] = p[min(max(x0 - 1 + j, 0), W - 1) * CX];
+            if (xedge) {
+#pragma unroll
+                for (int j = 0; j < 10; j++)
+                    if (x0 - 1 + j < 0 || x0 - 1 + j >= W) xv[i][j] = 0.0f;
+            }
+        }
+        constexpr int YI = (T * N + 255) / 256;
+        float yv[YI][8];
+        bool yin[YI];
+#pragma unroll
+        for (int i = 0; i < YI; i++) {
+            const int e = (int)threadIdx.x + 256 * i, yy = y0 + e / N;
+            yin[i] = e < T * N && yy < H;
+            const float* p = dY + (yin[i] ? ((long long)b * H + yy) * W * N : 0) + yn;
+#pragma unroll
+            for (int j = 0; j < 8; j++) yv[i][j] = p[min(x0 + j, W - 1) * N];
+            if (xedge) {
+#pragma unroll
+                for (int j = 0; j < 8; j++)
+                    if (x0 + j >= W) yv[i][j] = 0.0f;
+            }
+        }
+        __syncthreads();   // the previous tile's operands have been read
+#pragma unroll
+        for (int i = 0; i < XI; i++) {
+            const int e = (int)threadIdx.x + 256 * i;
+            const int pr = e / CX, c = e - pr * CX;
+            if (e < XR * CX) {
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    f32x8 v;
+#pragma unroll
+                    for (int j = 0; j < 8; j++) v[j] = xv[i][d + j];
+                    *reinterpret_cast<bf16x8*>(&xs[d][c][pr][0]) = xin[i] ? to_bf16x8(v) : bf16x8{};
                 }
             }
-            a[j] = va;
-            b[j] = vb;
-            pix_next(p, H, W);
         }
-        acc = mfma32(to_bf16x8(a), to_bf16x8(b), acc);
+#pragma unroll
+        for (int i = 0; i < YI; i++) {
+            const int e = (int)threadIdx.x + 256 * i;
+            f32x8 v;
+            float s = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                v[j] = yin[i] ? yv[i][j] : 0.0f;
+                s += v[j];
+            }
+            bsum += s;
+            if (e < T * N) *reinterpret_cast<bf16x8*>(&ys[yn][e / N][0]) = to_bf16x8(v);
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < T / 4; ks++) {   // 32 pixels: 4 rows of 8
+            const int pr = ks * 4 + kg;
+            bf16x8 a[NT];
+#pragma unroll
+            for (int t = 0; t < NT; t++) a[t] = *reinterpret_cast<const bf16x8*>(&ys[t * 16 + row][pr][0]);
+#pragma unroll
+            for (int i = 0; i < CW; i++) {
+                if (wave + 4 * i >= COLS) break;   // wave-uniform
+                const bf16x8 x = *reinterpret_cast<const bf16x8*>(&xs[0][0][0][0] + xoff[i] + pr * 8);
+#pragma unroll
+                for (int t = 0; t < NT; t++) acc[i][t] = mfma32(a[t], x, acc[i][t]);
+            }
+        }
     }
 #pragma unroll
-    for (int j = 0; j < 4; j++) sh[wave][4 * kg + j][row] = acc[j];   // [n][k]
+    for (int i = 0; i < CW; i++) {
+        const int col = wave + 4 * i;
+        if (col >= COLS) break;
+#pragma unroll
+        for (int t = 0; t < NT; t++)
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                part[((size_t)blockIdx.x * (NT * 16) + t * 16 + 4 * kg + j) * Kpad + col * 16 + row] = acc[i][t][j];
+    }
+    sb[threadIdx.x] = bsum;
     __syncthreads();
-    const int i = threadIdx.x >> 4, jj = threadIdx.x & 15;
-    const float s = ((sh[0][i][jj] + sh[1][i][jj]) + sh[2][i][jj]) + sh[3][i][jj];
-    const size_t Npad = (size_t)gridDim.y * 16;
-    part[((size_t)blockIdx.z * Npad + (n0 + i)) * Kpad + (k0 + jj)] = s;
-}
-
-// dW[n][k] = sum over the splits in order (k < K, n < N).
-__global__ __launch_bounds__(256) void k_wgrad_reduce(const float* __restrict__ part, int splits,
-                                                      int Npad, int Kpad, int N, int K,
-                                                      float* __restrict__ dW)
-{
-    const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx >= N * K) return;
-    const int n = idx / K, k = idx - n * K;
-    float s = 0.0f;
-    for (int sp = 0; sp < splits; sp++) s += part[((size_t)sp * Npad + n) * Kpad + k];
-    dW[idx] = s;
-}
-
-// Bias-gradient partials: block z sums dY over its pixel chunk, channel by
-// channel, in a fixed tree.
-__global__ __launch_bounds__(256) void k_bias_partial(const float* __restrict__ dY, int N, long long M,
-                                                      long long chunk, float* __restrict__ part)
-{
-    __shared__ float sh[256];
-    const long long p0 = (long long)blockIdx.x * chunk;
-    const long long p1 = p0 + chunk < M ? p0 + chunk : M;
-    for (int n = 0; n < N; n++) {
-        float s = 0.0f;
-        for (long long q = p0 + threadIdx.x; q < p1; q += 256) s += dY[q * N + n];
-        sh[threadIdx.x] = s;
-        __syncthreads();
-        for (int w = 128; w > 0; w >>= 1) {
-            if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-            __syncthreads();
-        }
-        if (threadIdx.x == 0) part[(size_t)blockIdx.x * N + n] = sh[0];
-        __syncthreads();
+    if ((int)threadIdx.x < N) {
+        float s = sb[threadIdx.x];
+        for (int q = (int)threadIdx.x + N; q < 256; q += N) s += sb[q];
+        bpart[(size_t)blockIdx.x * N + threadIdx.x] = s;
     }
 }
 
-__global__ void k_bias_reduce(const float* __restrict__ part, int splits, int N, float* __restrict__ db)
+// dW and db: sums of the partials in a fixed order.  A block sums 64 outputs,
+// 16 interleaved groups of partials each, then the groups in order (a single
+// thread per output took 16 us per layer, one chain of 256 loads).
+__global__ __launch_bounds__(1024) void k_grad_reduce(const float* __restrict__ part, int parts, int Npad,
+                                                      int Kpad, int N, int K, float* __restrict__ dW,
+                                                      const float* __restrict__ bpart,
+                                                      float* __restrict__ db)
 {
-    const int n = threadIdx.x;
-    if (n >= N) return;
+    __shared__ float sh[16][64];
+    const int o = threadIdx.x & 63, q = threadIdx.x >> 6;
+    const int idx = blockIdx.x * 64 + o;
     float s = 0.0f;
-    for (int sp = 0; sp < splits; sp++) s += part[(size_t)sp * N + n];
-    db[n] = s;
+    if (idx < N * K) {
+        const int n = idx / K, k = idx - n * K;
+        const float* p = part + (size_t)n * Kpad + k;
+#pragma unroll 8
+        for (int sp = q; sp < parts; sp += 16) s += p[(size_t)sp * Npad * Kpad];
+    } else if (idx < N * K + N) {
+#pragma unroll 8
+        for (int sp = q; sp < parts; sp += 16) s += bpart[(size_t)sp * N + (idx - N * K)];
+    }
+    sh[q][o] = s;
+    __syncthreads();
+    if (q == 0 && idx < N * K + N) {
+#pragma unroll
+        for (int g = 1; g < 16; g++) s += sh[g][o];
+        if (idx < N * K) dW[idx] = s;
+        else db[idx - N * K] = s;
+    }
 }
 
 // Mean-squared flow error against planar targets T[b][2][H*W]:
@@ -380,12 +418,21 @@ __global__ __launch_bounds__(256) void k_mse(const float* __restrict__ Y, const 
     if (threadIdx.x == 0) part[blockIdx.x] = sh[0];
 }
 
-__global__ void k_sum_f64(const double* __restrict__ part, int n, double scale, double* __restrict__ out)
+// Sum of the block partials, one workgroup, fixed order (one thread took 51 us
+// for 1024 of them, a chain of dependent loads).
+__global__ __launch_bounds__(256) void k_sum_f64(const double* __restrict__ part, int n, double scale,
+                                                 double* __restrict__ out)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    __shared__ double sh[256];
     double s = 0.0;
-    for (int i = 0; i < n; i++) s += part[i];
-    *out = s * scale;
+    for (int i = threadIdx.x; i < n; i += 256) s += part[i];
+    sh[threadIdx.x] = s;
+    __syncthreads();
+    for (int w = 128; w > 0; w >>= 1) {
+        if ((int)threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) *out = sh[0] * scale;
 }
 
 // Adam (Kingma & Ba 2015) with bias-correction factors c1 = 1 - b1^t,
@@ -405,27 +452,25 @@ __global__ __launch_bounds__(256) void k_adam(float* __restrict__ w, const float
     w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
-// bf16 packs of one layer's weights Wm[n][t][c] (N outputs, C inputs):
-//   fwd [Npad][Kpad]:  row n, k = t*C + c
-//   bwd [Cpad][Kbpad]: row c, k = t*N + n
+// bf16 packs of one layer's weights Wm[n][t][c] (N outputs, C inputs), zero
+// in the padding:
+//   fwd [Npad][pad_k(C)]: row n, k = t*pad_channels(C) + c
+//   bwd [Cpad][pad_k(N)]: row c, k = t*pad_channels(N) + n
 __global__ __launch_bounds__(256) void k_pack(const float* __restrict__ Wm, int N, int C, int Npad,
-                                              int Kpad, int Cpad, int Kbpad, short* __restrict__ fwd,
+                                              int Cpad, short* __restrict__ fwd,
                                               short* __restrict__ bwd)
 {
-    const int K = 9 * C;
+    const int Kf = pad_k(C), Kb = pad_k(N);
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-    if (idx < Npad * Kpad) {
-        const int n = idx / Kpad, k = idx - n * Kpad;
-        fwd[idx] = (n < N && k < K) ? to_bf16(Wm[n * K + k]) : (short)0;
+    if (idx < Npad * Kf) {
+        const int n = idx / Kf, k = idx - n * Kf;
+        const int t = k / pad_channels(C), c = k - t * pad_channels(C);
+        fwd[idx] = (n < N && t < 9 && c < C) ? to_bf16(Wm[(n * 9 + t) * C + c]) : (short)0;
     }
-    if (idx < Cpad * Kbpad) {
-        const int c = idx / Kbpad, kb = idx - c * Kbpad;
-        short v = 0;
-        if (c < C && kb < 9 * N) {
-            const int t = kb / N, n = kb - t * N;
-            v = to_bf16(Wm[(n * 9 + t) * C + c]);
-        }
-        bwd[idx] = v;
+    if (idx < Cpad * Kb) {
+        const int c = idx / Kb, k = idx - c * Kb;
+        const int t = k / pad_channels(N), n = k - t * pad_channels(N);
+        bwd[idx] = (c < C && t < 9 && n < N) ? to_bf16(Wm[(n * 9 + t) * C + c]) : (short)0;
     }
 }
 
@@ -461,6 +506,13 @@ __global__ __launch_bounds__(256) void k_to_planar(const float* __restrict__ Y, 
 }
 
 inline int pad16(int v) { return (v + 15) / 16 * 16; }
+// From two 16x8-pixel tiles per CU on, the convolution takes them; below, 16x4
+// tiles, whose workgroups are shorter and twice as many.  Measured per 32->32
+// layer of 68x120 pixels (us, 16x8 / 16x4): batch 1 4.4 / 3.8, 4 5.3 / 5.1,
+// 8 6.8 / 6.9, 16 10.5 / 10.9, 32 17.9 / 18.2 (16x16 tiles 10.2 and 19.1 at
+// 16 and 32).
+constexpr long long kConvTallTiles = 512;
+
 inline int pad32(int v) { return (v + 31) / 32 * 32; }
 inline unsigned blocks256(long long n)
 {
@@ -477,32 +529,29 @@ inline unsigned blocks256(long long n)
         }                                                   \
     } while (0)
 
-// Dispatch over the instantiated (input channels, output tiles) pairs.
-int launch_conv(const float* X, int B, int H, int W, int CX, const short* Wp, int Kpad, int N,
-                const float* bias, int sgn, int relu, const float* mask, float* Y, hipStream_t st)
+template <int CX, int NT, int TR>
+int launch_conv_tile(const float* X, int B, int H, int W, const short* Wp, int N, const float* bias, int sgn,
+                     int relu, const float* mask, float* Y, hipStream_t st)
 {
-    const long long M = (long long)B * H * W;
-    const unsigned blocks = (unsigned)((M + 63) / 64);
+    const unsigned tiles = (unsigned)B * ((H + TR - 1) / TR) * ((W + 15) / 16);
+    hipLaunchKernelGGL((k_conv_lds<CX, NT, TR>), dim3(tiles), dim3(256), 0, st, X, B, H, W, Wp, N, bias, sgn,
+                       relu, mask, Y);
+    CNN_CHECK("k_conv_lds");
+    return OF_OK;
+}
+
+// Dispatch over the instantiated (input channels, output tiles) pairs and the
+// tile height.
+int launch_conv(const float* X, int B, int H, int W, int CX, const short* Wp, int N, const float* bias,
+                int sgn, int relu, const float* mask, float* Y, hipStream_t st)
+{
     const int NT = N <= 16 ? 1 : 2;
-    if (N > 32 || Kpad != (9 * CX + 31) / 32 * 32) return OF_ERR_UNSUPPORTED;
-    if (CX == 32) {   // LDS-staged tiles of 8x8 pixels
-        const unsigned tiles = (unsigned)(B * ((H + 7) / 8) * ((W + 7) / 8));
-        if (NT == 2)
-            hipLaunchKernelGGL((k_conv_lds<32, 2>), dim3(tiles), dim3(256), 0, st, X, B, H, W, Wp, N, bias,
-                               sgn, relu, mask, Y);
-        else
-            hipLaunchKernelGGL((k_conv_lds<32, 1>), dim3(tiles), dim3(256), 0, st, X, B, H, W, Wp, N, bias,
-                               sgn, relu, mask, Y);
-        CNN_CHECK("k_conv_lds");
-        return OF_OK;
-    }
-#define CONV_CASE(cx, nt)                                                                          \
-    if (CX == cx && NT == nt) {                                                                    \
-        hipLaunchKernelGGL((k_conv<cx, nt>), dim3(blocks), dim3(256), 0, st, X, B, H, W, Wp, Kpad, \
-                           N, bias, sgn, relu, mask, Y);                                           \
-        CNN_CHECK("k_conv");                                                                       \
-        return OF_OK;                                                                              \
-    }
+    if (N > 32) return OF_ERR_UNSUPPORTED;
+    const bool tall = (long long)B * ((H + 7) / 8) * ((W + 15) / 16) >= kConvTallTiles;
+#define CONV_CASE(cx, nt)                                                                            \
+    if (CX == cx && NT == nt)                                                                        \
+        return tall ? launch_conv_tile<cx, nt, 8>(X, B, H, W, Wp, N, bias, sgn, relu, mask, Y, st)  \
+                    : launch_conv_tile<cx, nt, 4>(X, B, H, W, Wp, N, bias, sgn, relu, mask, Y, st);
     CONV_CASE(5, 2)
     CONV_CASE(32, 2)
     CONV_CASE(32, 1)
@@ -512,19 +561,22 @@ int launch_conv(const float* X, int B, int H, int W, int CX, const short* Wp, in
     return OF_ERR_UNSUPPORTED;
 }
 
-int launch_wgrad(const float* dY, int N, const float* X, int CX, int B, int H, int W, int Kpad,
-                 int Npad, int splits, long long chunk, float* part, hipStream_t st)
+int wgrad_tiles(int B, int H, int W) { return B * ((H + kWgRows - 1) / kWgRows) * ((W + 7) / 8); }
+
+int launch_wgrad(const float* dY, int N, const float* X, int CX, int B, int H, int W, int Kpad, int blocks,
+                 float* part, float* bpart, hipStream_t st)
 {
-    const dim3 grid(Kpad / 16, Npad / 16, splits);
-#define WG_CASE(cx)                                                                               \
-    if (CX == cx) {                                                                               \
-        hipLaunchKernelGGL((k_wgrad<cx>), grid, dim3(256), 0, st, dY, N, X, B, H, W, Kpad, chunk, \
-                           part);                                                                 \
-        CNN_CHECK("k_wgrad");                                                                     \
-        return OF_OK;                                                                             \
+    const int ntiles = wgrad_tiles(B, H, W);
+#define WG_CASE(cx, n)                                                                                 \
+    if (CX == cx && N == n) {                                                                          \
+        hipLaunchKernelGGL((k_wgrad<cx, n>), dim3(blocks), dim3(256), 0, st, dY, X, B, H, W, ntiles, \
+                           Kpad, part, bpart);                                                 \
+        CNN_CHECK("k_wgrad");                                                                          \
+        return OF_OK;                                                                                  \
     }
-    WG_CASE(5)
-    WG_CASE(32)
+    WG_CASE(5, 32)
+    WG_CASE(32, 32)
+    WG_CASE(32, 2)
 #undef WG_CASE
     return OF_ERR_UNSUPPORTED;
 }
@@ -532,7 +584,7 @@ int launch_wgrad(const float* dY, int N, const float* X, int CX, int B, int H, i
 struct Layer {
     int cin = 0, cout = 0, relu = 0;
     size_t woff = 0, boff = 0;   // offsets into the parameter vector
-    int Kpad = 0, Npad = 0, Cpad = 0, Kbpad = 0;
+    int Kpad = 0, Npad = 0, Cpad = 0;   // Kpad: 9*cin padded, the row of the weight-gradient partials
     short* fwd = nullptr;        // bf16 packs
     short* bwd = nullptr;
 };
@@ -573,11 +625,6 @@ namespace {
 
 constexpr int kLossBlocks = 1024;
 
-int splits_for(long long M)
-{
-    return (int)std::max<long long>(1, std::min<long long>(256, (M + 4095) / 4096));
-}
-
 void free_ws(of_cnn* h)
 {
     for (float*& p : h->act) dev_free(p);
@@ -595,13 +642,13 @@ int ensure_ws(of_cnn* h, long long px)
     free_ws(h);
     int maxc = 5;
     size_t need = 1;
-    const int splits = splits_for(px);
+    const size_t blocks = (size_t)std::min<long long>(kWgMaxBlocks, px);   // a tile holds a pixel at least
     for (const Layer& L : h->layers) {
         float* p = nullptr;
         OF_TRY(dev_alloc(&p, (size_t)px * L.cout));
         h->act.push_back(p);
         maxc = std::max(maxc, std::max(L.cin, L.cout));
-        need = std::max(need, (size_t)splits * (size_t)std::max(L.Npad * L.Kpad, L.cout));
+        need = std::max(need, blocks * (size_t)(L.Npad * L.Kpad + L.cout));
     }
     OF_TRY(dev_alloc(&h->dA, (size_t)px * maxc));
     OF_TRY(dev_alloc(&h->dB, (size_t)px * maxc));
@@ -626,22 +673,25 @@ int ensure_in(of_cnn* h, long long n)
 int pack(of_cnn* h, hipStream_t st)
 {
     for (Layer& L : h->layers) {
-        const int n = std::max(L.Npad * L.Kpad, L.Cpad * L.Kbpad);
+        const int n = std::max(L.Npad * pad_k(L.cin), L.Cpad * pad_k(L.cout));
         hipLaunchKernelGGL(k_pack, dim3(blocks256(n)), dim3(256), 0, st, h->w + L.woff, L.cout, L.cin,
-                           L.Npad, L.Kpad, L.Cpad, L.Kbpad, L.fwd, L.bwd);
+                           L.Npad, L.Cpad, L.fwd, L.bwd);
         CNN_CHECK("k_pack");
     }
     return OF_OK;
 }
 
-int forward(of_cnn* h, const float* X, int B, int H, int W, hipStream_t st)
+// The network's layers; the last one writes `Y`, or its activation buffer if
+// that is null.
+int forward(of_cnn* h, const float* X, int B, int H, int W, float* Y, hipStream_t st)
 {
     const float* in = X;
     for (size_t l = 0; l < h->layers.size(); l++) {
         const Layer& L = h->layers[l];
-        OF_TRY(launch_conv(in, B, H, W, L.cin, L.fwd, L.Kpad, L.cout, h->w + L.boff, 1, L.relu,
-                           nullptr, h->act[l], st));
-        in = h->act[l];
+        float* out = Y && l + 1 == h->layers.size() ? Y : h->act[l];
+        OF_TRY(launch_conv(in, B, H, W, L.cin, L.fwd, L.cout, h->w + L.boff, 1, L.relu,
+                           nullptr, out, st));
+        in = out;
     }
     return OF_OK;
 }
@@ -649,27 +699,22 @@ int forward(of_cnn* h, const float* X, int B, int H, int W, hipStream_t st)
 // Backward pass from the loss gradient in h->dA; fills h->g.
 int backward(of_cnn* h, const float* X, int B, int H, int W, hipStream_t st)
 {
-    const long long M = (long long)B * H * W;
-    const int splits = splits_for(M);
-    const long long chunk = (M + splits - 1) / splits;
+    const int blocks = std::min(kWgMaxBlocks, wgrad_tiles(B, H, W));
     float* dcur = h->dA;
     float* dnext = h->dB;
     for (int l = (int)h->layers.size() - 1; l >= 0; l--) {
         const Layer& L = h->layers[l];
         const float* in = l ? h->act[l - 1] : X;
         const int K = 9 * L.cin;
-        OF_TRY(launch_wgrad(dcur, L.cout, in, L.cin, B, H, W, L.Kpad, L.Npad, splits, chunk, h->part, st));
-        hipLaunchKernelGGL(k_wgrad_reduce, dim3(blocks256(L.cout * K)), dim3(256), 0, st, h->part, splits,
-                           L.Npad, L.Kpad, L.cout, K, h->g + L.woff);
-        CNN_CHECK("k_wgrad_reduce");
-        hipLaunchKernelGGL(k_bias_partial, dim3(splits), dim3(256), 0, st, dcur, L.cout, M, chunk, h->part);
-        CNN_CHECK("k_bias_partial");
-        hipLaunchKernelGGL(k_bias_reduce, dim3(1), dim3(64), 0, st, h->part, splits, L.cout, h->g + L.boff);
-        CNN_CHECK("k_bias_reduce");
+        float* bpart = h->part + (size_t)blocks * L.Npad * L.Kpad;
+        OF_TRY(launch_wgrad(dcur, L.cout, in, L.cin, B, H, W, L.Kpad, blocks, h->part, bpart, st));
+        hipLaunchKernelGGL(k_grad_reduce, dim3((L.cout * (K + 1) + 63) / 64), dim3(1024), 0, st, h->part,
+                           blocks, L.Npad, L.Kpad, L.cout, K, h->g + L.woff, bpart, h->g + L.boff);
+        CNN_CHECK("k_grad_reduce");
         if (l == 0) break;
         // gradient w.r.t. this layer's input, zero where the ReLU below was inactive
         const Layer& P = h->layers[l - 1];
-        OF_TRY(launch_conv(dcur, B, H, W, L.cout, L.bwd, L.Kbpad, L.cin, nullptr, -1, 0,
+        OF_TRY(launch_conv(dcur, B, H, W, L.cout, L.bwd, L.cin, nullptr, -1, 0,
                            P.relu ? h->act[l - 1] : nullptr, dnext, st));
         std::swap(dcur, dnext);
     }
@@ -683,7 +728,7 @@ int loss_grad(of_cnn* h, const float* T, int B, int H, int W, hipStream_t st)
     hipLaunchKernelGGL(k_mse, dim3(blocks), dim3(256), 0, st, h->act.back(), T, M, H * W,
                        1.0f / (float)M, h->dA, h->lpart);
     CNN_CHECK("k_mse");
-    hipLaunchKernelGGL(k_sum_f64, dim3(1), dim3(64), 0, st, h->lpart, (int)blocks, 0.5 / (double)M, h->loss);
+    hipLaunchKernelGGL(k_sum_f64, dim3(1), dim3(256), 0, st, h->lpart, (int)blocks, 0.5 / (double)M, h->loss);
     CNN_CHECK("k_sum_f64");
     return OF_OK;
 }
@@ -745,7 +790,6 @@ int of_cnn_create(int hidden_layers, int channels, unsigned long long seed, of_c
             L.Kpad = pad32(9 * L.cin);
             L.Npad = pad16(L.cout);
             L.Cpad = pad16(L.cin);
-            L.Kbpad = pad32(9 * L.cout);
             h->layers.push_back(L);
         }
         h->nparams = off;
@@ -764,8 +808,8 @@ int of_cnn_create(int hidden_layers, int channels, unsigned long long seed, of_c
         if (!st) st = dev_alloc(&h->lpart, kLossBlocks);
         if (!st) st = dev_alloc(&h->loss, 1);
         for (Layer& L : h->layers) {
-            if (!st) st = dev_alloc(&L.fwd, (size_t)L.Npad * L.Kpad);
-            if (!st) st = dev_alloc(&L.bwd, (size_t)L.Cpad * L.Kbpad);
+            if (!st) st = dev_alloc(&L.fwd, (size_t)L.Npad * pad_k(L.cin));
+            if (!st) st = dev_alloc(&L.bwd, (size_t)L.Cpad * pad_k(L.cout));
         }
         if (!st && hipMemcpy(h->w, w.data(), off * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) st = OF_ERR_HIP;
         if (!st && hipMemset(h->g, 0, off * sizeof(float)) != hipSuccess) st = OF_ERR_HIP;
@@ -823,10 +867,7 @@ int of_cnn_forward(of_cnn* h, const float* dX, int B, int H, int W, float* dY, v
         if (!dims_ok(h, dX, dY, B, H, W)) return OF_ERR_ARG;
         hipStream_t st = (hipStream_t)stream;
         OF_TRY(ensure_ws(h, (long long)B * H * W));
-        OF_TRY(forward(h, dX, B, H, W, st));
-        OF_HIP(hipMemcpyAsync(dY, h->act.back(), (size_t)B * H * W * 2 * sizeof(float),
-                              hipMemcpyDeviceToDevice, st));
-        return OF_OK;
+        return forward(h, dX, B, H, W, dY, st);
     });
 }
 
@@ -839,7 +880,7 @@ int of_cnn_predict(of_cnn* h, const float* dI0s, const float* dI1s, int H, int W
         OF_TRY(ensure_in(h, n));
         OF_TRY(ensure_ws(h, n));
         OF_TRY(of_cnn_features(dI0s, dI1s, H, W, h->xin, st));
-        OF_TRY(forward(h, h->xin, 1, H, W, st));
+        OF_TRY(forward(h, h->xin, 1, H, W, nullptr, st));
         hipLaunchKernelGGL(k_to_planar, dim3(blocks256(n)), dim3(256), 0, st, h->act.back(), (int)n, dU);
         CNN_CHECK("k_to_planar");
         return OF_OK;
@@ -852,7 +893,7 @@ int of_cnn_gradients(of_cnn* h, const float* dX, const float* dT, int B, int H, 
     return guarded([&]() -> int {
         if (!dims_ok(h, dX, dT, B, H, W)) return OF_ERR_ARG;
         OF_TRY(ensure_ws(h, (long long)B * H * W));
-        OF_TRY(forward(h, dX, B, H, W, nullptr));
+        OF_TRY(forward(h, dX, B, H, W, nullptr, nullptr));
         OF_TRY(loss_grad(h, dT, B, H, W, nullptr));
         OF_TRY(backward(h, dX, B, H, W, nullptr));
         OF_HIP(hipDeviceSynchronize());
@@ -868,7 +909,7 @@ int of_cnn_train_step(of_cnn* h, const float* dX, const float* dT, int B, int H,
     return guarded([&]() -> int {
         if (!dims_ok(h, dX, dT, B, H, W) || !(lr > 0.0f)) return OF_ERR_ARG;
         OF_TRY(ensure_ws(h, (long long)B * H * W));
-        OF_TRY(forward(h, dX, B, H, W, nullptr));
+        OF_TRY(forward(h, dX, B, H, W, nullptr, nullptr));
         OF_TRY(loss_grad(h, dT, B, H, W, nullptr));
         OF_TRY(backward(h, dX, B, H, W, nullptr));
         h->step++;
@@ -936,7 +977,7 @@ int of_tvl1_warm_run_device_u8(of_tvl1* tv, of_cnn* net, const uint8_t* dI0, con
     });
 }
 
-// ---- test entry point: MFMA operand layout through k_conv ----
+// ---- test entry point: MFMA operand layout through k_conv_lds ----
 
 // D = A (16x16) * B (16x16), row-major fp32 (operands rounded to bf16),
 // computed as a convolution of a 1x16 image with 16 channels whose only
@@ -948,7 +989,7 @@ int of_dbg_cnn_mfma(const float* A, const float* Bm, float* D)
         float* dX = nullptr;
         float* dY = nullptr;
         short* dW = nullptr;
-        const int Kpad = 160;
+        const int Kpad = pad_k(16);
         int st = dev_alloc(&dX, 256);
         if (!st) st = dev_alloc(&dY, 256);
         if (!st) st = dev_alloc(&dW, 16 * Kpad);
@@ -958,7 +999,7 @@ int of_dbg_cnn_mfma(const float* A, const float* Bm, float* D)
         if (!st && hipMemcpy(dX, A, 256 * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) st = OF_ERR_HIP;
         if (!st && hipMemcpy(dW, w.data(), w.size() * sizeof(short), hipMemcpyHostToDevice) != hipSuccess)
             st = OF_ERR_HIP;
-        if (!st) st = launch_conv(dX, 1, 1, 16, 16, dW, Kpad, 16, nullptr, 1, 0, nullptr, dY, nullptr);
+        if (!st) st = launch_conv(dX, 1, 1, 16, 16, dW, 16, nullptr, 1, 0, nullptr, dY, nullptr);
         if (!st && hipDeviceSynchronize() != hipSuccess) st = OF_ERR_HIP;
         if (!st && hipMemcpy(D, dY, 256 * sizeof(float), hipMemcpyDeviceToHost) != hipSuccess) st = OF_ERR_HIP;
         dev_free(dX);

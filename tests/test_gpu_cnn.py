@@ -105,6 +105,37 @@ def test_gradients_match_oracle(hidden, B, H, W):
     assert _rel(g, g_ex) <= 5e-2
 
 
+@pytest.mark.parametrize("B,H,W", [(1, 1, 1), (1, 3, 17), (2, 16, 8), (1, 17, 9), (3, 33, 31), (1, 2, 130),
+                                   (64, 9, 50)])
+def test_tile_edges_match_oracle(B, H, W):
+    """Image sizes around the convolution's 16x4 and 16x8 tiles (the last case
+    has enough of them for the tall ones) and the weight gradient's 8x16
+    tiles: one pixel, one short row, exact tiles, one pixel past a tile.  The
+    operands round as the emulated oracle's; what is left is the order of the
+    fp32 sums and the bf16 roundings that it flips, the tolerances of the two
+    tests above."""
+    torch = _torch()
+    rng = np.random.default_rng(B + H + W)
+    X = rng.normal(size=(B, H, W, 5)).astype(np.float32)
+    T = rng.normal(size=(B, 2, H, W)).astype(np.float32)
+    net, p = _net(1)
+    dX, dT = torch.from_numpy(X.reshape(-1)).cuda(), torch.from_numpy(T.reshape(-1)).cuda()
+    dY = torch.empty(B * H * W * 2, dtype=torch.float32, device="cuda")
+    net.forward(dX.data_ptr(), B, H, W, dY.data_ptr())
+    torch.cuda.synchronize()
+    emu = NO.forward(p, X, 1, bf16=True)[-1]
+    assert _rel(dY.cpu().numpy().reshape(B, H, W, 2), emu) <= 2e-3
+    loss, g = net.gradients(dX.data_ptr(), dT.data_ptr(), B, H, W)
+    l_emu, g_emu = NO.loss_and_grads(p, X, T, 1, bf16=True)
+    assert abs(loss - l_emu) <= 1e-4 * l_emu
+    off = 0
+    for cin, cout in NO.layer_dims(1):
+        nw = cout * 9 * cin
+        for sl in (slice(off, off + nw), slice(off + nw, off + nw + cout)):
+            assert _rel(g[sl], g_emu[sl]) <= 5e-3, (cin, cout)
+        off += nw + cout
+
+
 def test_training_is_deterministic_and_learns():
     torch = _torch()
     rng = np.random.default_rng(4)
