@@ -127,19 +127,18 @@ __device__ __forceinline__ float bicubic_at(const float* __restrict__ img, float
     return bicubic_sample(img, nx, t);
 }
 
-// Whole-wave lane shifts through DPP (no LDS traffic).  from_left(v) gives
-// lane i the value of lane i-1 and from_right(v) the value of lane i+1; the
-// lane without a source keeps its own value.
-__device__ __forceinline__ float from_left(float v)
+// Whole-wave lane shifts through DPP (no LDS traffic): lane_left(v) gives
+// lane i the value of lane i-1 and lane_right(v) the value of lane i+1; the
+// lane without a source gets 0 (keeping its own value would cost a copy, and
+// the shift could not fold into the instruction that uses it).
+__device__ __forceinline__ float lane_left(float v)
 {
-    const int i = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x138 /* wave_shr:1 */, 0xf, 0xf, false));
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138 /* wave_shr:1 */, 0xf, 0xf, true));
 }
 
-__device__ __forceinline__ float from_right(float v)
+__device__ __forceinline__ float lane_right(float v)
 {
-    const int i = __float_as_int(v);
-    return __int_as_float(__builtin_amdgcn_update_dpp(i, i, 0x130 /* wave_shl:1 */, 0xf, 0xf, false));
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
 }
 
 // hypotf as glibc 2.35 evaluates it for finite arguments: the double sum of

@@ -149,18 +149,6 @@ struct JacobiArgs {
     int zero_in;                   // the input increments are all zero
 };
 
-// Lane shifts with zero in the lane that has no source (its pixel is never
-// stored): without a value to keep, the shift folds into the addition.
-__device__ __forceinline__ float lane_left(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x138 /* wave_shr:1 */, 0xf, 0xf, true));
-}
-
-__device__ __forceinline__ float lane_right(float v)
-{
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x130 /* wave_shl:1 */, 0xf, 0xf, true));
-}
-
 // 1/d of a float in double, to about an ulp: the hardware reciprocal and two
 // Newton steps.  0, infinite and NaN divisors give garbage (div_by fixes it).
 __device__ __forceinline__ double recip_f64(double d)

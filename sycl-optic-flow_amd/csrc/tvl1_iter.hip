@@ -44,8 +44,9 @@ __device__ __forceinline__ void th_step(float rc, float gx, float gy, float u1, 
     const float grad = (gx * gx) + (gy * gy);
     const float rho = rc + ((gx * u1) + (gy * u2));
     const float fi = -rho / grad;
-    const bool c1 = rho >= -l_t * grad;
-    const bool c2 = rho > l_t * grad;
+    const float lg = l_t * grad;   // (-l_t) * grad is -lg bit for bit
+    const bool c1 = rho >= -lg;
+    const bool c2 = rho > lg;
     const bool c3 = grad < 1E-10f;
     const bool zero = c1 && !c2 && c3;
     const float k = c1 ? (c2 ? -l_t : fi) : l_t;
@@ -55,35 +56,144 @@ __device__ __forceinline__ void th_step(float rc, float gx, float gy, float u1, 
     v2 = u2 + d2;
 }
 
+// g = 1 + taut*hypot(fx, fy) and 1/g in double, both for one component of
+// the dual update.
+struct DualDiv {
+    float g;
+    double r;
+    unsigned near;   // below 2^12: the root is too close to a float rounding boundary to be sure
+};
+
+__device__ __forceinline__ DualDiv dual_div(float fx, float fy, float taut)
+{
+    DualDiv d;
+    const double x = (double)fx, y = (double)fy;
+    // the squares are exact in double.  The added 2^-200 keeps a zero gradient
+    // off the root's pole and otherwise only reaches sums below 2^-140, whose
+    // root leaves g at 1 (taut < 2^40).
+    const double s = __builtin_fma(x, x, __builtin_fma(y, y, 0x1p-200));
+    const double q = __builtin_amdgcn_rsq(s);
+    const double h0 = s * q;
+    const double h = __builtin_fma(0.5 * h0, __builtin_fma(-h0, q, 1.0), h0);
+    // h is within 2^-47 of sqrt(s) (the hardware root seed is within 2^-24).
+    // Its float rounding is that of the exact double root unless the 29
+    // dropped bits are within 2^8 of half a float ulp (2^28): 2^11 of 2^31
+    // after the shift.
+    d.near = ((unsigned)__double2loint(h) << 3) + (0x80000000u + (1u << 11));
+    d.g = 1.0f + taut * (float)h;
+    // 1/g to about an ulp: the float reciprocal and one cubic step
+    const double g = (double)d.g, r0 = (double)__builtin_amdgcn_rcpf(d.g);
+    const double e = __builtin_fma(-g, r0, 1.0);
+    d.r = __builtin_fma(__builtin_fma(e, e, e), r0, r0);
+    return d;
+}
+
+// The dual update of one pixel: p = (p + taut*grad u)/(1 + taut*|grad u|)
+// for both components (cblas_saxpy, then the division, tvl1.cpp:280-291).
+// The kernels are bound by VALU issue and this is the larger half of an
+// iteration, so it runs without the IEEE sequences (per pixel 2 roots of 21
+// instructions' cost and 4 divisions of 10): the root is refined once and
+// rounded, the quotients are products with a shared double reciprocal.  A
+// float quotient is never within 2^-49 of a rounding boundary and the product
+// is within 2^-52 of it, so the bits are the division's; a subnormal quotient
+// can lie on a boundary only if g is an even integer, and for 2 and 4 the
+// reciprocal is exact.  Roots near a boundary, g >= 6, infinities and NaN take
+// the full sequences, for the whole wave (the roots of about one row in 8000).
+__device__ __forceinline__ void dual_step(float fx1, float fy1, float fx2, float fy2, float taut,
+                                          float& p11, float& p12, float& p21, float& p22)
+{
+    const float n11 = p11 + taut * fx1, n12 = p12 + taut * fy1;
+    const float n21 = p21 + taut * fx2, n22 = p22 + taut * fy2;
+    const DualDiv a = dual_div(fx1, fy1, taut), b = dual_div(fx2, fy2, taut);
+    const bool sure = (a.g < 6.0f) & (b.g < 6.0f) & (min(a.near, b.near) >= (1u << 12)) & (taut < 0x1p40f);
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(!sure) == 0ull, 1)) {
+        p11 = (float)((double)n11 * a.r);
+        p12 = (float)((double)n12 * a.r);
+        p21 = (float)((double)n21 * b.r);
+        p22 = (float)((double)n22 * b.r);
+    } else {
+        const float g1 = 1.0f + taut * hypot_fin(fx1, fy1);
+        const float g2 = 1.0f + taut * hypot_fin(fx2, fy2);
+        p11 = n11 / g1;
+        p12 = n12 / g1;
+        p21 = n21 / g2;
+        p22 = n22 / g2;
+    }
+}
+
+// v plus the value of the lane that the DPP control names (0 where there is
+// none or the row mask excludes the lane).
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add_f64(double v)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, true);
+    const unsigned hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, true);
+    return v + __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// Sum over the wave, valid in lane 63: rows of 16 by shifts, then the rows'
+// totals broadcast.  DPP moves instead of cross-lane LDS permutes: the sums of
+// a tile's errors run once per tile and chunk (1920x1080, 2 iterations per
+// chunk: a seventh of a tile's instructions before).
 __device__ __forceinline__ double wave_sum_f64(double v)
 {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    v = dpp_add_f64<0x111, 0xf>(v);   // row_shr:1
+    v = dpp_add_f64<0x112, 0xf>(v);   // row_shr:2
+    v = dpp_add_f64<0x114, 0xf>(v);   // row_shr:4
+    v = dpp_add_f64<0x118, 0xf>(v);   // row_shr:8
+    v = dpp_add_f64<0x142, 0xa>(v);   // row_bcast:15 into rows 1 and 3
+    return dpp_add_f64<0x143, 0xc>(v);   // row_bcast:31 into rows 2 and 3
 }
+
+// A value that every lane holds alike, in a scalar register: what depends on
+// it (buffer pointers, tile addresses, loop exits) stays scalar too.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// Widest frame whose tile rows are addressed by 32-bit lane offsets (8 rows
+// of 4-byte values stay below 2^32 bytes).
+constexpr int kMaxLaneCols = 1 << 26;
+
+// A plane at an element offset, kept in scalar registers: accesses relative to
+// it take a 32-bit lane offset.  (Otherwise the compiler adds the lane to each
+// plane's base ahead of the loops, in vector registers, and the offset with
+// 64-bit vector instructions per access.)
+struct PlanePtr {
+    typedef __attribute__((address_space(1))) char gchar;
+    typedef __attribute__((address_space(1))) float gfloat;
+    gchar* p;
+    __device__ __forceinline__ PlanePtr(const float* plane, ptrdiff_t o) : p((gchar*)(plane + o))
+    {
+        asm("" : "+s"(p));
+    }
+    __device__ __forceinline__ gfloat* at(unsigned bytes) const { return (gfloat*)(p + bytes); }
+};
 
 // Loads and stores of the iteration state.  COH: device-scope atomic
 // accesses, coherent across XCDs without cache maintenance (used when other
 // workgroups of the same launch read the values).
-template <bool COH>
-__device__ __forceinline__ float ld(const float* p)
+template <bool COH, class P>
+__device__ __forceinline__ float ld(const P* p)
 {
     if constexpr (COH) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else return *p;
 }
 
-template <bool COH>
-__device__ __forceinline__ void st(float* p, float v)
+template <bool COH, class P>
+__device__ __forceinline__ void st(P* p, float v)
 {
     if constexpr (COH) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     else *p = v;
 }
 
-// Called by every thread of a tile's workgroup between its iterations and
-// its stores: false discards the tile's results (the neighbour-synchronised
-// warping checks its speculative chunk there).  The default stores always.
-struct StoreAlways {
-    __device__ bool operator()() const { return true; }
+// Called by every thread of a tile's workgroup.  ready(): before the loads of
+// the state (the warping's constants are on their way by then); store():
+// between the iterations and the stores.  false ends the tile there (the
+// neighbour-synchronised warping waits for its neighbours and checks its
+// speculative chunk in them).  The default does neither.
+struct NoSync {
+    __device__ bool ready() const { return true; }
+    __device__ bool store() const { return true; }
 };
 
 // One LDS row per wave and exchanged quantity; NW waves per workgroup.
@@ -103,20 +213,24 @@ using TileShared = TileSharedN<4>;
 // registers or, across waves, from one LDS row.  Values within K pixels of
 // the tile edge go stale one pixel per iteration; the central (64-2K) x
 // (NW*R-2K) pixels are exact.
-template <int K, int R, bool COH, bool INNER, int NW, class Pre>
+template <int K, int R, bool COH, bool INNER, int NW, class Sync>
 __device__ __forceinline__ void tile_iterate_impl(const IterArgs& a, int bx, int by, int cur, int kk,
-                                                  double (&acc)[K], TileSharedN<NW>& sh, Pre& pre)
+                                                  double (&acc)[K], TileSharedN<NW>& sh, Sync& sync)
 {
     constexpr int TW = 64 - 2 * K;
     constexpr int TH = NW * R - 2 * K;
+    bx = uniform(bx);
+    by = uniform(by);
+    cur = uniform(cur);
     const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform
+    const int wave = uniform(threadIdx.x >> 6);
     const int nx = a.nx, ny = a.ny;
     const int x = bx * TW - K + lane;
     const int ybase = by * TH - K + wave * R;
     const int oy0 = by * TH;
     // INNER: the extended tile lies within columns 1..nx-2 and rows 1..ny-2,
-    // so every border test below is known and folds away
+    // so every border test below is known and folds away, and the frame is
+    // at most kMaxLaneCols wide
     const bool xin = INNER || (x >= 0 && x < nx);
     const bool xout = xin && lane >= K && lane < K + TW;
     const bool fc = !INNER && x == 0, lc = !INNER && x == nx - 1;
@@ -124,28 +238,62 @@ __device__ __forceinline__ void tile_iterate_impl(const IterArgs& a, int bx, int
     // divergence on every row away from the first/last image row
     const bool edge_cols = !INNER && __any(fc || lc);
 
-    const float* uin = a.u[cur];
-    const float* pin = a.p[cur];
+    // (selects: an indexed kernel argument would be loaded per lane)
+    const float* uin = cur ? a.u[1] : a.u[0];
+    const float* pin = cur ? a.p[1] : a.p[0];
     const size_t plane = (size_t)a.plane;
 
     float u1[R], u2[R], p11[R], p12[R], p21[R], p22[R], gx[R], gy[R], rc[R];
+    const ptrdiff_t o0 = (ptrdiff_t)ybase * nx + (bx * TW - K);   // the wave's first pixel
+    const unsigned ob = (unsigned)lane * 4u, onx = (unsigned)nx * 4u;
+    if constexpr (INNER) {
+        const PlanePtr GX(a.wx, o0), GY(a.wy, o0), RC(a.rhoc, o0);
 #pragma unroll
-    for (int r = 0; r < R; r++) {
-        const int y = ybase + r;
-        if (INNER || (xin && y >= 0 && y < ny)) {
-            const size_t idx = (size_t)y * nx + x;
-            u1[r] = ld<COH>(uin + idx);
-            u2[r] = ld<COH>(uin + plane + idx);
-            p11[r] = ld<COH>(pin + idx);
-            p12[r] = ld<COH>(pin + plane + idx);
-            p21[r] = ld<COH>(pin + 2 * plane + idx);
-            p22[r] = ld<COH>(pin + 3 * plane + idx);
-            gx[r] = a.wx[idx];
-            gy[r] = a.wy[idx];
-            rc[r] = a.rhoc[idx];
-        } else {
-            u1[r] = u2[r] = p11[r] = p12[r] = p21[r] = p22[r] = 0.0f;
+        for (int r = 0; r < R; r++) {
+            const unsigned o = ob + (unsigned)r * onx;
+            gx[r] = *GX.at(o);
+            gy[r] = *GY.at(o);
+            rc[r] = *RC.at(o);
+        }
+        if (!sync.ready()) return;
+        const PlanePtr U1(uin, o0), U2(uin + plane, o0), P11(pin, o0), P12(pin + plane, o0),
+            P21(pin + 2 * plane, o0), P22(pin + 3 * plane, o0);
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const unsigned o = ob + (unsigned)r * onx;
+            u1[r] = ld<COH>(U1.at(o));
+            u2[r] = ld<COH>(U2.at(o));
+            p11[r] = ld<COH>(P11.at(o));
+            p12[r] = ld<COH>(P12.at(o));
+            p21[r] = ld<COH>(P21.at(o));
+            p22[r] = ld<COH>(P22.at(o));
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int y = ybase + r;
             gx[r] = gy[r] = rc[r] = 0.0f;
+            if (xin && y >= 0 && y < ny) {
+                const size_t idx = (size_t)y * nx + x;
+                gx[r] = a.wx[idx];
+                gy[r] = a.wy[idx];
+                rc[r] = a.rhoc[idx];
+            }
+        }
+        if (!sync.ready()) return;
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int y = ybase + r;
+            u1[r] = u2[r] = p11[r] = p12[r] = p21[r] = p22[r] = 0.0f;
+            if (xin && y >= 0 && y < ny) {
+                const size_t idx = (size_t)y * nx + x;
+                u1[r] = ld<COH>(uin + idx);
+                u2[r] = ld<COH>(uin + plane + idx);
+                p11[r] = ld<COH>(pin + idx);
+                p12[r] = ld<COH>(pin + plane + idx);
+                p21[r] = ld<COH>(pin + 2 * plane + idx);
+                p22[r] = ld<COH>(pin + 3 * plane + idx);
+            }
         }
     }
 
@@ -162,8 +310,8 @@ __device__ __forceinline__ void tile_iterate_impl(const IterArgs& a, int bx, int
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 const int y = ybase + r;
-                const float p11l = from_left(p11[r]);
-                const float p21l = from_left(p21[r]);
+                const float p11l = lane_left(p11[r]);
+                const float p21l = lane_left(p21[r]);
                 const float p12u = r ? p12[r - 1] : up12;
                 const float p22u = r ? p22[r - 1] : up22;
                 const bool fr = !INNER && y == 0, lr = !INNER && y == ny - 1;
@@ -182,7 +330,7 @@ __device__ __forceinline__ void tile_iterate_impl(const IterArgs& a, int bx, int
                 const float e1 = nu1 - u1[r], e2 = nu2 - u2[r];
                 const float e = e1 * e1 + e2 * e2;
                 const bool mine = xout && y >= oy0 && y < oy0 + TH && (INNER || y < ny);
-                acc[t] += mine ? (double)e : 0.0;
+                acc[t] += (double)(mine ? e : 0.0f);
                 u1[r] = nu1;
                 u2[r] = nu2;
             }
@@ -195,8 +343,8 @@ __device__ __forceinline__ void tile_iterate_impl(const IterArgs& a, int bx, int
 #pragma unroll
             for (int r = 0; r < R; r++) {
                 const int y = ybase + r;
-                const float u1r = from_right(u1[r]);
-                const float u2r = from_right(u2[r]);
+                const float u1r = lane_right(u1[r]);
+                const float u2r = lane_right(u2[r]);
                 const float u1d = r < R - 1 ? u1[r + 1] : dn1;
                 const float u2d = r < R - 1 ? u2[r + 1] : dn2;
                 const bool xl = INNER || x < nx - 1, yl = INNER || y < ny - 1;
@@ -204,25 +352,36 @@ __device__ __forceinline__ void tile_iterate_impl(const IterArgs& a, int bx, int
                 const float fy1 = yl ? u1d - u1[r] : 0.0f;
                 const float fx2 = xl ? u2r - u2[r] : 0.0f;
                 const float fy2 = yl ? u2d - u2[r] : 0.0f;
-                const float g1 = 1.0f + taut * hypot_fin(fx1, fy1);
-                const float g2 = 1.0f + taut * hypot_fin(fx2, fy2);
-                // cblas_saxpy (p += taut*grad) then the division, tvl1.cpp:280-291
-                p11[r] = (p11[r] + taut * fx1) / g1;
-                p12[r] = (p12[r] + taut * fy1) / g1;
-                p21[r] = (p21[r] + taut * fx2) / g2;
-                p22[r] = (p22[r] + taut * fy2) / g2;
+                dual_step(fx1, fy1, fx2, fy2, taut, p11[r], p12[r], p21[r], p22[r]);
             }
         }
     }
 
-    if (!pre()) return;
-    float* uout = a.u[cur ^ 1];
-    float* pout = a.p[cur ^ 1];
-    if (xout) {
+    if (!sync.store()) return;
+    float* uout = cur ? a.u[0] : a.u[1];
+    float* pout = cur ? a.p[0] : a.p[1];
+    if (!xout) return;
+    if constexpr (INNER) {
+        const PlanePtr U1(uout, o0), U2(uout + plane, o0), P11(pout, o0), P12(pout + plane, o0),
+            P21(pout + 2 * plane, o0), P22(pout + 3 * plane, o0);
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int y = ybase + r;
-            if (y >= oy0 && y < oy0 + TH && (INNER || y < ny)) {
+            if (y >= oy0 && y < oy0 + TH) {
+                const unsigned o = ob + (unsigned)r * onx;
+                st<COH>(U1.at(o), u1[r]);
+                st<COH>(U2.at(o), u2[r]);
+                st<COH>(P11.at(o), p11[r]);
+                st<COH>(P12.at(o), p12[r]);
+                st<COH>(P21.at(o), p21[r]);
+                st<COH>(P22.at(o), p22[r]);
+            }
+        }
+    } else {
+#pragma unroll
+        for (int r = 0; r < R; r++) {
+            const int y = ybase + r;
+            if (y >= oy0 && y < oy0 + TH && y < ny) {
                 const size_t idx = (size_t)y * nx + x;
                 st<COH>(uout + idx, u1[r]);
                 st<COH>(uout + plane + idx, u2[r]);
@@ -237,16 +396,17 @@ __device__ __forceinline__ void tile_iterate_impl(const IterArgs& a, int bx, int
 
 // Tiles whose extended area (64 columns x 4R rows from (bx*TW-K, by*TH-K))
 // stays clear of the image border run the INNER variant.
-template <int K, int R, bool COH, int NW, class Pre = StoreAlways>
+template <int K, int R, bool COH, int NW, class Sync>
 __device__ __forceinline__ void tile_iterate(const IterArgs& a, int bx, int by, int cur, int kk,
-                                             double (&acc)[K], TileSharedN<NW>& sh, Pre pre = Pre{})
+                                             double (&acc)[K], TileSharedN<NW>& sh, Sync& sync)
 {
     constexpr int TW = 64 - 2 * K;
     constexpr int TH = NW * R - 2 * K;
     const int x0 = bx * TW - K, y0 = by * TH - K;
-    const bool inner = x0 >= 1 && x0 + 63 <= a.nx - 2 && y0 >= 1 && y0 + NW * R - 1 <= a.ny - 2;
-    if (inner) tile_iterate_impl<K, R, COH, true, NW>(a, bx, by, cur, kk, acc, sh, pre);
-    else tile_iterate_impl<K, R, COH, false, NW>(a, bx, by, cur, kk, acc, sh, pre);
+    const bool inner = x0 >= 1 && x0 + 63 <= a.nx - 2 && y0 >= 1 && y0 + NW * R - 1 <= a.ny - 2 &&
+                       a.nx <= kMaxLaneCols;
+    if (inner) tile_iterate_impl<K, R, COH, true, NW>(a, bx, by, cur, kk, acc, sh, sync);
+    else tile_iterate_impl<K, R, COH, false, NW>(a, bx, by, cur, kk, acc, sh, sync);
 }
 
 // Square tiles for the small scales: one workgroup of 256 lanes covers a
@@ -271,9 +431,9 @@ struct SqShared {
 // term over the central tile to acc[t].  Same per-pixel expressions as
 // tile_iterate_impl; pixels outside the image never feed pixels inside (the
 // border rules do not read across the border).
-template <int K, bool COH, class Pre = StoreAlways>
+template <int K, bool COH, class Sync>
 __device__ __forceinline__ void tile_iterate_sq(const IterArgs& a, int bx, int by, int cur, int kk,
-                                                double (&acc)[K], SqShared& sh, Pre pre = Pre{})
+                                                double (&acc)[K], SqShared& sh, Sync& sync)
 {
     constexpr int T = kSqTile, C = T - 2 * K;
     const int lx = threadIdx.x % T, ly = threadIdx.x / T;
@@ -283,10 +443,16 @@ __device__ __forceinline__ void tile_iterate_sq(const IterArgs& a, int bx, int b
     const bool mine = in && lx >= K && lx < K + C && ly >= K && ly < K + C;
     const size_t plane = (size_t)a.plane;
     const size_t idx = (size_t)y * nx + x;
-    const float* uin = a.u[cur];
-    const float* pin = a.p[cur];
+    const float* uin = cur ? a.u[1] : a.u[0];
+    const float* pin = cur ? a.p[1] : a.p[0];
     float u1 = 0.0f, u2 = 0.0f, p11 = 0.0f, p12 = 0.0f, p21 = 0.0f, p22 = 0.0f;
     float gx = 0.0f, gy = 0.0f, rc = 0.0f;
+    if (in) {
+        gx = a.wx[idx];
+        gy = a.wy[idx];
+        rc = a.rhoc[idx];
+    }
+    if (!sync.ready()) return;
     if (in) {
         u1 = ld<COH>(uin + idx);
         u2 = ld<COH>(uin + plane + idx);
@@ -294,9 +460,6 @@ __device__ __forceinline__ void tile_iterate_sq(const IterArgs& a, int bx, int b
         p12 = ld<COH>(pin + plane + idx);
         p21 = ld<COH>(pin + 2 * plane + idx);
         p22 = ld<COH>(pin + 3 * plane + idx);
-        gx = a.wx[idx];
-        gy = a.wy[idx];
-        rc = a.rhoc[idx];
     }
     const bool fc = x == 0, lc = x == nx - 1, fr = y == 0, lr = y == ny - 1;
     // neighbour slots, clamped to the tile: the edge lanes read their own
@@ -324,7 +487,7 @@ __device__ __forceinline__ void tile_iterate_sq(const IterArgs& a, int bx, int b
             const float nu2 = v2 + theta * div2;
             const float e1 = nu1 - u1, e2 = nu2 - u2;
             const float e = e1 * e1 + e2 * e2;
-            acc[t] += mine ? (double)e : 0.0;
+            acc[t] += (double)(mine ? e : 0.0f);
             u1 = nu1;
             u2 = nu2;
             // ---- p update: forward gradient of u, g, p = (p + taut*grad)/g ----
@@ -337,19 +500,13 @@ __device__ __forceinline__ void tile_iterate_sq(const IterArgs& a, int bx, int b
             const float fy1 = yl ? u1d - u1 : 0.0f;
             const float fx2 = xl ? u2r - u2 : 0.0f;
             const float fy2 = yl ? u2d - u2 : 0.0f;
-            const float g1 = 1.0f + taut * hypot_fin(fx1, fy1);
-            const float g2 = 1.0f + taut * hypot_fin(fx2, fy2);
-            // cblas_saxpy (p += taut*grad) then the division, tvl1.cpp:280-291
-            p11 = (p11 + taut * fx1) / g1;
-            p12 = (p12 + taut * fy1) / g1;
-            p21 = (p21 + taut * fx2) / g2;
-            p22 = (p22 + taut * fy2) / g2;
+            dual_step(fx1, fy1, fx2, fy2, taut, p11, p12, p21, p22);
         }
     }
-    if (!pre()) return;
+    if (!sync.store()) return;
     if (mine) {
-        float* uout = a.u[cur ^ 1];
-        float* pout = a.p[cur ^ 1];
+        float* uout = cur ? a.u[0] : a.u[1];
+        float* pout = cur ? a.p[0] : a.p[1];
         st<COH>(uout + idx, u1);
         st<COH>(uout + plane + idx, u2);
         st<COH>(pout + idx, p11);
@@ -369,7 +526,7 @@ __device__ __forceinline__ double block_sum(const double (&acc)[K], double (*sh_
 #pragma unroll
     for (int t = 0; t < K; t++) {
         const double v = wave_sum_f64(acc[t]);
-        if (lane == 0) sh_err[wave][t] = v;
+        if (lane == 63) sh_err[wave][t] = v;
     }
     __syncthreads();
     double s = 0.0;
@@ -406,7 +563,7 @@ __device__ __forceinline__ void grid_sums(const double* part, unsigned nb, int k
 #pragma unroll
     for (int t = 0; t < K; t++) {
         const double v = wave_sum_f64(s[t]);
-        if (lane == 0) sh[t * NW + wave] = v;
+        if (lane == 63) sh[t * NW + wave] = v;
     }
     __syncthreads();
     if (threadIdx.x < (unsigned)K) {
@@ -443,16 +600,15 @@ constexpr int kIterBlocksPerCU = 3;
 // which hides the latency of an iteration better than 4 waves of R rows:
 // host-paced, every shape was faster at every scale of a 1920x1080 pyramid
 // (e.g. (4,4) at 480x270: 5.22 -> 4.87 us per iteration; (4,8) at 960x540:
-// 9.29 -> 8.18 us).  OF_ITER_BOUNDS asks for at least 2 waves per SIMD
-// (its second argument counts waves per SIMD, not workgroups per CU); the
-// 8-wave kernels hold 2 workgroups per CU wherever they stay within 128
-// VGPRs, which all shapes but (8,8) do.
+// 9.29 -> 8.18 us).  OF_ITER_BOUNDS asks for 4 waves per SIMD (its second
+// argument counts waves per SIMD, not workgroups per CU), 128 VGPRs, so that 2
+// workgroups of 8 waves share a CU; all shapes but (8,8) fit without spills.
 constexpr int kIterWaves = 8;
 // The lockstep batch kernel keeps 4 waves of R rows: with 8 waves of R/2 the
 // batch of 64 mixed-size pairs took 79.0 ms instead of 75.7 ms (same box).
 constexpr int kLsWaves = 4;
 // __launch_bounds__(threads, minimum waves per SIMD)
-#define OF_ITER_BOUNDS(NW) __launch_bounds__(64 * (NW), (NW) == 4 ? kIterBlocksPerCU : 2)
+#define OF_ITER_BOUNDS(NW, K) __launch_bounds__(64 * (NW), (NW) == 4 ? kIterBlocksPerCU : (K) == 8 ? 2 : 4)
 
 // ---------------------------------------------------------------------------
 // launch-per-chunk driver
@@ -463,7 +619,7 @@ constexpr int kLsWaves = 4;
 // iteration, the launch's output is discarded and the next launch re-runs
 // exactly that many iterations from the same input buffer.
 template <int K, int R, int NW = 4, bool SQ = false>
-__global__ OF_ITER_BOUNDS(NW) void k_tvl1_iter(IterArgs a)
+__global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_iter(IterArgs a)
 {
     __shared__ TileSharedN<NW> sh;
     __shared__ SqShared sh_sq;
@@ -474,18 +630,19 @@ __global__ OF_ITER_BOUNDS(NW) void k_tvl1_iter(IterArgs a)
 
     TvCtl* ctl = a.ctl;
     if (ctl->stop) return;
-    const int cur = ctl->cur[a.level];
-    const int redo = ctl->redo;
-    const int n0 = ctl->n;
+    const int cur = uniform(ctl->cur[a.level]);
+    const int redo = uniform(ctl->redo);
+    const int n0 = uniform(ctl->n);
     int kk = redo ? redo : a.max_iter - n0;
     if (kk > K) kk = K;
     if (kk <= 0) return;
 
+    NoSync no_sync;
     double acc[K];
 #pragma unroll
     for (int t = 0; t < K; t++) acc[t] = 0.0;
-    if constexpr (SQ) tile_iterate_sq<K, false>(a, blockIdx.x, blockIdx.y, cur, kk, acc, sh_sq);
-    else tile_iterate<K, R, false, NW>(a, blockIdx.x, blockIdx.y, cur, kk, acc, sh);
+    if constexpr (SQ) tile_iterate_sq<K, false>(a, blockIdx.x, blockIdx.y, cur, kk, acc, sh_sq, no_sync);
+    else tile_iterate<K, R, false, NW>(a, blockIdx.x, blockIdx.y, cur, kk, acc, sh, no_sync);
 
     const unsigned nblocks = gridDim.x * gridDim.y;
     const unsigned bid = blockIdx.y * gridDim.x + blockIdx.x;
@@ -615,7 +772,7 @@ __device__ __forceinline__ bool grid_barrier(TvCtl* ctl, unsigned nb, unsigned& 
         *sh_ok = ok;
     }
     __syncthreads();
-    return *sh_ok != 0;
+    return uniform(*sh_ok) != 0;
 }
 
 // Two-level grid barrier, for grids of many workgroups (the square-tile
@@ -693,7 +850,7 @@ __device__ __forceinline__ bool grid_barrier2(TvCtl* ctl, unsigned nb, BarEpoch&
         *sh_ok = ok;
     }
     __syncthreads();
-    return *sh_ok != 0;
+    return uniform(*sh_ok) != 0;
 }
 
 // A whole warping: chunks of K iterations over all tiles (workgroup b takes
@@ -705,7 +862,7 @@ __device__ __forceinline__ bool grid_barrier2(TvCtl* ctl, unsigned nb, BarEpoch&
 // other XCDs are seen without cache maintenance.  Partials are
 // double-buffered by chunk parity.
 template <int K, int R, int NW = 4, bool SQ = false>
-__global__ OF_ITER_BOUNDS(NW) void k_tvl1_persist(IterArgs a, unsigned tiles_x, unsigned ntiles)
+__global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist(IterArgs a, unsigned tiles_x, unsigned ntiles)
 {
     __shared__ TileSharedN<NW> sh;
     __shared__ SqShared sh_sq;
@@ -724,12 +881,13 @@ __global__ OF_ITER_BOUNDS(NW) void k_tvl1_persist(IterArgs a, unsigned tiles_x, 
         ep.grp = __hip_atomic_load(&ctl->grp_gen[blockIdx.x % kBarGroups].v, __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
     }
-    int cur = ctl->cur[a.level];
+    int cur = uniform(ctl->cur[a.level]);
     int n = 0;
     int redo = 0;
     int parity = 0;
     // the first barrier of a plain launch also checks that the grid is resident
     FirstBound fb{a.resident_ticks, a.force_not_resident};
+    NoSync no_sync;
     while (true) {
         int kk = redo ? redo : a.max_iter - n;
         if (kk > K) kk = K;
@@ -739,9 +897,9 @@ __global__ OF_ITER_BOUNDS(NW) void k_tvl1_persist(IterArgs a, unsigned tiles_x, 
         for (int t = 0; t < K; t++) acc[t] = 0.0;
         for (unsigned tile = blockIdx.x; tile < ntiles; tile += nb)
             if constexpr (SQ)
-                tile_iterate_sq<K, true>(a, (int)(tile % tiles_x), (int)(tile / tiles_x), cur, kk, acc, sh_sq);
+                tile_iterate_sq<K, true>(a, (int)(tile % tiles_x), (int)(tile / tiles_x), cur, kk, acc, sh_sq, no_sync);
             else
-                tile_iterate<K, R, true, NW>(a, (int)(tile % tiles_x), (int)(tile / tiles_x), cur, kk, acc, sh);
+                tile_iterate<K, R, true, NW>(a, (int)(tile % tiles_x), (int)(tile / tiles_x), cur, kk, acc, sh, no_sync);
         if (redo) {   // the re-run chunk is final: no decision needed
             n += redo;
             cur ^= 1;
@@ -757,7 +915,7 @@ __global__ OF_ITER_BOUNDS(NW) void k_tvl1_persist(IterArgs a, unsigned tiles_x, 
             return;
         fb = FirstBound{0ull, 0};
         grid_sums<K, NW>(pp, nb, kk, sh4, sh_tot);
-        const int keep = stop_after(sh_tot, kk, n, a);
+        const int keep = uniform(stop_after(sh_tot, kk, n, a));
         if (a.err_log && blockIdx.x == 0 && threadIdx.x < (unsigned)kk)
             a.err_log[n + threadIdx.x] = sh_tot[threadIdx.x];
         parity ^= 1;
@@ -785,101 +943,172 @@ __global__ OF_ITER_BOUNDS(NW) void k_tvl1_persist(IterArgs a, unsigned tiles_x, 
 // neighbour-synchronised persistent driver
 // ---------------------------------------------------------------------------
 
-// Bounded wait of one thread until the 64-bit word at `w` reaches `want`
-// (the words only grow within a warping).  Returns false after flagging
-// kBarTimeout past ~1 s of polls, after the first bound (kBarNotResident),
-// or once another workgroup has flagged an error.
-__device__ __forceinline__ bool word_wait_ge(const unsigned long long* w, unsigned long long want,
-                                             TvCtl* ctl, const FirstBound& fb)
+// Bounded wait of one wave until every lane's 64-bit word at `w` (lanes with a
+// null pointer have none) reaches `want`; the words only grow within a
+// warping.  Returns 1 then, 2 once the referee has published that the
+// warping stops, 0 after flagging kBarTimeout past ~1 s of polls, after the
+// first bound (kBarNotResident), or once another workgroup has flagged an
+// error.
+__device__ __forceinline__ int wave_wait(const IterArgs& a, const unsigned long long* w,
+                                         unsigned long long want, const FirstBound& fb)
 {
+    TvCtl* ctl = a.ctl;
     const unsigned long long t_end = fb.ticks ? (unsigned long long)wall_clock64() + fb.ticks : 0ull;
     if (fb.force) {
         __hip_atomic_store(&ctl->error, kBarNotResident, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        return false;
+        return 0;
     }
     unsigned spins = 0;
-    while (__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want) {
+    while (true) {
+        const bool wait = w && __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want;
+        if (!__any(wait)) return 1;
+        if ((spins & 3u) == 3u) {
+            bool stopped = false;
+            if ((threadIdx.x & 63) < 2) {
+                const unsigned long long d = __hip_atomic_load(&ctl->decision[threadIdx.x & 1].v,
+                                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                stopped = (d >> 24) == a.seq && (d & 0xFull) != 0;
+            }
+            if (__any(stopped)) return 2;
+        }
         __builtin_amdgcn_s_sleep(1);
         if (++spins > (1u << 21)) {
             __hip_atomic_store(&ctl->error, kBarTimeout, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            return false;
+            return 0;
         }
-        if (past_first_bound(fb, t_end, spins, ctl)) return false;
+        if (past_first_bound(fb, t_end, spins, ctl)) return 0;
         if ((spins & 1023u) == 0 &&
             __hip_atomic_load(&ctl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            return false;
+            return 0;
     }
-    return true;
 }
 
-// The referee's bounded wait for a chunk's counter to reach `want`.
-__device__ __forceinline__ bool count_wait(const unsigned* w, unsigned want, TvCtl* ctl)
-{
-    unsigned spins = 0;
-    while (__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want) {
-        __builtin_amdgcn_s_sleep(1);
-        if (++spins > (1u << 21)) {
-            __hip_atomic_store(&ctl->error, kBarTimeout, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// Synchronisation of one workgroup of k_tvl1_persist_nbr with the others.
+// `stop_chunk`/`stop_keep`: set once the warping is known to stop after
+// stop_keep iterations of chunk stop_chunk.  Members are uniform.
+struct NbrSync {
+    const IterArgs& a;
+    FirstBound fb;   // the first wait of a plain launch also checks that the grid is resident
+    int* sh;         // LDS word for results of wave 0
+    unsigned tiles_x, tiles_y, tile;
+    int c;           // chunk of the current tile
+    int seen;        // decisions up to this chunk are known to continue
+    int stop_chunk, stop_keep;
+    bool failed;
+    bool rerun;      // the last pass: no waits, every tile is stored
+
+    // Result of wave 0's wait, in every thread.  The first barrier also
+    // orders the waits of a workgroup's earlier LDS reads of the word.
+    __device__ __forceinline__ int share(int r)
+    {
+        __syncthreads();
+        if (threadIdx.x == 0) *sh = r;
+        __syncthreads();
+        fb = FirstBound{0ull, 0};
+        return uniform(*sh);
+    }
+
+    __device__ __forceinline__ int wait(const unsigned long long* w, unsigned long long want)
+    {
+        return share(threadIdx.x < 64 ? wave_wait(a, w, want, fb) : 0);
+    }
+
+    // Decision of chunk q once published: keep, or -1 if the wait failed.
+    __device__ __forceinline__ int decision(int q)
+    {
+        int r = -1;
+        if (threadIdx.x < 64) {
+            const unsigned long long* w = &a.ctl->decision[q & 1].v;
+            if (wave_wait(a, threadIdx.x == 0 ? w : nullptr, (a.seq << 24) | ((unsigned long long)(q + 1) << 4), fb))
+                r = (int)(__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFull);
+        }
+        return share(r);
+    }
+
+    // The published stop (chunk, keep), if any.
+    __device__ __forceinline__ void read_stop()
+    {
+        for (int q = 0; q < 2; q++) {
+            unsigned long long d = 0ull;
+            if (threadIdx.x == 0)
+                d = __hip_atomic_load(&a.ctl->decision[q].v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            const int r = share((int)((d >> 24) == a.seq ? (unsigned)(d & 0xFFFFFFull) : 0u));
+            if (r & 15) {
+                stop_chunk = (r >> 4) - 1;
+                stop_keep = r & 15;
+            }
+        }
+    }
+
+    // The tile may start chunk c once its (up to) 8 neighbours have completed
+    // chunk c-1: its extended tile reads their centres, and its stores
+    // overwrite values their chunk c-1 read.  Lanes 0..8 poll one tile each.
+    __device__ __forceinline__ bool ready()
+    {
+        if (c == 0 || rerun) return true;
+        const unsigned long long* w = nullptr;
+        if (threadIdx.x < 9 && threadIdx.x != 4) {
+            const int x = (int)(tile % tiles_x) + (int)(threadIdx.x % 3) - 1;
+            const int y = (int)(tile / tiles_x) + (int)(threadIdx.x / 3) - 1;
+            if (x >= 0 && y >= 0 && x < (int)tiles_x && y < (int)tiles_y)
+                w = a.tile_flags + (size_t)y * tiles_x + x;
+        }
+        const int r = wait(w, (a.seq << 20) | (unsigned)c);
+        if (r == 2) read_stop();
+        failed |= r == 0;
+        return r == 1;
+    }
+
+    // Decision c-1 before a store of chunk c: false discards the tile.
+    __device__ __forceinline__ bool store()
+    {
+        if (c == 0 || seen >= c - 1 || rerun) return true;
+        const int r = decision(c - 1);
+        failed |= r < 0;
+        if (r < 0) return false;
+        if (r) {
+            stop_chunk = c - 1;
+            stop_keep = r;
             return false;
         }
-        if ((spins & 1023u) == 0 &&
-            __hip_atomic_load(&ctl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-            return false;
+        seen = c - 1;
+        return true;
     }
-    return true;
-}
 
-// Tile (bx, by) may start chunk c once its (up to) 8 neighbours have
-// completed chunk c-1: its extended tile reads their centres, and its
-// stores overwrite values their chunk c-1 read.  Threads 0..8 poll one
-// neighbour each; the workgroup learns whether every wait ended normally.
-__device__ __forceinline__ bool wait_neighbours(const IterArgs& a, unsigned tiles_x, unsigned tiles_y,
-                                                int bx, int by, int c, const FirstBound& fb)
-{
-    int ok = 1;
-    const unsigned t = threadIdx.x;
-    if (t < 9 && t != 4) {
-        const int x = bx + (int)(t % 3) - 1, y = by + (int)(t / 3) - 1;
-        if (x >= 0 && y >= 0 && x < (int)tiles_x && y < (int)tiles_y)
-            ok = word_wait_ge(a.tile_flags + (size_t)y * tiles_x + x, (a.seq << 20) | (unsigned)c,
-                              a.ctl, fb);
+    // Past the last chunk: its decision stops the warping.
+    __device__ __forceinline__ void last(int nchunks)
+    {
+        const int r = decision(nchunks - 1);
+        failed |= r < 0;
+        stop_chunk = nchunks - 1;
+        stop_keep = r;
     }
-    return __syncthreads_and(ok) != 0;
-}
-
-// The stopping decision of chunk c as published by the referee workgroup:
-// keep (0: continue) in every thread, or -1 if the wait failed.
-__device__ __forceinline__ int wait_decision(const IterArgs& a, int c, int parity, const FirstBound& fb,
-                                             int* sh_keep)
-{
-    if (threadIdx.x == 0) {
-        const unsigned long long want = (a.seq << 24) | ((unsigned long long)(c + 1) << 4);
-        const unsigned long long* w = &a.ctl->decision[parity].v;
-        *sh_keep = word_wait_ge(w, want, a.ctl, fb)
-                       ? (int)(__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFull)
-                       : -1;
-    }
-    __syncthreads();
-    const int keep = *sh_keep;
-    __syncthreads();
-    return keep;
-}
+};
 
 // A whole warping without grid barriers.  Workgroups 0..nbw-1 iterate tiles
 // (workgroup b takes tiles b, b+nbw, ...); a tile starts chunk c as soon as
 // its neighbours have completed chunk c-1 (per-tile flags), so no workgroup
-// waits for the whole grid.  Workgroup nbw is the referee: it waits for the
-// error partials of chunk c from every workgroup, sums them in the fixed
-// order of the barrier kernel (grid_sums), applies the stopping rule and
-// publishes the decision.  Tiles do not wait for it: they iterate chunk c+1
-// from chunk c's output and check decision c before their first store of
-// chunk c+1.  "Continue": they store as usual.  "Stop after keep
+// waits for the whole grid.  Workgroup nbw is the referee: once every
+// workgroup has completed its last tile of chunk c it sums their error
+// partials in the fixed order of the barrier kernel, applies the stopping
+// rule and publishes the decision.  Tiles do not wait for it: they iterate
+// chunk c+1 from chunk c's output and check decision c before their first
+// store of chunk c+1.  "Continue": they store as usual.  "Stop after keep
 // iterations": they discard chunk c+1, and if keep is short of chunk c's
 // length they re-run keep iterations from chunk c's input, which no store of
-// chunk c+1 has touched.  Same arithmetic, partial sums, order and
-// decisions as k_tvl1_persist, so the same bits and iteration counts.
+// chunk c+1 has touched.  Same arithmetic, partial sums and decisions as
+// k_tvl1_persist, so the same bits and iteration counts.
+// What a chunk costs beyond its arithmetic is the round trip to the neighbours
+// (stores, flag, flag read, loads) and the scalar work around it: one wave
+// polls for the workgroup, the warping's constants are loaded before the wait,
+// everything uniform stays in scalar registers.  With the shorter dual update,
+// 1920x1080 per scale (ms per solve): 2.12 -> 2.03, 960x540 (4,8) 1.04 ->
+// 0.96..0.99, 480x270 0.67 -> 0.63, 240x135 (4,4) 0.56 -> 0.54, 120x68 0.40
+// -> 0.32.  Dealing tiles to workgroups in rotation, so that all get the same
+// number, was 5% slower at 1920x1080: two workgroups with 2 and 3 tiles
+// already share a CU evenly.
 template <int K, int R, int NW = 4, bool SQ = false>
-__global__ OF_ITER_BOUNDS(NW) void k_tvl1_persist_nbr(IterArgs a, unsigned tiles_x, unsigned ntiles)
+__global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist_nbr(IterArgs a, unsigned tiles_x, unsigned ntiles)
 {
     static_assert(SQ ? (kSqTile - 2 * K >= K) : (NW * R - 2 * K >= K && 64 - 2 * K >= K),
                   "the halo of a tile must lie within its neighbours");
@@ -887,53 +1116,55 @@ __global__ OF_ITER_BOUNDS(NW) void k_tvl1_persist_nbr(IterArgs a, unsigned tiles
     __shared__ SqShared sh_sq;
     __shared__ double sh_err[NW][K];
     __shared__ double sh_tot[K];
-    __shared__ double sh4[K * NW];
-    __shared__ int sh_keep;
+    __shared__ int sh_word;
 
     TvCtl* ctl = a.ctl;
     const unsigned nbw = gridDim.x - 1;   // tile workgroups; the last one is the referee
-    const unsigned tiles_y = ntiles / tiles_x;
-    int cur = ctl->cur[a.level];
-    int n = 0, c = 0, parity = 0;
-    // the first wait of a plain launch also checks that the grid is resident
-    FirstBound fb{a.resident_ticks, a.force_not_resident};
+    const int cur0 = uniform(ctl->cur[a.level]);
+    const int nchunks = (a.max_iter + K - 1) / K;
 
     if (blockIdx.x == nbw) {   // referee
-        while (true) {
-            int kk = a.max_iter - n;
-            if (kk > K) kk = K;
-            if (kk <= 0) break;
-            if (threadIdx.x == 0) {
-                // every tile workgroup's first wait checks residency; the
-                // referee waits for chunk 0 of all of them without that bound
-                sh_keep = count_wait(&ctl->chunk_count[parity].v, nbw, ctl) ? 1 : 0;
-            }
-            __syncthreads();
-            if (!sh_keep) return;
-            const double* pp = a.partials + (size_t)parity * K * nbw;
-            grid_sums<K, NW>(pp, nbw, kk, sh4, sh_tot);
-            const int keep = stop_after(sh_tot, kk, n, a);
-            if (a.err_log && threadIdx.x < (unsigned)kk) a.err_log[n + threadIdx.x] = sh_tot[threadIdx.x];
-            if (threadIdx.x == 0) {
-                // the counter is reused two chunks on, by increments that
-                // follow this decision
-                __hip_atomic_store(&ctl->chunk_count[parity].v, 0u, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-                __builtin_amdgcn_s_waitcnt(0);
+        int n = 0, c = 0;
+        while (c < nchunks) {
+            const int kk = min(K, a.max_iter - n);
+            const double* pp = a.partials + (size_t)(c & 1) * K * nbw;
+            const unsigned long long want = (a.seq << 20) | (unsigned)(c + 1);
+            double s[K];
+#pragma unroll
+            for (int t = 0; t < K; t++) s[t] = 0.0;
+            bool ok = true;
+            for (unsigned j0 = threadIdx.x & ~63u; j0 < nbw && ok; j0 += 64 * NW) {
+                const unsigned j = j0 + (threadIdx.x & 63);   // workgroup
+                const bool mine = j < nbw;
+                const unsigned last = mine ? j + (ntiles - 1 - j) / nbw * nbw : 0u;
+                ok = wave_wait(a, mine ? a.tile_flags + last : nullptr, want, FirstBound{0ull, 0}) == 1;
                 __atomic_signal_fence(__ATOMIC_SEQ_CST);
-                __hip_atomic_store(&ctl->decision[parity].v,
+                if (ok && mine) {
+#pragma unroll
+                    for (int t = 0; t < K; t++)
+                        if (t < kk)
+                            s[t] += __hip_atomic_load(pp + (size_t)t * nbw + j, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+            if (!uniform(__syncthreads_and(ok))) return;
+            const double v = block_sum<K, NW>(s, sh_err, threadIdx.x);
+            if (threadIdx.x < (unsigned)K) sh_tot[threadIdx.x] = v;
+            __syncthreads();
+            const int keep = uniform(stop_after(sh_tot, kk, n, a));
+            if (a.err_log && threadIdx.x < (unsigned)kk) a.err_log[n + threadIdx.x] = sh_tot[threadIdx.x];
+            if (threadIdx.x == 0)
+                __hip_atomic_store(&ctl->decision[c & 1].v,
                                    (a.seq << 24) | ((unsigned long long)(c + 1) << 4) |
                                        (unsigned long long)keep,
                                    __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            }
             n += keep ? keep : kk;
-            cur ^= 1;
-            parity ^= 1;
             c++;
             if (keep) break;
+            __syncthreads();   // sh_tot is rewritten next chunk
         }
         if (threadIdx.x == 0) {
-            ctl->cur[a.level] = cur;
+            ctl->cur[a.level] = cur0 ^ (c & 1);
             ctl->n = n;
             ctl->stop = 1;
             *a.iters_slot = n;
@@ -941,82 +1172,51 @@ __global__ OF_ITER_BOUNDS(NW) void k_tvl1_persist_nbr(IterArgs a, unsigned tiles
         return;
     }
 
-    int kk_prev = 0;
-    int keep_prev = 0;
+    NbrSync sync{a, FirstBound{a.resident_ticks, a.force_not_resident}, &sh_word, tiles_x, ntiles / tiles_x,
+                 0, 0, -1, 0, 0, false, false};
+    double acc[K];
+    // chunk after chunk; the last pass re-runs part of the chunk that stopped
     while (true) {
-        int kk = a.max_iter - n;
-        if (kk > K) kk = K;
-        if (kk <= 0) {   // past the last chunk: its decision says whether to re-run part of it
-            if (c > 0) keep_prev = wait_decision(a, c - 1, parity ^ 1, fb, &sh_keep);
-            break;
+        if (!sync.stop_keep && sync.c >= nchunks) {
+            if (nchunks == 0) return;
+            sync.last(nchunks);
         }
-        double acc[K];
+        if (sync.failed) return;
+        if (sync.stop_keep) {
+            // the warping stopped after stop_keep iterations of chunk
+            // stop_chunk: if that is short of the chunk, re-run them from its
+            // input into its output
+            if (sync.rerun || sync.stop_keep >= min(K, a.max_iter - sync.stop_chunk * K)) return;
+            sync.rerun = true;
+            sync.c = sync.stop_chunk;
+        }
+        const int c = sync.c, cur = cur0 ^ (c & 1);
+        const int kk = sync.rerun ? sync.stop_keep : min(K, a.max_iter - c * K);
 #pragma unroll
         for (int t = 0; t < K; t++) acc[t] = 0.0;
-        bool decided = c == 0;
-        bool failed = false;
-        // decision c-1 before the chunk's first store: false discards
-        auto check = [&]() -> bool {
-            if (decided) return true;
-            decided = true;
-            keep_prev = wait_decision(a, c - 1, parity ^ 1, fb, &sh_keep);
-            fb = FirstBound{0ull, 0};
-            if (keep_prev < 0) failed = true;
-            return keep_prev == 0;
-        };
         for (unsigned tile = blockIdx.x; tile < ntiles; tile += nbw) {
+            sync.tile = tile;
             const int bx = (int)(tile % tiles_x), by = (int)(tile / tiles_x);
-            if (c > 0) {
-                if (!wait_neighbours(a, tiles_x, tiles_y, bx, by, c, fb)) return;
-                fb = FirstBound{0ull, 0};
-            }
-            if constexpr (SQ) tile_iterate_sq<K, true>(a, bx, by, cur, kk, acc, sh_sq, check);
-            else tile_iterate<K, R, true, NW>(a, bx, by, cur, kk, acc, sh, check);
-            if (failed) return;
-            if (keep_prev != 0) break;
+            if constexpr (SQ) tile_iterate_sq<K, true>(a, bx, by, cur, kk, acc, sh_sq, sync);
+            else tile_iterate<K, R, true, NW>(a, bx, by, cur, kk, acc, sh, sync);
+            if (sync.rerun) continue;
+            if (sync.failed || sync.stop_keep) break;
             // after the workgroup's last tile of the chunk, its error partials
-            // go out with the tile's stores, so one wait for completion
-            // covers both
-            const bool last = tile + nbw >= ntiles;
-            if (last) {
+            // go out with the tile's stores; the flag once both have completed
+            if (tile + nbw >= ntiles) {
                 const double part = block_sum<K, NW>(acc, sh_err, threadIdx.x);
-                double* pp = a.partials + (size_t)parity * K * nbw;
                 if (threadIdx.x < (unsigned)kk)
-                    __hip_atomic_store(pp + (size_t)threadIdx.x * nbw + blockIdx.x, part,
+                    __hip_atomic_store(a.partials + ((size_t)(c & 1) * K + threadIdx.x) * nbw + blockIdx.x, part,
                                        __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            // publish the tile's chunk (and the partials) once the stores
-            // have completed
             __builtin_amdgcn_s_waitcnt(0);
             __atomic_signal_fence(__ATOMIC_SEQ_CST);
             __syncthreads();
-            if (threadIdx.x == 0) {
-                __hip_atomic_store(a.tile_flags + tile, (a.seq << 20) | (unsigned)(c + 1),
-                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (last)
-                    __hip_atomic_fetch_add(&ctl->chunk_count[parity].v, 1u, __ATOMIC_RELAXED,
-                                           __HIP_MEMORY_SCOPE_AGENT);
-            }
+            if (threadIdx.x == 0)
+                __hip_atomic_store(a.tile_flags + tile, (a.seq << 20) | (unsigned)(c + 1), __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
         }
-        if (keep_prev != 0) break;
-        kk_prev = kk;
-        n += kk;
-        cur ^= 1;
-        parity ^= 1;
-        c++;
-    }
-    if (keep_prev < 0) return;
-    // the warping stopped after keep_prev iterations of chunk c-1: re-run
-    // them from its input (buffer cur^1) into its output (buffer cur)
-    if (keep_prev > 0 && keep_prev < kk_prev) {
-        double acc[K];
-#pragma unroll
-        for (int t = 0; t < K; t++) acc[t] = 0.0;
-        for (unsigned tile = blockIdx.x; tile < ntiles; tile += nbw) {
-            const int bx = (int)(tile % tiles_x), by = (int)(tile / tiles_x);
-            if constexpr (SQ) tile_iterate_sq<K, true>(a, bx, by, cur ^ 1, keep_prev, acc, sh_sq);
-            else tile_iterate<K, R, true, NW>(a, bx, by, cur ^ 1, keep_prev, acc, sh);
-        }
+        sync.c++;
     }
 }
 
@@ -1060,16 +1260,17 @@ __device__ __forceinline__ void ls_tile(const LsPhase& ph, const LsPair* P, unsi
     // `cur` at run time and live in scratch memory
     const IterArgs& a = P->a;
     TvCtl* ctl = a.ctl;
-    const int cur = ctl->cur[a.level];
-    const int redo = ctl->redo;
-    const int n0 = ctl->n;
+    const int cur = uniform(ctl->cur[a.level]);
+    const int redo = uniform(ctl->redo);
+    const int n0 = uniform(ctl->n);
     int kk = redo ? redo : a.max_iter - n0;
     if (kk > K) kk = K;
     const unsigned nblocks = P->ntiles;
+    NoSync no_sync;
     double acc[K];
 #pragma unroll
     for (int t = 0; t < K; t++) acc[t] = 0.0;
-    if (kk > 0) tile_iterate<K, R, false, NW>(a, (int)(bid % P->gx), (int)(bid / P->gx), cur, kk, acc, sh);
+    if (kk > 0) tile_iterate<K, R, false, NW>(a, (int)(bid % P->gx), (int)(bid / P->gx), cur, kk, acc, sh, no_sync);
     const double part = block_sum<K, NW>(acc, sh_err, threadIdx.x);
     if ((int)threadIdx.x < kk)
         __hip_atomic_store(a.partials + (size_t)threadIdx.x * nblocks + bid, part, __ATOMIC_RELAXED,
@@ -1115,7 +1316,7 @@ __device__ __forceinline__ void ls_tile(const LsPhase& ph, const LsPair* P, unsi
 }
 
 template <int K, int R, int NW>
-__global__ OF_ITER_BOUNDS(NW) void k_ls_iter(LsPhase ph, const LsPair* __restrict__ pairs,
+__global__ OF_ITER_BOUNDS(NW, K) void k_ls_iter(LsPhase ph, const LsPair* __restrict__ pairs,
                                              LsCtl* mc, unsigned long long* host_status,
                                              unsigned epoch)
 {

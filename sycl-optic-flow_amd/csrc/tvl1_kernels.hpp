@@ -41,10 +41,8 @@ struct TvCtl {
     alignas(256) unsigned bar_gen;
     BarWord grp_count[kBarGroups];   // two-level barrier: per-group arrivals
     BarWord grp_gen[kBarGroups];     // and per-group release epochs
-    // neighbour-synchronised warping kernel, by chunk parity: workgroups
-    // whose error partials of the chunk are published, and the stopping
+    // neighbour-synchronised warping kernel, by chunk parity: the stopping
     // decision of the chunk, (seq << 24) | ((chunk + 1) << 4) | keep
-    BarWord chunk_count[2];
     SeqWord decision[2];
     alignas(256) int error;         // kBarTimeout or kBarNotResident, else 0
 };

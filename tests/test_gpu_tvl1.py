@@ -158,6 +158,46 @@ def test_iterations_bitexact(K, R, h, w):
     np.testing.assert_allclose(gerr, np.array(errs), rtol=1e-12, atol=0)
 
 
+@pytest.mark.parametrize("K,R", [(2, 8), (4, 0)])
+@pytest.mark.parametrize("kind", ["midpoints", "steep", "tiny", "mixed"])
+def test_dual_update_special_gradients_bitexact(K, R, kind):
+    """The dual update's short root and quotients against the full sequences'
+    cases: gradients whose length is exactly halfway between two floats (and
+    an ulp to either side), lengths that make g = 1 + taut*|grad u| an even
+    integer or large, zero and subnormal gradients, and subnormal next to
+    ordinary components.  Flat data (rho = 0, p = 0) leaves u as it is, so the
+    pixel at (2i, 2j) sees its own pair (fx, fy)."""
+    rng = np.random.default_rng(11)
+    h, w = 96, 130
+    n = (h // 2) * (w // 2)
+    if kind == "midpoints":
+        m, v = rng.integers(2900, 4097, 40 * n), rng.integers(1, 2900, 40 * n)
+        A, B, M = m * m - v * v, 2 * m * v, m * m + v * v
+        ok = (A > 0) & (A < 2 ** 24) & (B < 2 ** 24) & (M >= 2 ** 24) & (M < 2 ** 25) & (M % 2 == 1)
+        A, B = A[ok][:n], B[ok][:n]
+        k = rng.integers(-29, -22, n)
+        fx, fy = (A * 2.0 ** k).astype(np.float32), (B * 2.0 ** k).astype(np.float32)
+        fx[::3] = np.nextafter(fx[::3], np.float32(0))
+        fx[1::3] = np.nextafter(fx[1::3], np.float32(9))
+    elif kind == "steep":
+        fx = (rng.choice([3.0, 6.0, 7.2, 10.8, 1e3, 1e20, 1e38], n) * rng.choice([-1, 1], n)).astype(np.float32)
+        fy = (rng.choice([0.0, 4.0, 1e-3, 1e18], n)).astype(np.float32)
+    else:
+        tiny = (rng.integers(-40, 41, n) * rng.choice([1e-45, 1e-41, 1e-38, 1e-30, 1e-20], n))
+        fx = tiny.astype(np.float32)
+        fy = (rng.permutation(tiny) if kind == "tiny" else
+              rng.choice([6.0, 3.6, 0.5, 6.2], n)).astype(np.float32)
+    u1 = np.zeros((h, w), np.float32)
+    u1[0::2, 1::2] = fx.reshape(h // 2, w // 2)
+    u1[1::2, 0::2] = fy.reshape(h // 2, w // 2)
+    u2 = np.ascontiguousarray(u1[::-1])
+    zero = np.zeros((h, w), np.float32)
+    got, _ = D.tvl1_iterations(zero, zero, zero, u1, u2, zero, zero, zero, zero, 1, K, R)
+    want, _ = O.tvl1_iteration(zero, zero, zero, u1, u2, zero, zero, zero, zero)
+    for g, o in zip(got, want):
+        assert np.array_equal(g.view(np.uint32), o.view(np.uint32))
+
+
 def _solve_both(q0, q1, **kw):
     h, w = q0.shape
     with TV_L1(w, h, **kw) as tv:
