@@ -197,6 +197,13 @@ int run_warping(of_tvl1* h, int s, int w, hipStream_t st)
 
     if (persistent && persist_host_paced()) {
         persistent = 0;   // the process gave up persistent launches
+        // (4, 0) with neighbour flags picks its tiles by size (launch_persist);
+        // 16 x 16 ones host-paced are the slower choice from about 20 000
+        // pixels on (1920x1080 pyramid, ms: 120x68 0.64 against 0.78 of (4, 4);
+        // 240x135 0.95 / 0.79; 480x270 2.10 / 1.00; 960x540 5.18 / 1.46)
+        if (K == 4 && R == 0 && h->scale_P[s] == kPersistNeighbour &&
+            (long long)h->nx[s] * h->ny[s] >= 20000)
+            h->scale_R[s] = R = 4;
         h->scale_P[s] = 0;
     }
     if (persistent) {
@@ -603,7 +610,7 @@ int of_tvl1_create(const of_tvl1_params* params, int width, int height, of_tvl1*
         if (st) { delete h; return st; }
     
         const size_t N0 = (size_t)width * height;
-        size_t maxpart = 1, maxtiles = 1;
+        size_t maxpart = kSqOnePerCu * kSqMaxIters, maxtiles = kSqOnePerCu;
         const int Ks[] = {1, 2, 4, 8}, Rs[] = {0, 2, 4, 8};
         for (int K : Ks)
             for (int R : Rs)

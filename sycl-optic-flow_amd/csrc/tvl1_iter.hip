@@ -409,111 +409,163 @@ __device__ __forceinline__ void tile_iterate(const IterArgs& a, int bx, int by, 
     else tile_iterate_impl<K, R, COH, false, NW>(a, bx, by, cur, kk, acc, sh, sync);
 }
 
-// Square tiles for the small scales: one workgroup of 256 lanes covers a
-// 16 x 16 pixel tile, one pixel per lane, neighbours exchanged through LDS.
-// With K iterations per launch the central (16-2K) x (16-2K) pixels are
+// Square tiles for the small scales: one workgroup of T*T lanes covers a
+// T x T pixel tile, one pixel per lane, neighbours exchanged through LDS.
+// With K iterations per launch the central (T-2K) x (T-2K) pixels are
 // exact.  One pixel per lane and more workgroups hide less latency per
 // lane but keep many more CUs busy than 64-column tiles at scales of a few
-// ten thousand pixels (120x68: 1.2 instead of 3.3 us per iteration).
-constexpr int kSqTile = 16;
+// ten thousand pixels (120x68: 1.2 instead of 3.3 us per iteration).  All
+// neighbours go through LDS: at T = 32, where a wave is two whole rows, lane
+// shifts for the horizontal ones cost more than they saved (641x479, two tiles
+// per CU: 0.48 against 0.44 ms).
+constexpr int kSqTile = 16;   // the tile of launch shapes with rows_per_wave 0
 
 // p exchange in a..d, u exchange in e, f: the two halves of an iteration
 // use different arrays, so each needs one barrier, between its writes and
 // its reads.  A half's next writes come after the other half's barrier,
 // which every thread reaches only after its reads of this half.
+template <int T>
 struct SqShared {
-    float a[kSqTile][kSqTile + 1], b[kSqTile][kSqTile + 1], c[kSqTile][kSqTile + 1],
-        d[kSqTile][kSqTile + 1], e[kSqTile][kSqTile + 1], f[kSqTile][kSqTile + 1];
+    float a[T][T + 1], b[T][T + 1], c[T][T + 1], d[T][T + 1], e[T][T + 1], f[T][T + 1];
 };
 
-// kk (<= K) iterations on square tile (bx, by): reads buffer `cur`, writes
-// the central tile into buffer cur^1, adds each iteration's per-lane error
-// term over the central tile to acc[t].  Same per-pixel expressions as
-// tile_iterate_impl; pixels outside the image never feed pixels inside (the
-// border rules do not read across the border).
-template <int K, bool COH, class Sync>
-__device__ __forceinline__ void tile_iterate_sq(const IterArgs& a, int bx, int by, int cur, int kk,
-                                                double (&acc)[K], SqShared& sh, Sync& sync)
+// One pixel of a square tile: its state, the warping's constants, and where
+// it lies.
+struct SqPixel {
+    float u1, u2, p11, p12, p21, p22;
+    float gx, gy, rc;
+    bool fc, lc, fr, lr;   // first/last image column and row
+    bool mine;             // its error counts
+};
+
+// kk (<= K) iterations of a tile of T columns (one pixel per lane, row ly =
+// threadIdx.x / T of the workgroup's rows), each adding its error term to
+// acc[t].  Same per-pixel expressions as tile_iterate_impl; pixels outside
+// the image never feed pixels inside (the border rules do not read across
+// the border).
+template <int T, int K>
+__device__ __forceinline__ void sq_iterations(const IterArgs& a, SqPixel& q, int kk, int rows,
+                                              double (&acc)[K], SqShared<T>& sh)
 {
-    constexpr int T = kSqTile, C = T - 2 * K;
     const int lx = threadIdx.x % T, ly = threadIdx.x / T;
-    const int nx = a.nx, ny = a.ny;
-    const int x = bx * C - K + lx, y = by * C - K + ly;
-    const bool in = x >= 0 && x < nx && y >= 0 && y < ny;
-    const bool mine = in && lx >= K && lx < K + C && ly >= K && ly < K + C;
-    const size_t plane = (size_t)a.plane;
-    const size_t idx = (size_t)y * nx + x;
-    const float* uin = cur ? a.u[1] : a.u[0];
-    const float* pin = cur ? a.p[1] : a.p[0];
-    float u1 = 0.0f, u2 = 0.0f, p11 = 0.0f, p12 = 0.0f, p21 = 0.0f, p22 = 0.0f;
-    float gx = 0.0f, gy = 0.0f, rc = 0.0f;
-    if (in) {
-        gx = a.wx[idx];
-        gy = a.wy[idx];
-        rc = a.rhoc[idx];
-    }
-    if (!sync.ready()) return;
-    if (in) {
-        u1 = ld<COH>(uin + idx);
-        u2 = ld<COH>(uin + plane + idx);
-        p11 = ld<COH>(pin + idx);
-        p12 = ld<COH>(pin + plane + idx);
-        p21 = ld<COH>(pin + 2 * plane + idx);
-        p22 = ld<COH>(pin + 3 * plane + idx);
-    }
-    const bool fc = x == 0, lc = x == nx - 1, fr = y == 0, lr = y == ny - 1;
     // neighbour slots, clamped to the tile: the edge lanes read their own
     // slot (their results are outside the exact centre)
     const int xm = lx > 0 ? lx - 1 : lx, xp = lx < T - 1 ? lx + 1 : lx;
-    const int ym = ly > 0 ? ly - 1 : ly, yp = ly < T - 1 ? ly + 1 : ly;
-    const bool xl = x < nx - 1, yl = y < ny - 1;
+    const int ym = ly > 0 ? ly - 1 : ly, yp = ly < rows - 1 ? ly + 1 : ly;
+    // waves off the image border take the body formulas
+    const bool edge = __any(q.fc || q.lc || q.fr || q.lr);
     const float l_t = a.l_t, theta = a.theta, taut = a.taut;
 #pragma unroll
     for (int t = 0; t < K; t++) {
         if (t < kk) {
             // ---- u update: TH, divergence of p, u = v + theta*div p ----
-            sh.a[ly][lx] = p11;
-            sh.b[ly][lx] = p21;
-            sh.c[ly][lx] = p12;
-            sh.d[ly][lx] = p22;
+            sh.a[ly][lx] = q.p11;
+            sh.b[ly][lx] = q.p21;
+            sh.c[ly][lx] = q.p12;
+            sh.d[ly][lx] = q.p22;
             __syncthreads();
             const float p11l = sh.a[ly][xm], p21l = sh.b[ly][xm];
             const float p12u = sh.c[ym][lx], p22u = sh.d[ym][lx];
-            const float div1 = div_rule(p11, p11l, p12, p12u, fr, lr, fc, lc);
-            const float div2 = div_rule(p21, p21l, p22, p22u, fr, lr, fc, lc);
+            float div1 = (q.p11 - p11l) + (q.p12 - p12u);
+            float div2 = (q.p21 - p21l) + (q.p22 - p22u);
+            if (edge) {
+                div1 = div_rule(q.p11, p11l, q.p12, p12u, q.fr, q.lr, q.fc, q.lc);
+                div2 = div_rule(q.p21, p21l, q.p22, p22u, q.fr, q.lr, q.fc, q.lc);
+            }
             float v1, v2;
-            th_step(rc, gx, gy, u1, u2, l_t, v1, v2);
+            th_step(q.rc, q.gx, q.gy, q.u1, q.u2, l_t, v1, v2);
             const float nu1 = v1 + theta * div1;
             const float nu2 = v2 + theta * div2;
-            const float e1 = nu1 - u1, e2 = nu2 - u2;
+            const float e1 = nu1 - q.u1, e2 = nu2 - q.u2;
             const float e = e1 * e1 + e2 * e2;
-            acc[t] += (double)(mine ? e : 0.0f);
-            u1 = nu1;
-            u2 = nu2;
+            acc[t] += (double)(q.mine ? e : 0.0f);
+            q.u1 = nu1;
+            q.u2 = nu2;
             // ---- p update: forward gradient of u, g, p = (p + taut*grad)/g ----
-            sh.e[ly][lx] = u1;
-            sh.f[ly][lx] = u2;
+            sh.e[ly][lx] = q.u1;
+            sh.f[ly][lx] = q.u2;
             __syncthreads();
             const float u1r = sh.e[ly][xp], u2r = sh.f[ly][xp];
             const float u1d = sh.e[yp][lx], u2d = sh.f[yp][lx];
-            const float fx1 = xl ? u1r - u1 : 0.0f;
-            const float fy1 = yl ? u1d - u1 : 0.0f;
-            const float fx2 = xl ? u2r - u2 : 0.0f;
-            const float fy2 = yl ? u2d - u2 : 0.0f;
-            dual_step(fx1, fy1, fx2, fy2, taut, p11, p12, p21, p22);
+            float fx1 = u1r - q.u1, fy1 = u1d - q.u1, fx2 = u2r - q.u2, fy2 = u2d - q.u2;
+            if (edge) {
+                fx1 = q.lc ? 0.0f : fx1;
+                fy1 = q.lr ? 0.0f : fy1;
+                fx2 = q.lc ? 0.0f : fx2;
+                fy2 = q.lr ? 0.0f : fy2;
+            }
+            dual_step(fx1, fy1, fx2, fy2, taut, q.p11, q.p12, q.p21, q.p22);
         }
     }
-    if (!sync.store()) return;
-    if (mine) {
-        float* uout = cur ? a.u[0] : a.u[1];
-        float* pout = cur ? a.p[0] : a.p[1];
-        st<COH>(uout + idx, u1);
-        st<COH>(uout + plane + idx, u2);
-        st<COH>(pout + idx, p11);
-        st<COH>(pout + plane + idx, p12);
-        st<COH>(pout + 2 * plane + idx, p21);
-        st<COH>(pout + 3 * plane + idx, p22);
+}
+
+template <bool COH>
+__device__ __forceinline__ void sq_load_constants(const IterArgs& a, SqPixel& q, bool in, size_t idx)
+{
+    q.gx = q.gy = q.rc = 0.0f;
+    if (in) {
+        q.gx = a.wx[idx];
+        q.gy = a.wy[idx];
+        q.rc = a.rhoc[idx];
     }
+}
+
+template <bool COH>
+__device__ __forceinline__ void sq_load_state(const IterArgs& a, SqPixel& q, bool in, size_t idx, int cur)
+{
+    const size_t plane = (size_t)a.plane;
+    const float* uin = cur ? a.u[1] : a.u[0];
+    const float* pin = cur ? a.p[1] : a.p[0];
+    q.u1 = q.u2 = q.p11 = q.p12 = q.p21 = q.p22 = 0.0f;
+    if (in) {
+        q.u1 = ld<COH>(uin + idx);
+        q.u2 = ld<COH>(uin + plane + idx);
+        q.p11 = ld<COH>(pin + idx);
+        q.p12 = ld<COH>(pin + plane + idx);
+        q.p21 = ld<COH>(pin + 2 * plane + idx);
+        q.p22 = ld<COH>(pin + 3 * plane + idx);
+    }
+}
+
+template <bool COH>
+__device__ __forceinline__ void sq_store_state(const IterArgs& a, const SqPixel& q, size_t idx, int cur)
+{
+    const size_t plane = (size_t)a.plane;
+    float* uout = cur ? a.u[1] : a.u[0];
+    float* pout = cur ? a.p[1] : a.p[0];
+    st<COH>(uout + idx, q.u1);
+    st<COH>(uout + plane + idx, q.u2);
+    st<COH>(pout + idx, q.p11);
+    st<COH>(pout + plane + idx, q.p12);
+    st<COH>(pout + 2 * plane + idx, q.p21);
+    st<COH>(pout + 3 * plane + idx, q.p22);
+}
+
+// kk (<= K) iterations on square tile (bx, by): reads buffer `cur`, writes
+// the central tile into buffer cur^1, adds each iteration's per-lane error
+// term over the central tile to acc[t].
+template <int T, int K, bool COH, class Sync>
+__device__ __forceinline__ void tile_iterate_sq(const IterArgs& a, int bx, int by, int cur, int kk,
+                                                double (&acc)[K], SqShared<T>& sh, Sync& sync)
+{
+    constexpr int C = T - 2 * K;
+    const int lx = threadIdx.x % T, ly = threadIdx.x / T;
+    const int nx = a.nx, ny = a.ny;
+    const int x = bx * C - K + lx, y = by * C - K + ly;
+    const bool in = x >= 0 && x < nx && y >= 0 && y < ny;
+    const size_t idx = (size_t)y * nx + x;
+    SqPixel q;
+    q.fc = x == 0;
+    q.lc = x == nx - 1;
+    q.fr = y == 0;
+    q.lr = y == ny - 1;
+    q.mine = in && lx >= K && lx < K + C && ly >= K && ly < K + C;
+    sq_load_constants<COH>(a, q, in, idx);
+    if (!sync.ready()) return;
+    sq_load_state<COH>(a, q, in, idx, cur);
+    sq_iterations<T, K>(a, q, kk, T, acc, sh);
+    if (!sync.store()) return;
+    if (q.mine) sq_store_state<COH>(a, q, idx, cur ^ 1);
 }
 
 // Workgroup sum of the per-lane partials, fixed order: wave tree, then
@@ -608,7 +660,9 @@ constexpr int kIterWaves = 8;
 // batch of 64 mixed-size pairs took 79.0 ms instead of 75.7 ms (same box).
 constexpr int kLsWaves = 4;
 // __launch_bounds__(threads, minimum waves per SIMD)
-#define OF_ITER_BOUNDS(NW, K) __launch_bounds__(64 * (NW), (NW) == 4 ? kIterBlocksPerCU : (K) == 8 ? 2 : 4)
+// Square tiles of 16 waves with 3 iterations: 8, i.e. two workgroups per CU.
+#define OF_ITER_BOUNDS(NW, K) \
+    __launch_bounds__(64 * (NW), (NW) == 4 ? kIterBlocksPerCU : (NW) == 16 && (K) == 3 ? 8 : (K) == 8 ? 2 : 4)
 
 // ---------------------------------------------------------------------------
 // launch-per-chunk driver
@@ -618,11 +672,11 @@ constexpr int kLsWaves = 4;
 // iteration that meets it falls inside the launch before its last
 // iteration, the launch's output is discarded and the next launch re-runs
 // exactly that many iterations from the same input buffer.
-template <int K, int R, int NW = 4, bool SQ = false>
+template <int K, int R, int NW = 4, int T = 0>
 __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_iter(IterArgs a)
 {
     __shared__ TileSharedN<NW> sh;
-    __shared__ SqShared sh_sq;
+    __shared__ SqShared<T ? T : 1> sh_sq;
     __shared__ double sh_err[NW][K];
     __shared__ double sh_tot[K];
     __shared__ double sh4[K * NW];
@@ -641,7 +695,7 @@ __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_iter(IterArgs a)
     double acc[K];
 #pragma unroll
     for (int t = 0; t < K; t++) acc[t] = 0.0;
-    if constexpr (SQ) tile_iterate_sq<K, false>(a, blockIdx.x, blockIdx.y, cur, kk, acc, sh_sq, no_sync);
+    if constexpr (T != 0) tile_iterate_sq<T, K, false>(a, blockIdx.x, blockIdx.y, cur, kk, acc, sh_sq, no_sync);
     else tile_iterate<K, R, false, NW>(a, blockIdx.x, blockIdx.y, cur, kk, acc, sh, no_sync);
 
     const unsigned nblocks = gridDim.x * gridDim.y;
@@ -861,11 +915,11 @@ __device__ __forceinline__ bool grid_barrier2(TvCtl* ctl, unsigned nb, BarEpoch&
 // with device-scope atomic accesses so that halos written by workgroups on
 // other XCDs are seen without cache maintenance.  Partials are
 // double-buffered by chunk parity.
-template <int K, int R, int NW = 4, bool SQ = false>
+template <int K, int R, int NW = 4, int T = 0>
 __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist(IterArgs a, unsigned tiles_x, unsigned ntiles)
 {
     __shared__ TileSharedN<NW> sh;
-    __shared__ SqShared sh_sq;
+    __shared__ SqShared<T ? T : 1> sh_sq;
     __shared__ double sh_err[NW][K];
     __shared__ double sh_tot[K];
     __shared__ double sh4[K * NW];
@@ -896,8 +950,8 @@ __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist(IterArgs a, unsigned tiles_
 #pragma unroll
         for (int t = 0; t < K; t++) acc[t] = 0.0;
         for (unsigned tile = blockIdx.x; tile < ntiles; tile += nb)
-            if constexpr (SQ)
-                tile_iterate_sq<K, true>(a, (int)(tile % tiles_x), (int)(tile / tiles_x), cur, kk, acc, sh_sq, no_sync);
+            if constexpr (T != 0)
+                tile_iterate_sq<T, K, true>(a, (int)(tile % tiles_x), (int)(tile / tiles_x), cur, kk, acc, sh_sq, no_sync);
             else
                 tile_iterate<K, R, true, NW>(a, (int)(tile % tiles_x), (int)(tile / tiles_x), cur, kk, acc, sh, no_sync);
         if (redo) {   // the re-run chunk is final: no decision needed
@@ -911,7 +965,7 @@ __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist(IterArgs a, unsigned tiles_
             __hip_atomic_store(pp + (size_t)threadIdx.x * nb + blockIdx.x, part, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_AGENT);
         // square tiles run one workgroup per small tile: many workgroups
-        if (!(SQ ? grid_barrier2(ctl, nb, ep, &sh_ok, fb) : grid_barrier(ctl, nb, gen, &sh_ok, fb)))
+        if (!(T != 0 ? grid_barrier2(ctl, nb, ep, &sh_ok, fb) : grid_barrier(ctl, nb, gen, &sh_ok, fb)))
             return;
         fb = FirstBound{0ull, 0};
         grid_sums<K, NW>(pp, nb, kk, sh4, sh_tot);
@@ -1019,7 +1073,8 @@ struct NbrSync {
         int r = -1;
         if (threadIdx.x < 64) {
             const unsigned long long* w = &a.ctl->decision[q & 1].v;
-            if (wave_wait(a, threadIdx.x == 0 ? w : nullptr, (a.seq << 24) | ((unsigned long long)(q + 1) << 4), fb))
+            const unsigned long long want = (a.seq << 24) | ((unsigned long long)(q + 1) << 4);
+            if (wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, fb))
                 r = (int)(__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFull);
         }
         return share(r);
@@ -1107,13 +1162,13 @@ struct NbrSync {
 // -> 0.32.  Dealing tiles to workgroups in rotation, so that all get the same
 // number, was 5% slower at 1920x1080: two workgroups with 2 and 3 tiles
 // already share a CU evenly.
-template <int K, int R, int NW = 4, bool SQ = false>
+template <int K, int R, int NW = 4, int T = 0>
 __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist_nbr(IterArgs a, unsigned tiles_x, unsigned ntiles)
 {
-    static_assert(SQ ? (kSqTile - 2 * K >= K) : (NW * R - 2 * K >= K && 64 - 2 * K >= K),
+    static_assert(T ? (T - 2 * K >= K) : (NW * R - 2 * K >= K && 64 - 2 * K >= K),
                   "the halo of a tile must lie within its neighbours");
     __shared__ TileSharedN<NW> sh;
-    __shared__ SqShared sh_sq;
+    __shared__ SqShared<T ? T : 1> sh_sq;
     __shared__ double sh_err[NW][K];
     __shared__ double sh_tot[K];
     __shared__ int sh_word;
@@ -1197,7 +1252,7 @@ __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist_nbr(IterArgs a, unsigned ti
         for (unsigned tile = blockIdx.x; tile < ntiles; tile += nbw) {
             sync.tile = tile;
             const int bx = (int)(tile % tiles_x), by = (int)(tile / tiles_x);
-            if constexpr (SQ) tile_iterate_sq<K, true>(a, bx, by, cur, kk, acc, sh_sq, sync);
+            if constexpr (T != 0) tile_iterate_sq<T, K, true>(a, bx, by, cur, kk, acc, sh_sq, sync);
             else tile_iterate<K, R, true, NW>(a, bx, by, cur, kk, acc, sh, sync);
             if (sync.rerun) continue;
             if (sync.failed || sync.stop_keep) break;
@@ -1217,6 +1272,86 @@ __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist_nbr(IterArgs a, unsigned ti
                                    __HIP_MEMORY_SCOPE_AGENT);
         }
         sync.c++;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// one-workgroup driver
+// ---------------------------------------------------------------------------
+
+// A whole warping of a scale of at most 32 x 32 pixels in one workgroup of 32
+// lanes per image row: the state stays in registers, no other workgroup takes
+// part.  Chunks of K iterations; a stop inside a chunk re-runs that many from
+// the state at its start.  Bound by the dependent chain of an iteration and its
+// two exchanges (0.7 us at 15 rows); the neighbour kernel's chunks add their
+// round trip through memory (20x15: 1.5 us per iteration).
+constexpr int kSingleCols = 32;
+template <int K>
+__global__ __launch_bounds__(1024) void k_tvl1_single(IterArgs a)
+{
+    constexpr int T = kSingleCols;
+    __shared__ SqShared<T> sh;
+    __shared__ double sh_err[16][K];
+    const int lx = threadIdx.x % T, ly = threadIdx.x / T;
+    const int nx = a.nx, ny = a.ny;
+    const int rows = blockDim.x / T, nw = blockDim.x / 64;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool in = lx < nx && ly < ny;
+    const size_t idx = (size_t)ly * nx + lx;
+    const int cur = uniform(a.ctl->cur[a.level]);
+    SqPixel q;
+    q.fc = lx == 0;
+    q.lc = lx == nx - 1;
+    q.fr = ly == 0;
+    q.lr = ly == ny - 1;
+    q.mine = in;
+    sq_load_constants<false>(a, q, in, idx);
+    sq_load_state<false>(a, q, in, idx, cur);
+    int n = 0;
+    while (n < a.max_iter) {
+        const int kk = min(K, a.max_iter - n);
+        const SqPixel start = q;
+        double acc[K];
+#pragma unroll
+        for (int t = 0; t < K; t++) acc[t] = 0.0;
+        sq_iterations<T, K>(a, q, kk, rows, acc, sh);
+#pragma unroll
+        for (int t = 0; t < K; t++) {
+            const double v = wave_sum_f64(acc[t]);
+            if (lane == 63) sh_err[wave][t] = v;
+        }
+        __syncthreads();
+        double tot[K];
+#pragma unroll
+        for (int t = 0; t < K; t++) tot[t] = 0.0;
+        for (int w = 0; w < nw; w++) {
+#pragma unroll
+            for (int t = 0; t < K; t++) tot[t] += sh_err[w][t];
+        }
+        if (a.err_log && threadIdx.x == 0) {
+#pragma unroll
+            for (int t = 0; t < K; t++)
+                if (t < kk) a.err_log[n + t] = tot[t];
+        }
+        int keep = 0;
+#pragma unroll
+        for (int t = K - 1; t >= 0; t--)
+            if (t < kk && !(tot[t] / (double)a.plane > a.eps2)) keep = t + 1;
+        keep = uniform(keep);
+        if (keep && keep < kk) {
+            q = start;
+            sq_iterations<T, K>(a, q, keep, rows, acc, sh);
+        }
+        n += keep ? keep : kk;
+        if (keep) break;
+        __syncthreads();   // sh_err is rewritten next chunk
+    }
+    if (n > 0 && in) sq_store_state<false>(a, q, idx, cur ^ 1);
+    if (threadIdx.x == 0) {
+        if (n > 0) a.ctl->cur[a.level] = cur ^ 1;
+        a.ctl->n = n;
+        a.ctl->stop = 1;
+        *a.iters_slot = n;
     }
 }
 
@@ -1420,7 +1555,7 @@ static hipError_t launch_kr(const IterArgs& a, hipStream_t s)
     unsigned gx, gy;
     iter_grid(K, R, a.nx, a.ny, &gx, &gy);
     if constexpr (R == 0)
-        hipLaunchKernelGGL((k_tvl1_iter<K, 0, 4, true>), dim3(gx, gy), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_tvl1_iter<K, 0, 4, kSqTile>), dim3(gx, gy), dim3(256), 0, s, a);
     else
         hipLaunchKernelGGL((k_tvl1_iter<K, R * 4 / kIterWaves, kIterWaves>), dim3(gx, gy),
                            dim3(64 * kIterWaves), 0, s, a);
@@ -1450,10 +1585,10 @@ template <int K, int R, bool NBR>
 static const void* persist_kernel()
 {
     if constexpr (NBR) {
-        if constexpr (R == 0) return (const void*)k_tvl1_persist_nbr<K, 0, 4, true>;
+        if constexpr (R == 0) return (const void*)k_tvl1_persist_nbr<K, 0, 4, kSqTile>;
         else return (const void*)k_tvl1_persist_nbr<K, R * 4 / kIterWaves, kIterWaves>;
     } else {
-        if constexpr (R == 0) return (const void*)k_tvl1_persist<K, 0, 4, true>;
+        if constexpr (R == 0) return (const void*)k_tvl1_persist<K, 0, 4, kSqTile>;
         else return (const void*)k_tvl1_persist<K, R * 4 / kIterWaves, kIterWaves>;
     }
 }
@@ -1507,20 +1642,20 @@ static std::atomic<unsigned long long> g_warp_seq{0};
 
 unsigned long long next_warp_seq() { return g_warp_seq.fetch_add(1) + 1; }
 
-// NBR: the neighbour-synchronised kernel, whose grid is the tile
-// workgroups plus one referee workgroup.
-template <int K, int R, bool NBR>
-static int launch_persist_kr(const IterArgs& a, int nblocks, hipStream_t s)
+// Launches the persistent kernel `fn` of `threads` threads over gx x gy tiles.
+// nbr: the neighbour-synchronised kernel with K iterations per chunk, whose
+// grid is the tile workgroups plus one referee workgroup.  `resident` caches
+// the kernel's co-resident workgroups on the device (-1: not known yet).
+static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, unsigned gx, unsigned gy,
+                               const IterArgs& a, int nblocks, int* resident, hipStream_t s)
 {
-    static int resident = -1;   // co-resident workgroups of this kernel on the device
     static unsigned long long bound_ticks = 0;
-    if (resident < 0) {
+    if (*resident < 0) {
         int dev = 0, per_cu = 0, cus = 0, clock_khz = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
             hipDeviceGetAttribute(&clock_khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, persist_kernel<K, R, NBR>(),
-                                                         persist_threads<R>(), 0) != hipSuccess) {
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, 0) != hipSuccess) {
             (void)hipGetLastError();
             return OF_ERR_HIP;
         }
@@ -1529,16 +1664,18 @@ static int launch_persist_kr(const IterArgs& a, int nblocks, hipStream_t s)
         // at most 4 workgroups per CU: 1024 arrivals on one counter and
         // pollers of one word per barrier are already plenty (the compiled
         // bound allows 2 of 8 waves)
-        resident = std::min(per_cu, 4) * cus;
+        // a workgroup's waves are dealt to the 4 SIMDs from the first on: one of
+        // 9 waves puts 3 on one SIMD, which the occupancy query does not see
+        const int waves = threads / 64, per_simd = (waves + 3) / 4;
+        per_cu = std::min(per_cu, per_cu * waves / 4 / per_simd);
+        *resident = std::min(per_cu, 4) * cus;
     }
-    if (resident <= (NBR ? 1 : 0)) return OF_ERR_UNSUPPORTED;
-    unsigned gx, gy;
-    iter_grid(K, R, a.nx, a.ny, &gx, &gy);
+    if (*resident <= (nbr ? 1 : 0)) return OF_ERR_UNSUPPORTED;
     const unsigned ntiles = gx * gy;
     unsigned nb = nblocks > 0 ? (unsigned)nblocks : ntiles;
     if (nb > ntiles) nb = ntiles;
-    if (nb > (unsigned)resident - (NBR ? 1u : 0u)) nb = (unsigned)resident - (NBR ? 1u : 0u);
-    if (NBR) {
+    if (nb > (unsigned)*resident - (nbr ? 1u : 0u)) nb = (unsigned)*resident - (nbr ? 1u : 0u);
+    if (nbr) {
         if (!a.tile_flags || a.seq == 0 || a.seq >= kNbrMaxSeq) return OF_ERR_ARG;
         if ((long long)a.max_iter / K + 1 >= kNbrMaxChunks) return OF_ERR_UNSUPPORTED;
         nb += 1;   // the referee
@@ -1548,8 +1685,7 @@ static int launch_persist_kr(const IterArgs& a, int nblocks, hipStream_t s)
     args.force_not_resident = g_force_not_resident.load(std::memory_order_relaxed);
     unsigned tx = gx, nt = ntiles;
     void* kargs[] = {(void*)&args, (void*)&tx, (void*)&nt};
-    const hipError_t e =
-        hipLaunchKernel(persist_kernel<K, R, NBR>(), dim3(nb), dim3(persist_threads<R>()), kargs, 0, s);
+    const hipError_t e = hipLaunchKernel(fn, dim3(nb), dim3(threads), kargs, 0, s);
     if (e != hipSuccess) {
         record_hip_error(e, "k_tvl1_persist launch", __FILE__, __LINE__);
         return OF_ERR_HIP;
@@ -1557,14 +1693,84 @@ static int launch_persist_kr(const IterArgs& a, int nblocks, hipStream_t s)
     return OF_OK;
 }
 
+template <int K, int R, bool NBR>
+static int launch_persist_kr(const IterArgs& a, int nblocks, hipStream_t s)
+{
+    static int resident = -1;
+    unsigned gx, gy;
+    iter_grid(K, R, a.nx, a.ny, &gx, &gy);
+    return launch_persist_grid(persist_kernel<K, R, NBR>(), persist_threads<R>(), K, NBR, gx, gy, a, nblocks,
+                               &resident, s);
+}
+
+// Square tiles of T x T pixels with K iterations per chunk.
+template <int T, int K>
+static int launch_persist_sq(const IterArgs& a, int nblocks, hipStream_t s)
+{
+    static int resident = -1;
+    static_assert(T * T % 64 == 0 && T * T <= 1024, "whole waves");
+    static_assert(K <= kSqMaxIters, "room for the partials");
+    const unsigned gx = cdiv((size_t)a.nx, (size_t)(T - 2 * K)), gy = cdiv((size_t)a.ny, (size_t)(T - 2 * K));
+    return launch_persist_grid((const void*)k_tvl1_persist_nbr<K, 0, T * T / 64, T>, T * T, K, true, gx, gy, a,
+                               nblocks, &resident, s);
+}
+
+// The shape (4, 0) with neighbour flags: square tiles of a size chosen by the
+// scale's.  A chunk costs its iterations (one tile per CU: 0.5 us each at 16 x
+// 16, 0.74 at 24 x 24, 0.9 at 32 x 32, the chain of an iteration and its two
+// barriers) plus 4.5 us of exchange with the neighbours, so the line lies where
+// the next smaller tile no longer has a CU of its own: within that, more
+// iterations per chunk and smaller tiles win.  Whole scales, five warpings with
+// their set-up, MI355X:
+//    scale      16x16 K4   16x16 K5   24x24 K5   32x32 K5   32x32 K4   32x32 K3
+//    80x60         0.31       0.29       0.33                             0.53   ms
+//    120x68        0.31       0.30       0.37       0.47       0.47       0.55
+//    161x120       0.36       0.41       0.33       0.40       0.41       0.46
+//    240x135       0.44       0.57       0.37       0.44       0.47       0.55
+//    321x240       0.53       0.58                  0.33       0.33       0.38
+//    512x218       0.55       0.65                  0.32       0.35       0.38
+//    480x270       0.78       1.03                  0.73       0.52       0.61
+//    641x479       0.70       1.10                  0.60       0.58       0.44
+//    1024x436      0.90       1.40                  0.66       0.66       0.52
+// Scales with more 32 x 32 tiles than CUs take three iterations per chunk, whose
+// registers let two tiles share a CU.  A scale that fits one workgroup needs no
+// exchange at all (30x17: 0.15 against 0.20 ms, 20x15: 0.29 against 0.33).
+static bool one_per_cu(const IterArgs& a, int centre)
+{
+    return (long long)cdiv((size_t)a.nx, (size_t)centre) * cdiv((size_t)a.ny, (size_t)centre) <= kSqOnePerCu;
+}
+
+static int launch_persist_square(const IterArgs& a, int nblocks, hipStream_t s)
+{
+    if (a.nx <= kSingleCols && a.ny <= kSingleCols) {
+        const unsigned threads = 64 * cdiv((size_t)a.ny * kSingleCols, 64);
+        hipLaunchKernelGGL(k_tvl1_single<4>, dim3(1), dim3(threads), 0, s, a);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) {
+            record_hip_error(e, "k_tvl1_single launch", __FILE__, __LINE__);
+            return OF_ERR_HIP;
+        }
+        return OF_OK;
+    }
+    if (one_per_cu(a, 6)) return launch_persist_sq<16, 5>(a, nblocks, s);
+    if (one_per_cu(a, 14)) return launch_persist_sq<24, 5>(a, nblocks, s);
+    if (one_per_cu(a, 22)) return launch_persist_sq<32, 5>(a, nblocks, s);
+    // a flag counts the chunks of 4 iterations of any accepted limit, not those of 3
+    if (one_per_cu(a, 24) || (long long)a.max_iter / 3 + 1 >= kNbrMaxChunks)
+        return launch_persist_sq<32, 4>(a, nblocks, s);
+    return launch_persist_sq<32, 3>(a, nblocks, s);
+}
+
 int launch_persist(int K, int R, const IterArgs& a, int nblocks, hipStream_t s, int mode)
 {
     if (mode != kPersistBarrier && mode != kPersistNeighbour) return OF_ERR_ARG;
+    if (K == 4 && R == 0 && mode == kPersistNeighbour) return launch_persist_square(a, nblocks, s);
 #define OF_PCASE(k, r)                                                            \
     if (K == k && R == r)                                                         \
         return mode == kPersistNeighbour ? launch_persist_kr<k, r, true>(a, nblocks, s) \
                                          : launch_persist_kr<k, r, false>(a, nblocks, s);
-    OF_PCASE(1, 0) OF_PCASE(2, 0) OF_PCASE(4, 0)
+    if (K == 4 && R == 0) return launch_persist_kr<4, 0, false>(a, nblocks, s);
+    OF_PCASE(1, 0) OF_PCASE(2, 0)
     OF_PCASE(1, 2) OF_PCASE(2, 2)
     OF_PCASE(1, 4) OF_PCASE(2, 4) OF_PCASE(4, 4)
     OF_PCASE(1, 8) OF_PCASE(2, 8) OF_PCASE(4, 8) OF_PCASE(8, 8)

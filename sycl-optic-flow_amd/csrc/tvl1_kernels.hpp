@@ -100,6 +100,10 @@ unsigned long long next_warp_seq();
 int launch_iter(int K, int R, const IterArgs& a, hipStream_t s);
 bool iter_config_ok(int K, int R);
 void iter_grid(int K, int R, int nx, int ny, unsigned* gx, unsigned* gy);
+// The square tiles of shape (4, 0) with neighbour flags may be smaller than
+// iter_grid's: at most kSqOnePerCu then (a CU each, one left for the referee),
+// with up to kSqMaxIters iterations per chunk.
+constexpr int kSqOnePerCu = 255, kSqMaxIters = 5;
 // Whole warping in one launch of a grid that fits the device at once;
 // `nblocks` = 0 picks the largest such grid not above the tile count.  Its
 // first grid barrier reports kBarNotResident if the grid did not fully start.

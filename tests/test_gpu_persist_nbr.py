@@ -72,6 +72,26 @@ def test_stops_inside_and_at_chunk_ends(K, R, eps, cap):
         assert (it == cap).any() or (it % K != 0).any()
 
 
+# Shape (4, 0): the sizes on either side of each change of tile -- one
+# workgroup up to 32 x 32; 255 tiles with centres of 6, 14, 22 and 24 pixels;
+# beyond, tiles sharing a CU, then several tiles per workgroup; one-tile-high
+# and one-tile-wide scales -- with caps inside and at the end of chunks of 3, 4
+# and 5 iterations.  The arithmetic is the oracle's: no difference.
+@pytest.mark.parametrize("w,h,cap", [(32, 32, 300), (32, 32, 8), (19, 31, 7), (33, 32, 300),
+                                     (31, 33, 11), (102, 90, 15), (103, 90, 14), (238, 210, 300),
+                                     (239, 210, 300), (374, 330, 12), (375, 330, 13), (408, 360, 17),
+                                     (409, 360, 300), (409, 361, 10), (821, 604, 9), (1500, 17, 16),
+                                     (17, 900, 300)])
+def test_square_tiles_by_size_match_oracle(w, h, cap):
+    print("nbr square", w, h, cap, flush=True)
+    q0, q1 = _pair(w, h, 3.0, 41 + w + h)
+    prm = dict(nscales=2 if min(w, h) > 40 else 1, warps=3, max_iterations=cap)
+    u, it = _solve(q0, q1, [(0, 4, 0, NBR)], **prm)
+    uo, ito = _oracle(q0, q1, **prm)
+    assert np.array_equal(it, ito)
+    assert np.array_equal(u, uo)
+
+
 def test_zero_iteration_cap():
     q0, q1 = _pair(160, 120, 3.0, 19)
     u, it = _solve(q0, q1, [(0, 4, 4, NBR)], nscales=3, max_iterations=0)
