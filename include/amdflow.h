@@ -124,8 +124,9 @@ int of_tvl1_get_stats(const of_tvl1 *h, of_tvl1_stats *st);
  * launch on tiles of 64 x (4*rows_per_wave) pixels with a halo of
  * iters_per_launch pixels.  Supported: iters_per_launch in {1,2,4,8},
  * rows_per_wave in {2,4,8}; rows_per_wave 0 selects square 16 x 16 tiles,
- * one pixel per lane (iters_per_launch in {1,2,4}; the built-in choice,
- * host-paced, below 200000 pixels).  `persistent` = 0 runs host-paced launches;
+ * one pixel per lane (iters_per_launch in {1,2,4}; with neighbour flags,
+ * iters_per_launch 4 stands for square tiles of 16, 24 or 32 pixels, chosen by
+ * the scale's size).  `persistent` = 0 runs host-paced launches;
  * 1 runs each warping of those scales as one launch of a co-resident grid,
  * chunks of iters_per_launch iterations separated by grid barriers; 2 runs
  * the same single launch with neighbour flags instead of grid barriers (a
@@ -133,7 +134,8 @@ int of_tvl1_get_stats(const of_tvl1 *h, of_tvl1_stats *st);
  * and one extra workgroup applies the stopping rule while the tiles go on;
  * see of_set_persist_launch_mode); other values return OF_ERR_ARG.  Rules are
  * matched largest min_pixels first; calling with min_pixels < 0 clears all
- * rules (back to the built-in table). */
+ * rules (back to the built-in table: neighbour flags while no other solve of
+ * the process runs persistent warpings on the device, host-paced otherwise). */
 int of_tvl1_set_launch_rule(of_tvl1 *h, long long min_pixels, int iters_per_launch,
                             int rows_per_wave, int persistent);
 
@@ -144,9 +146,12 @@ int of_tvl1_set_launch_rule(of_tvl1 *h, long long min_pixels, int iters_per_laun
  * every workgroup started.  If one did not (another persistent kernel on
  * another stream or process held the CUs, a CU-masked stream), the solve is
  * repeated and the process stays in OF_PERSIST_HOST_PACED: those warpings
- * then run host-paced with the same launch shape, which needs no
+ * then run host-paced with the same launch shape (square tiles by size: with
+ * 16 x 16 ones, or 64 x 16 from 20000 pixels on), which needs no
  * co-residency.  AMDFLOW_HOST_PACED=1 in the environment starts a process in
- * host-paced mode.  Results are the same bits in both modes. */
+ * host-paced mode.  Where only the built-in rules made a warping persistent,
+ * the process keeps its mode and the handle's next solves run host-paced.
+ * Results are the same bits in both modes. */
 enum { OF_PERSIST_PLAIN = 0, OF_PERSIST_HOST_PACED = 1 };
 int of_persist_launch_mode(void);
 int of_set_persist_launch_mode(int mode);

@@ -2,17 +2,19 @@
 //
 // Mirrors TV_L1 of src/tvl1/sequential/tvl1.{hpp,cpp}: the constructor fixes
 // the pyramid, runDualTVL1Multiscale builds it and solves coarse to fine.
-// All work is enqueued on one HIP stream.  The only host involvement inside
-// a solve is pacing the iteration launches of each warping: the device
-// decides when a warping has converged and publishes its progress in a
-// host-mapped word that the host polls.
+// All work is enqueued on one HIP stream.  A warping is one launch that stops
+// by itself, or a row of launches that the host paces: the device decides when
+// the warping has converged and publishes its progress in a host-mapped word
+// that the host polls.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <mutex>
 #include <new>
+#include <shared_mutex>
 #include <vector>
 
 #include "amdflow.h"
@@ -26,14 +28,32 @@ using namespace amdflow;
 
 namespace {
 
-// Built-in launch shapes per scale size (pixels): large scales are bound by
-// memory traffic and use short temporal blocking with host-paced launches;
-// small scales are bound by launch latency and run each warping in one
-// persistent launch.
+// Built-in launch shapes per scale size (pixels), warpings in one launch with
+// neighbour flags: square tiles by size, 64-column tiles of 32 rows from 1.6
+// million pixels on (whole scales, ms: 1280x720 1.01 / 1.08, 1536x864 0.99 / 1.07,
+// 1664x936 1.31 / 1.45, 1760x990 1.38 / 1.34, 1920x1080 2.50 / 2.09).  They save
+// the host's part in every chunk, 9 to 14 us at the small scales where a chunk's
+// work is 2 to 4 (320x240, five scales: 2.92 -> 1.31 ms per solve; 1024x436: 3.27 ->
+// 1.52; 1920x1080: 5.82 -> 3.30).
 const LaunchRule kDefaultRules[] = {
-    {200000, 2, 8, 0},
-    {0, 4, 0, 0},   // square tiles (rows_per_wave 0), host-paced
+    {1600000, 2, 8, kPersistNeighbour},
+    {0, 4, 0, kPersistNeighbour},
 };
+
+// The same where a warping must not wait for other workgroups: another solve
+// has the device's turn (PersistTurn), the process is host-paced, or a launch
+// was not co-resident.
+const LaunchRule kPacedRules[] = {
+    {200000, 2, 8, kHostPaced},
+    {0, 4, 0, kHostPaced},   // square tiles (rows_per_wave 0)
+};
+
+// Largest scale of the built-in persistent rules.  A workgroup's first wait,
+// which bounds the residency check at 2 ms, comes after its tiles of the first
+// chunk: 0.3 ms at this size.  Also the longest warping they take, for the
+// chunk numbers of the flags.
+constexpr long long kPersistMaxPixels = 1ll << 24;
+constexpr int kPersistMaxIters = 1 << 20;
 
 constexpr int kEnergyBlocks = 1024;
 
@@ -56,20 +76,95 @@ int own_stream(of_tvl1* h, hipStream_t* out)
     return OF_OK;
 }
 
-int pick_rule(const of_tvl1* h, long long npx, int* K, int* R, int* persistent)
+// The rule of a scale of npx pixels: the handle's, or null where none reaches.
+const LaunchRule* handle_rule(const of_tvl1* h, long long npx)
 {
     const LaunchRule* best = nullptr;
     for (const LaunchRule& r : h->rules)
         if (npx >= r.min_pixels && (!best || r.min_pixels > best->min_pixels)) best = &r;
-    if (!best)
-        for (const LaunchRule& r : kDefaultRules)
-            if (npx >= r.min_pixels) { best = &r; break; }
-    if (!best) best = &kDefaultRules[sizeof(kDefaultRules) / sizeof(kDefaultRules[0]) - 1];
+    return best;
+}
+
+void pick_rule(const of_tvl1* h, long long npx, int* K, int* R, int* persistent)
+{
+    const LaunchRule* best = handle_rule(h, npx);
+    if (!best) {
+        const bool paced = !h->run_persist || npx > kPersistMaxPixels || h->run_max > kPersistMaxIters;
+        best = paced ? kPacedRules : kDefaultRules;
+        while (npx < best->min_pixels) best++;
+    }
     *K = best->K;
     *R = best->R;
     *persistent = best->persistent;
-    return OF_OK;
 }
+
+// Who may run persistent warpings on a device of this process.  The grids of two
+// such solves at once need not both be resident, and then both are repeated
+// host-paced.  So a solve takes the built-in persistent rules only while no
+// other solve of the process runs persistent warpings on the device.  Otherwise
+// a frame below kTurnPixels runs host-paced beside the other one, which leaves
+// CUs free (3 threads at 320x240, ms per solve of all threads together: host-paced
+// alone 1.07, so 0.87, taking turns 1.25); a larger one waits for its turn (2
+// threads at 640x480: 1.54, 1.58, 1.28; at 1024x436: 1.92, 1.92, 1.38; at
+// 1920x1080: 4.11, 3.96, 2.81).  A solve whose own rules are persistent runs next
+// to others of its kind, as it asks for, and waits for one on built-in rules to
+// end.  No wait is longer than kTurnWait, since the other solve may itself wait
+// for work on its stream; a handle that waited in vain does not wait again for a
+// number of solves.  (Other processes are not seen: the residency check covers
+// them.)
+constexpr int kTurnDevices = 64;
+constexpr long long kTurnPixels = 200000;
+constexpr std::chrono::milliseconds kTurnWait{20};
+
+class PersistTurn {
+public:
+    PersistTurn(of_tvl1* h, int first)
+    {
+        const bool back_off = h->paced_solves > 0;
+        if (back_off) h->paced_solves--;
+        bool own = false, builtin = false;
+        for (int s = 0; s <= first; s++) {
+            const LaunchRule* r = handle_rule(h, (long long)h->nx[s] * h->ny[s]);
+            if (!r) builtin = true;
+            else if (r->persistent) own = true;
+        }
+        int dev = 0;
+        if (persist_host_paced() || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kTurnDevices)
+            return;
+        own_rules_ = own;
+        std::shared_timed_mutex& m = turns()[dev];
+        if (builtin && !back_off) {
+            const bool wait = (long long)h->nx[0] * h->ny[0] >= kTurnPixels;
+            unique_ = std::unique_lock<std::shared_timed_mutex>(m, std::defer_lock);
+            if (wait ? unique_.try_lock_for(kTurnWait) : unique_.try_lock()) return;
+            if (wait) pace(h);
+        }
+        if (own) {
+            shared_ = std::shared_lock<std::shared_timed_mutex>(m, std::defer_lock);
+            if (!(back_off ? shared_.try_lock() : shared_.try_lock_for(kTurnWait))) pace(h);
+        }
+    }
+    // The handle's next solves neither take the built-in persistent rules nor wait.
+    static void pace(of_tvl1* h)
+    {
+        if (h->paced_solves > 0) return;
+        h->paced_solves = h->paced_next;
+        h->paced_next = std::min(2 * h->paced_next, kPacedMost);
+    }
+    bool builtin() const { return unique_.owns_lock(); }   // the built-in persistent rules apply
+    bool own_rules() const { return own_rules_; }          // some scale's own rule is persistent
+
+private:
+    // never destroyed: a solve may run while the process ends
+    static std::shared_timed_mutex* turns()
+    {
+        static std::shared_timed_mutex* const m = new std::shared_timed_mutex[kTurnDevices];
+        return m;
+    }
+    std::unique_lock<std::shared_timed_mutex> unique_;
+    std::shared_lock<std::shared_timed_mutex> shared_;
+    bool own_rules_ = false;
+};
 
 void release(of_tvl1* h)
 {
@@ -413,16 +508,21 @@ int solve_levels_once(of_tvl1* h, const float* init, int first, const int* warps
     return OF_OK;
 }
 
-// solve_levels_once, repeated once with host-paced launches (from then on,
-// for the whole process) if a persistent launch was not co-resident.  The
-// repeat starts from the same pyramids and `init`, which a solve does not
-// write.
+// solve_levels_once, repeated once with host-paced launches if a persistent
+// launch was not co-resident: from then on, for the whole process, where the
+// handle's own rules asked for persistent launches; for a number of solves of
+// the handle, doubled each time, where only the built-in ones did.  The repeat
+// starts from the same pyramids and `init`, which a solve does not write.
 int solve_levels_schedule(of_tvl1* h, const float* init, int first, const int* warps_s,
                           const int* max_s, float* dst, hipStream_t st)
 {
+    const PersistTurn turn(h, first);
+    h->run_persist = turn.builtin();
     const int rc = solve_levels_once(h, init, first, warps_s, max_s, dst, st);
     if (rc != kRetryHostPaced) return rc;
-    set_persist_host_paced(true);
+    if (turn.own_rules()) set_persist_host_paced(true);
+    else PersistTurn::pace(h);
+    h->run_persist = false;
     h->timed.clear();   // launch events of the abandoned solve
     const int rc2 = solve_levels_once(h, init, first, warps_s, max_s, dst, st);
     if (rc2 == kRetryHostPaced) {   // the mode was set back to persistent meanwhile

@@ -15,6 +15,8 @@ namespace amdflow {
 
 constexpr int kInFlight = 3;   // iteration launches kept queued ahead of the device
 
+constexpr int kPacedMost = 4096;   // host-paced solves after a launch that was not co-resident, at most
+
 // Launch shape for scales of at least `min_pixels` pixels.
 struct LaunchRule {
     long long min_pixels;
@@ -72,6 +74,9 @@ struct of_tvl1 {
     std::vector<int> h_iters;
     amdflow::GaussTaps g_pre{}, g_zoom{};
     std::vector<amdflow::LaunchRule> rules;
+    bool run_persist = false;   // the built-in persistent rules apply to this solve
+    int paced_solves = 0;       // solves that still take the host-paced ones
+    int paced_next = 16;        // how many after the next launch that is not co-resident
     long long launches_issued = 0;
     int inflight = amdflow::kInFlight;
     double host_launch_s = 0.0, host_wait_s = 0.0;

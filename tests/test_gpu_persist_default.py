@@ -1,0 +1,119 @@
+"""Built-in launch rules: one launch per warping with neighbour flags while no
+other solve of the process runs persistent warpings on the device, host-paced
+launches otherwise.  The kernels compute the oracle's expressions in the
+oracle's order, so every path has to give its bits."""
+import threading
+
+import numpy as np
+import pytest
+
+import oracle as O
+from amdflow import PERSIST_HOST_PACED, PERSIST_PLAIN, TV_L1, persist_launch_mode, \
+    set_persist_launch_mode, synth
+from amdflow import debug as D
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture
+def restore_mode():
+    set_persist_launch_mode(PERSIST_PLAIN)
+    yield
+    D.persist_force_not_resident(False)
+    set_persist_launch_mode(PERSIST_PLAIN)
+
+
+def _pair(w, h, seed):
+    I0, I1, _, _ = synth.make_pair(w, h, 4.0, seed, bumps=True)
+    return synth.quantize(I0), synth.quantize(I1)
+
+
+def _solve(tv, q0, q1):
+    """(flow, iterations, the launch modes the solve's scales took)."""
+    tv.profile(True)
+    tv.runDualTVL1Multiscale(q0, q1)
+    modes = {p["persistent"] for p in tv.profile_results() if p["launches"]}
+    tv.profile(False)
+    return tv.getU().copy(), tv.iterations(), modes
+
+
+def _check(got, q0, q1, **prm):
+    uo, ito = O.tvl1(q0, q1, O.default_params(**prm))
+    assert np.array_equal(got[1], ito)
+    assert np.array_equal(got[0], uo)
+
+
+@pytest.mark.parametrize("w,h,ns", [(16, 9, 1), (320, 240, 5), (641, 479, 5), (1600, 999, 2),
+                                    (1601, 1000, 2)])
+def test_builtin_rules_match_oracle(w, h, ns, restore_mode):
+    print("builtin", w, h, flush=True)
+    q0, q1 = _pair(w, h, 61)
+    prm = dict(nscales=ns, max_iterations=60)
+    with TV_L1(w, h, **prm) as tv:
+        got = _solve(tv, q0, q1)
+    assert got[2] == {2}
+    _check(got, q0, q1, **prm)
+
+
+def test_iteration_limits_past_the_flags_run_host_paced(restore_mode):
+    """A flag numbers up to 2^20 chunks: longer limits keep the host-paced
+    launches, and stop where the flow does."""
+    q0, q1 = _pair(64, 48, 62)
+    prm = dict(nscales=2, max_iterations=(1 << 20) + 1)
+    with TV_L1(64, 48, **prm) as tv:
+        got = _solve(tv, q0, q1)
+    assert got[2] == {0}
+    _check(got, q0, q1, **prm)
+
+
+def test_not_resident_keeps_the_process_and_paces_the_handle(restore_mode):
+    q0, q1 = _pair(160, 120, 63)
+    with TV_L1(160, 120, nscales=3) as tv:
+        D.persist_force_not_resident(True)
+        tv.runDualTVL1Multiscale(q0, q1)
+        first = (tv.getU().copy(), tv.iterations())
+        D.persist_force_not_resident(False)
+        assert persist_launch_mode() == PERSIST_PLAIN
+        again = [_solve(tv, q0, q1) for _ in range(17)]
+    assert all(g[2] == {0} for g in again[:16]) and again[16][2] == {2}
+    for got in [first] + again:
+        _check(got, q0, q1, nscales=3)
+
+
+def test_host_paced_process_takes_host_paced_rules(restore_mode):
+    q0, q1 = _pair(160, 120, 64)
+    set_persist_launch_mode(PERSIST_HOST_PACED)
+    with TV_L1(160, 120, nscales=3) as tv:
+        got = _solve(tv, q0, q1)
+    assert got[2] == {0}
+    _check(got, q0, q1, nscales=3)
+
+
+def test_solves_from_several_threads(restore_mode):
+    """One solve at a time takes the persistent rules, the others run host-paced
+    beside it."""
+    pairs = [_pair(320, 240, 70 + k) for k in range(3)]
+    want = [O.tvl1(q0, q1, O.default_params(nscales=4)) for q0, q1 in pairs]
+    results, errors = [[] for _ in pairs], []
+
+    def worker(k):
+        try:
+            with TV_L1(320, 240, nscales=4) as tv:
+                for _ in range(5):
+                    tv.runDualTVL1Multiscale(*pairs[k])
+                    results[k].append((tv.getU().copy(), tv.iterations()))
+        except Exception as e:   # reported by the main thread
+            errors.append(e)
+
+    th = [threading.Thread(target=worker, args=(k,)) for k in range(len(pairs))]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not errors, errors
+    assert persist_launch_mode() == PERSIST_PLAIN
+    for k, (uo, ito) in enumerate(want):
+        assert len(results[k]) == 5
+        for u, it in results[k]:
+            assert np.array_equal(it, ito)
+            assert np.array_equal(u, uo)
