@@ -119,6 +119,50 @@ __device__ __forceinline__ void bicubic_sample3(const float4* __restrict__ img, 
     c = cubic_cell(vc[0], vc[1], vc[2], vc[3], t.fx);
 }
 
+// v of the lane's partner in its pair of lanes (2k, 2k+1).
+__device__ __forceinline__ float lane_partner(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0xB1 /* quad_perm 1,0,3,2 */, 0xf, 0xf, true));
+}
+
+__device__ __forceinline__ int lane_partner(int v)
+{
+    return __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, true);
+}
+
+// bicubic_sample of two images by a whole wave whose lanes sample neighbouring
+// points: where every pair of lanes shares its 16 taps and the vertical
+// fraction (an enlargement by about 2), each lane forms two of the four
+// vertical cells and takes the others from its partner.  Same cells, same bits.
+__device__ __forceinline__ void bicubic_sample_pairs(const float* __restrict__ a, const float* __restrict__ b,
+                                                     int nx, const BicubicTaps& t, float& ra, float& rb)
+{
+    bool same = t.fy == __int_as_float(lane_partner(__float_as_int(t.fy)));
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+        same &= (t.cols[c] == lane_partner(t.cols[c])) & (t.rows[c] == lane_partner(t.rows[c]));
+    if (!__all(same)) {
+        ra = bicubic_sample(a, nx, t);
+        rb = bicubic_sample(b, nx, t);
+        return;
+    }
+    const bool odd = threadIdx.x & 1;
+    float va[2], vb[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        const int col = odd ? t.cols[c + 2] : t.cols[c];
+        const float *ca = a + col, *cb = b + col;
+        va[c] = cubic_cell(ca[(size_t)nx * t.rows[0]], ca[(size_t)nx * t.rows[1]], ca[(size_t)nx * t.rows[2]],
+                           ca[(size_t)nx * t.rows[3]], t.fy);
+        vb[c] = cubic_cell(cb[(size_t)nx * t.rows[0]], cb[(size_t)nx * t.rows[1]], cb[(size_t)nx * t.rows[2]],
+                           cb[(size_t)nx * t.rows[3]], t.fy);
+    }
+    const float pa0 = lane_partner(va[0]), pa1 = lane_partner(va[1]);
+    const float pb0 = lane_partner(vb[0]), pb1 = lane_partner(vb[1]);
+    ra = cubic_cell(odd ? pa0 : va[0], odd ? pa1 : va[1], odd ? va[0] : pa0, odd ? va[1] : pa1, t.fx);
+    rb = cubic_cell(odd ? pb0 : vb[0], odd ? pb1 : vb[1], odd ? vb[0] : pb0, odd ? vb[1] : pb1, t.fx);
+}
+
 __device__ __forceinline__ float bicubic_at(const float* __restrict__ img, float uu, float vv,
                                             int nx, int ny, bool border_out)
 {

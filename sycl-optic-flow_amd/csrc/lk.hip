@@ -183,25 +183,44 @@ __global__ __launch_bounds__(256) void k_lk_tensor_products(const float* __restr
 // 1280x720 3-level solve took 0.260 ms with 8 everywhere, 0.265 ms with 8
 // below 300,000 pixels and 16 above, 0.290 ms with 16 everywhere.
 constexpr int kLkTileRows = 8;
+constexpr int kLkMaxLevels = 16;
+constexpr int kLkCUs = 256;
 
 // The gradient, its products and their window sums in one launch, on a
 // 64 x kLkTileRows output tile: the products on the tile plus a WC-pixel halo (LDS),
 // their row sums, then the column sums into G (Gxx, Gxy, Gyy planes); Ix and
 // Iy are written for the output pixels.  Same expressions and summation
 // order as k_lk_tensor_products followed by k_lk_boxsum along rows and then
-// columns (windows clipped to the image, ascending order).
+// columns (windows clipped to the image, ascending order).  The tensors do not
+// depend on the flow, so one launch takes all levels: the coarse ones, too
+// small to fill the device, run beside the finest instead of before it, and
+// their launches go.
+struct LkTensorLevels {
+    int n;
+    int first[kLkMaxLevels];   // first block of each level
+    int w[kLkMaxLevels], h[kLkMaxLevels];
+    const float* p0[kLkMaxLevels];
+    float *Ix[kLkMaxLevels], *Iy[kLkMaxLevels], *G[kLkMaxLevels];
+};
+
 template <int WC, int TH = kLkTileRows>
-__global__ __launch_bounds__(256) void k_lk_tensor_fused(const float* __restrict__ P0, int w,
-                                                         int h, float* __restrict__ Ix,
-                                                         float* __restrict__ Iy,
-                                                         float* __restrict__ G)
+__global__ __launch_bounds__(256) void k_lk_tensor_fused(LkTensorLevels L)
 {
+    int l = 0;
+    while (l + 1 < L.n && (int)blockIdx.x >= L.first[l + 1]) l++;
+    const float* __restrict__ P0 = L.p0[l];
+    float* __restrict__ Ix = L.Ix[l];
+    float* __restrict__ Iy = L.Iy[l];
+    float* __restrict__ G = L.G[l];
+    const int w = L.w[l], h = L.h[l];
+    const int tiles_x = (w + 63) / 64, tile = (int)blockIdx.x - L.first[l];
+    const int bx = tile % tiles_x, by = tile / tiles_x;
     constexpr int TW = 64, EW = TW + 2 * WC, EH = TH + 2 * WC;
     constexpr int NE = (EW * EH + 255) / 256;
     constexpr int NO = TW * TH / 256;
     __shared__ float pr[3][EH][EW];
     __shared__ float rs[3][EH][TW];
-    const int x0 = blockIdx.x * TW, y0 = blockIdx.y * TH;
+    const int x0 = bx * TW, y0 = by * TH;
     const size_t n = (size_t)w * h;
     // the four neighbour loads of every element are issued without branches
     // (outside the image: clamped, in-range addresses, result discarded)
@@ -354,20 +373,24 @@ __global__ __launch_bounds__(256) void k_lk_update(const float* __restrict__ row
     }
 }
 
-// kk whole iterations on a 64 x 64 tile in one launch (temporal blocking):
-// the iteration at a pixel reads the flow of every pixel of its window, so
-// after t iterations a tile's flow is exact at distance >= t*WC from its
-// edge, and the tile stores its central (64 - 2*kk*WC)^2 pixels.  Wave r of
-// the 16 holds tile rows 4r .. 4r+3 (lane = column) with their flow, frame,
-// gradient and tensor values in registers.  A row of window products lies
-// in one wave, so the row sums take their neighbours through DPP lane
-// shifts; the column sums read the 2*WC rows next to a thread's four from
-// LDS (row sums, double-buffered: one barrier per iteration).  The
-// per-pixel arithmetic and both summation orders are those of the
-// three-kernel iteration k_lk_it_products / k_lk_boxsum / k_lk_update (the
-// windows clipped to the image), so the flow is the same bits as kk rounds
-// of it.
-constexpr int kLkBlockEdge = 64;
+// kk whole iterations on a tile of 64 columns by 16*NP rows in one launch
+// (temporal blocking): the iteration at a pixel reads the flow of every pixel
+// of its window, so after t iterations a tile's flow is exact at distance >=
+// t*WC from its edge, and the tile stores its centre, 2*kk*WC pixels smaller
+// each way.  Wave r of the 16 holds tile rows NP*r .. NP*r+NP-1 (lane =
+// column) with their flow, frame, gradient and tensor values in registers.  A
+// row of window products lies in one wave, so the row sums take their
+// neighbours through DPP lane shifts; the column sums read the 2*WC rows next
+// to a thread's own from LDS (row sums, double-buffered: one barrier per
+// iteration).  The per-pixel arithmetic and both summation orders are those of
+// the three-kernel iteration k_lk_it_products / k_lk_boxsum / k_lk_update (the
+// windows clipped to the image), so the flow is the same bits as kk rounds of
+// it.  A null u starts from zero flow.
+// Bound by VALU issue: 0.95 us per iteration and row of each wave.  Row sums as
+// shifted adds and tap pairs from one address took a 1280 x 720 solve (3 levels,
+// 7 x 7, 5 iterations) from 172 to 157 us.  Tried and slower: 512 threads of 8
+// rows (172 us), a cap of 64 registers so that two workgroups share a CU (204
+// us, spills).
 
 // Whole-wave lane shifts for the row sums: lane i gets lane i-1's (from the
 // left) or lane i+1's value; the lane without a source gets 0.  Those lanes
@@ -398,7 +421,14 @@ __device__ __forceinline__ float load_at(const float* __restrict__ img, int idx)
     return *reinterpret_cast<const float*>(reinterpret_cast<const char*>(img) + (unsigned)idx * 4u);
 }
 
-template <int WC>
+// img[idx], img[idx + 1] in one load of 4-byte alignment.
+typedef float PairAt __attribute__((ext_vector_type(2), aligned(4)));
+__device__ __forceinline__ PairAt load_pair(const float* __restrict__ img, int idx)
+{
+    return *reinterpret_cast<const PairAt*>(reinterpret_cast<const char*>(img) + (unsigned)idx * 4u);
+}
+
+template <int WC, int NP>
 __global__ __launch_bounds__(1024) void k_lk_iters_blocked(const float* __restrict__ P0,
                                                            const float* __restrict__ P1,
                                                            const float* __restrict__ Ix,
@@ -410,17 +440,16 @@ __global__ __launch_bounds__(1024) void k_lk_iters_blocked(const float* __restri
                                                            float* __restrict__ uo,
                                                            float* __restrict__ vo)
 {
-    constexpr int E = kLkBlockEdge;
-    constexpr int NP = E * E / 1024;   // rows per thread
-    __shared__ float rs[2][2][E][E];   // [buffer][plane][row][column]
+    constexpr int E = 64, EY = 16 * NP;   // columns and rows of the tile
+    __shared__ float rs[2][2][EY][E];     // [buffer][plane][row][column]
     const int halo = kk * WC;
-    const int O = E - 2 * halo;
-    const int x0 = (int)blockIdx.x * O - halo, y0 = (int)blockIdx.y * O - halo;
+    const int x0 = (int)blockIdx.x * (E - 2 * halo) - halo, y0 = (int)blockIdx.y * (EY - 2 * halo) - halo;
     const int ex = threadIdx.x & 63, ey0 = (threadIdx.x >> 6) * NP;
     const size_t n = (size_t)w * h;
     const int gx = x0 + ex;
     const bool xin = gx >= 0 && gx < w;
 
+    constexpr int kRowsAtOnce = NP < 2 ? 1 : 2;
     float uu[NP], vv[NP], i0[NP], gxv[NP], gyv[NP], gxx[NP], gxy[NP], gyy[NP];
     bool in[NP];
     const float* __restrict__ Gxy = G + n;
@@ -430,8 +459,8 @@ __global__ __launch_bounds__(1024) void k_lk_iters_blocked(const float* __restri
         const int gy = y0 + ey0 + k;
         in[k] = xin && gy >= 0 && gy < h;
         const int p = in[k] ? gy * w + gx : 0;
-        uu[k] = in[k] ? load_at(u, p) : 0.0f;
-        vv[k] = in[k] ? load_at(v, p) : 0.0f;
+        uu[k] = in[k] && u ? load_at(u, p) : 0.0f;
+        vv[k] = in[k] && u ? load_at(v, p) : 0.0f;
         i0[k] = load_at(P0, p);
         gxv[k] = load_at(Ix, p);
         gyv[k] = load_at(Iy, p);
@@ -440,61 +469,86 @@ __global__ __launch_bounds__(1024) void k_lk_iters_blocked(const float* __restri
         gyy[k] = load_at(Gyy, p);
     }
     for (int it = 0; it < kk; it++) {
-        const int lo1 = (it + 1) * WC, hi1 = E - (it + 1) * WC;   // flow exact here after it
+        // the flow is exact in columns lo1 .. hi1-1 and rows lo1 .. hy1-1 after it
+        const int lo1 = (it + 1) * WC, hi1 = E - (it + 1) * WC, hy1 = EY - (it + 1) * WC;
         const int b = it & 1;
-        // the window products of all four rows (k_lk_it_products'); the taps
-        // are clamped into the frame, so every gather is in bounds and all of
-        // them are issued before the first is used.  Values outside the
-        // square where the flow is exact are computed and never used.
-        float ta[NP], tb[NP], tc[NP], td[NP], ax[NP], ay[NP];
-#pragma unroll
-        for (int k = 0; k < NP; k++) {
-            const int gy = y0 + ey0 + k;
-            const float x = (float)gx + uu[k], y = (float)gy + vv[k];
-            const float fx0 = floorf(x), fy0 = floorf(y);
-            ax[k] = x - fx0;
-            ay[k] = y - fy0;
-            const int xi = floor_index(fx0, w), yi = floor_index(fy0, h);
-            const int xa = clampi(xi, 0, w - 1), xb = clampi(xi + 1, 0, w - 1);
-            const int ya = clampi(yi, 0, h - 1), yb = clampi(yi + 1, 0, h - 1);
-            const int ra = (int)__umul24((unsigned)ya, (unsigned)w);
-            const int rb = (int)__umul24((unsigned)yb, (unsigned)w);
-            ta[k] = load_at(P1, ra + xa);
-            tb[k] = load_at(P1, ra + xb);
-            tc[k] = load_at(P1, rb + xa);
-            td[k] = load_at(P1, rb + xb);
-        }
+        // the window products (k_lk_it_products'), kRowsAtOnce rows at a
+        // time.  A wave whose taps all lie in the frame loads them in pairs
+        // from one address; otherwise they are clamped into the frame.  Every
+        // gather is in bounds and those of the rows are issued before the
+        // first is used.  Values outside the square where the flow is exact
+        // are computed and never used.
         float r0[NP], r1[NP];   // row sums of this thread's rows
 #pragma unroll
-        for (int k = 0; k < NP; k++) {
-            const float top = (1.0f - ax[k]) * ta[k] + ax[k] * tb[k];
-            const float bot = (1.0f - ax[k]) * tc[k] + ax[k] * td[k];
-            const float wv = (1.0f - ay[k]) * top + ay[k] * bot;
-            const float itv = wv - i0[k];
-            float a[2 * WC + 1], c[2 * WC + 1];   // products at columns ex - WC .. ex + WC
-            a[WC] = in[k] ? gxv[k] * itv : 0.0f;
-            c[WC] = in[k] ? gyv[k] * itv : 0.0f;
+        for (int h0 = 0; h0 < NP; h0 += kRowsAtOnce) {
+            constexpr int M = kRowsAtOnce;
+            float ta[M], tb[M], tc[M], td[M], ax[M], ay[M], fx0[M], fy0[M];
+            bool inner = true;
 #pragma unroll
-            for (int d = 1; d <= WC; d++) {
-                a[WC + d] = lane_from_right0(a[WC + d - 1]);
-                c[WC + d] = lane_from_right0(c[WC + d - 1]);
-                a[WC - d] = lane_from_left0(a[WC - d + 1]);
-                c[WC - d] = lane_from_left0(c[WC - d + 1]);
+            for (int k = 0; k < M; k++) {
+                const int gy = y0 + ey0 + h0 + k;
+                const float x = (float)gx + uu[h0 + k], y = (float)gy + vv[h0 + k];
+                fx0[k] = floorf(x);
+                fy0[k] = floorf(y);
+                ax[k] = x - fx0[k];
+                ay[k] = y - fy0[k];
+                inner &= (fx0[k] >= 0.0f) & (fx0[k] < (float)(w - 1)) & (fy0[k] >= 0.0f) & (fy0[k] < (float)(h - 1));
             }
-            // every tap is added: a tap outside the image carries +0.0 (its
-            // lane's `in` is false), and s + (+0.0) is s for every s but
-            // -0.0, which a sum that starts at +0.0 never is; so the sum has
-            // the bits of the image-clipped window sum
-            float s0 = 0.0f, s1 = 0.0f;
+            if (__all(inner)) {
 #pragma unroll
-            for (int q = 0; q <= 2 * WC; q++) {
-                s0 += a[q];
-                s1 += c[q];
+                for (int k = 0; k < M; k++) {
+                    const int p = (int)(__umul24((unsigned)(int)fy0[k], (unsigned)w) + (unsigned)(int)fx0[k]);
+                    const PairAt top = load_pair(P1, p), bot = load_pair(P1, p + w);
+                    ta[k] = top.x;
+                    tb[k] = top.y;
+                    tc[k] = bot.x;
+                    td[k] = bot.y;
+                }
+            } else {
+#pragma unroll
+                for (int k = 0; k < M; k++) {
+                    const int xi = floor_index(fx0[k], w), yi = floor_index(fy0[k], h);
+                    const int xa = clampi(xi, 0, w - 1), xb = clampi(xi + 1, 0, w - 1);
+                    const int ya = clampi(yi, 0, h - 1), yb = clampi(yi + 1, 0, h - 1);
+                    const int ra = (int)__umul24((unsigned)ya, (unsigned)w);
+                    const int rb = (int)__umul24((unsigned)yb, (unsigned)w);
+                    ta[k] = load_at(P1, ra + xa);
+                    tb[k] = load_at(P1, ra + xb);
+                    tc[k] = load_at(P1, rb + xa);
+                    td[k] = load_at(P1, rb + xb);
+                }
             }
-            r0[k] = s0;
-            r1[k] = s1;
-            rs[b][0][ey0 + k][ex] = s0;
-            rs[b][1][ey0 + k][ex] = s1;
+#pragma unroll
+            for (int k = 0; k < M; k++) {
+                const int r = h0 + k;
+                const float top = (1.0f - ax[k]) * ta[k] + ax[k] * tb[k];
+                const float bot = (1.0f - ax[k]) * tc[k] + ax[k] * td[k];
+                const float wv = (1.0f - ay[k]) * top + ay[k] * bot;
+                const float itv = wv - i0[r];
+                const float a = in[r] ? gxv[r] * itv : 0.0f, c = in[r] ? gyv[r] * itv : 0.0f;
+                // the sums of the 2*WC+1 products that end at this column,
+                // left to right from +0.0: shift the sum, add this column's
+                // (the shift is part of the add).  Then WC shifts put them at
+                // their centre.  Every tap is added: a tap outside the image
+                // carries +0.0 (its lane's `in` is false), and s + (+0.0) is s
+                // for every s but -0.0, which a sum that starts at +0.0 never
+                // is; so the sum has the bits of the image-clipped window sum
+                float s0 = 0.0f + a, s1 = 0.0f + c;
+#pragma unroll
+                for (int d = 1; d <= 2 * WC; d++) {
+                    s0 = lane_from_left0(s0) + a;
+                    s1 = lane_from_left0(s1) + c;
+                }
+#pragma unroll
+                for (int d = 0; d < WC; d++) {
+                    s0 = lane_from_right0(s0);
+                    s1 = lane_from_right0(s1);
+                }
+                r0[r] = s0;
+                r1[r] = s1;
+                rs[b][0][ey0 + r][ex] = s0;
+                rs[b][1][ey0 + r][ex] = s1;
+            }
         }
         __syncthreads();
         // column sums of rows ey0 - WC .. ey0 + NP - 1 + WC: the thread's own
@@ -504,7 +558,7 @@ __global__ __launch_bounds__(1024) void k_lk_iters_blocked(const float* __restri
 #pragma unroll
         for (int j = 0; j < WC; j++) {
             const int ra = ey0 - WC + j < 0 ? 0 : ey0 - WC + j;
-            const int rb = ey0 + NP + j > E - 1 ? E - 1 : ey0 + NP + j;
+            const int rb = ey0 + NP + j > EY - 1 ? EY - 1 : ey0 + NP + j;
             y0s[j] = rs[b][0][ra][ex];
             y1s[j] = rs[b][1][ra][ex];
             y0s[WC + NP + j] = rs[b][0][rb][ex];
@@ -520,7 +574,7 @@ __global__ __launch_bounds__(1024) void k_lk_iters_blocked(const float* __restri
 #pragma unroll
         for (int k = 0; k < NP; k++) {
             const int ey = ey0 + k;
-            if (!in[k] || ey < lo1 || ey >= hi1 || ex < lo1 || ex >= hi1) continue;
+            if (!in[k] || ey < lo1 || ey >= hy1 || ex < lo1 || ex >= hi1) continue;
             float bx = 0.0f, by = 0.0f;
 #pragma unroll
             for (int q = -WC; q <= WC; q++) {
@@ -542,28 +596,44 @@ __global__ __launch_bounds__(1024) void k_lk_iters_blocked(const float* __restri
 #pragma unroll
     for (int k = 0; k < NP; k++) {
         const int ey = ey0 + k, gy = y0 + ey;
-        if (!in[k] || ey < halo || ey >= E - halo || ex < halo || ex >= E - halo) continue;
+        if (!in[k] || ey < halo || ey >= EY - halo || ex < halo || ex >= E - halo) continue;
         const size_t p = (size_t)gy * w + gx;
         uo[p] = uu[k];
         vo[p] = vv[k];
     }
 }
 
-// Iterations per launch of k_lk_iters_blocked.  A launch stores the centre
-// (64 - 2*kk*WC)^2 of each 64 x 64 tile, so (64 / (64 - 2*kk*WC))^2 pixels
-// are read and iterated per stored pixel.  Levels of at most kLkSmallLevel
-// pixels have too few tiles to fill the GPU and take the deepest blocks (a
-// centre of at least 32 pixels per side); larger levels keep the halo within
-// 9 pixels (1.9 pixels iterated per stored one at WC = 3, kk = 3).  On 1280 x
-// 720 frames, 3 levels and 7 x 7 windows the solve took 0.241 ms with one
-// launch per iteration on every level, 0.226 ms with blocks on the two small
-// levels only, 0.212 ms with level 0 in blocks of 3 and 0.244 ms in blocks
-// of 5 (blocks of 2 were slower than blocks of 3 in an earlier version of
-// the kernel).
-constexpr long long kLkSmallLevel = 300000;
-constexpr int lk_block_iters(int wc, long long npix)
+// Shape of k_lk_iters_blocked for the iterations of one level: rows per thread
+// and iterations per launch, the cheapest of all by this estimate: a launch
+// costs 3 us, a row of its threads 0.75 us for the loads and stores and 0.95 us
+// per iteration, times the tiles per CU.  Small levels thus take fewer rows per
+// thread, which spread over more CUs, large ones the least work in halos.
+// Estimated and measured: 1280x720, 7 x 7: (4 rows, 3 iterations) 31.8, 33.3 us,
+// (4, 2) 24.2, 24.7; 640x360 (4, 5) 25.0, 23.9; 320x180 (2, 3) 10.2, 7.9 and (2,
+// 2) 8.3, 5.7, in place of (4, 5) 18.6; 161x121, 5 x 5: (1, 3) 6.6, 6.1.
+// Whole solves against one shape of 4 rows: 161x121, 2 levels, 3 iterations 55 ->
+// 38 us; 640x480, 3 levels, 3 x 3, 4 iterations 103 -> 76 us.
+struct LkShape {
+    int rows, iters;
+};
+
+inline LkShape lk_block_shape(int wc, int w, int h, int iters)
 {
-    return npix <= kLkSmallLevel ? (kLkBlockEdge - 32) / (2 * wc) : (9 / wc > 1 ? 9 / wc : 1);
+    LkShape best{4, 1};
+    double least = 1e300;
+    for (int rows = 4; rows >= 1; rows /= 2)
+        for (int kk = 1; kk <= iters && 16 * rows - 2 * kk * wc > 0; kk++) {
+            auto cost = [&](int k) {
+                const long long tiles = (long long)cdiv(w, 64 - 2 * k * wc) * cdiv(h, 16 * rows - 2 * k * wc);
+                return 3.0 + (0.75 + 0.95 * k) * rows * (double)((tiles + kLkCUs - 1) / kLkCUs);
+            };
+            const double c = iters / kk * cost(kk) + (iters % kk ? cost(iters % kk) : 0.0);
+            if (c < least) {
+                least = c;
+                best = LkShape{rows, kk};
+            }
+        }
+    return best;
 }
 
 // One pyramid step of both frames per launch (blockIdx.z = frame): the
@@ -628,8 +698,8 @@ unsigned g1(size_t n) { const unsigned g = cdiv(n, 256); return g > 4096 ? 4096 
 // caller's frames in place).
 struct LkPlan {
     int levels = 0;
-    int nx[16], ny[16];
-    size_t off[16];
+    int nx[kLkMaxLevels], ny[kLkMaxLevels];
+    size_t off[kLkMaxLevels];
     size_t pyr = 0;   // floats of levels 1.. per frame
     size_t n0 = 0;    // pixels of level 0
     GaussTaps g;
@@ -638,7 +708,7 @@ struct LkPlan {
 int lk_plan(int W, int H, int levels, float zf, float sigma, int win, int iters, LkPlan* P)
 {
     if (W < 2 || H < 2) return OF_ERR_ARG;
-    if (levels < 1 || levels > 16 || win < 1 || (win & 1) == 0 || iters < 0) return OF_ERR_ARG;
+    if (levels < 1 || levels > kLkMaxLevels || win < 1 || (win & 1) == 0 || iters < 0) return OF_ERR_ARG;
     if (!(zf > 0 && zf < 1) || !(sigma > 0)) return OF_ERR_ARG;
     OF_TRY(gaussian_taps((double)sigma, &P->g));
     P->levels = levels;
@@ -664,7 +734,9 @@ struct LkBufs {
     float *P0, *P1;            // pyramid levels 1.. of each frame (LkPlan::off)
     float *Ix, *Iy, *u, *v, *nu, *nv;   // one plane of level 0's size each
     float *PROD, *ROWS, *GT;   // three planes each: per-pixel products, their
-                               // row sums, the structure tensor Gxx, Gxy, Gyy
+                               // row sums, the structure tensor Gxx, Gxy, Gyy;
+                               // PROD and ROWS also hold blurred frames, PROD the
+                               // coarser levels' gradients and tensors
 };
 
 size_t lk_round(size_t n) { return (n + 63) & ~(size_t)63; }   // 256-byte multiples
@@ -766,23 +838,55 @@ int lk_pyr_run(const LkPlan& P, const LkBufs& B, const float* dI0, const float* 
                         !overlaps(du, dI0, n0) && !overlaps(du, dI1, n0) &&
                         !overlaps(dv, dI0, n0) && !overlaps(dv, dI1, n0);
     const float invZ = 1 / zf;
-    {
+    const bool zero_start = blocked && iters >= 1;   // the first iterations need no cleared flow
+    if (!zero_start) {
         const size_t nc = (size_t)nx[levels - 1] * ny[levels - 1];
         hipLaunchKernelGGL(k_lk_zero2, dim3(g1(nc)), dim3(256), 0, st, u, v, nc);
         LK_CHECK("k_lk_zero2");
     }
+    // gradient, products and both window sums of levels l0 .. l1 in one launch
+    auto tensors = [&](int l0, int l1, auto&& planes) -> int {
+        LkTensorLevels T{};
+        size_t blocks = 0;
+        for (int l = l0; l <= l1; l++) {
+            const int i = T.n++;
+            T.first[i] = (int)blocks;
+            T.w[i] = nx[l];
+            T.h[i] = ny[l];
+            T.p0[i] = L0[l];
+            planes(l, &T.Ix[i], &T.Iy[i], &T.G[i]);
+            blocks += (size_t)cdiv(nx[l], 64) * cdiv(ny[l], kLkTileRows);
+        }
+        const dim3 tgrid((unsigned)blocks);
+        if (wc == 1) hipLaunchKernelGGL((k_lk_tensor_fused<1>), tgrid, dim3(256), 0, st, T);
+        if (wc == 2) hipLaunchKernelGGL((k_lk_tensor_fused<2>), tgrid, dim3(256), 0, st, T);
+        if (wc == 3) hipLaunchKernelGGL((k_lk_tensor_fused<3>), tgrid, dim3(256), 0, st, T);
+        if (wc == 4) hipLaunchKernelGGL((k_lk_tensor_fused<4>), tgrid, dim3(256), 0, st, T);
+        LK_CHECK("k_lk_tensor_fused");
+        return OF_OK;
+    };
+    // The coarser levels' tensors take the blur buffers, free by now, where
+    // five planes of every level fit one (at a zoom factor of 1/2: 5/3 of the
+    // 3 planes); otherwise each level's are formed when it is its turn.
+    const bool fused = wc >= 1 && wc <= 4;
+    const bool together = fused && 5 * P.pyr <= 3 * n0;
+    auto level_planes = [&](int l, float** ix, float** iy, float** gt) {
+        const bool own = l > 0 && together;
+        const size_t m = (size_t)nx[l] * ny[l];
+        float* q = own ? PROD + 5 * off[l] : nullptr;
+        *ix = own ? q : Ix;
+        *iy = own ? q + m : Iy;
+        *gt = own ? q + 2 * m : GT;
+    };
+    if (together) OF_TRY(tensors(0, levels - 1, level_planes));
     for (int l = levels - 1; l >= 0; l--) {
         const int w = nx[l], h = ny[l];
         const float* p0 = L0[l];
         const float* p1 = L1[l];
-        const dim3 fgrid(cdiv(w, 64), cdiv(h, kLkTileRows));
-        if (wc >= 1 && wc <= 4) {
-            // gradient, products and both window sums in one launch
-            if (wc == 1) hipLaunchKernelGGL((k_lk_tensor_fused<1>), fgrid, dim3(256), 0, st, p0, w, h, Ix, Iy, GT);
-            if (wc == 2) hipLaunchKernelGGL((k_lk_tensor_fused<2>), fgrid, dim3(256), 0, st, p0, w, h, Ix, Iy, GT);
-            if (wc == 3) hipLaunchKernelGGL((k_lk_tensor_fused<3>), fgrid, dim3(256), 0, st, p0, w, h, Ix, Iy, GT);
-            if (wc == 4) hipLaunchKernelGGL((k_lk_tensor_fused<4>), fgrid, dim3(256), 0, st, p0, w, h, Ix, Iy, GT);
-            LK_CHECK("k_lk_tensor_fused");
+        float *lix, *liy, *lgt;
+        level_planes(l, &lix, &liy, &lgt);
+        if (fused) {
+            if (!together) OF_TRY(tensors(l, l, level_planes));
         } else {
             hipLaunchKernelGGL(k_lk_tensor_products, grid2d(w, h), dim3(256), 0, st, p0, w, h, Ix,
                                Iy, PROD);
@@ -795,19 +899,24 @@ int lk_pyr_run(const LkPlan& P, const LkBufs& B, const float* dI0, const float* 
             LK_CHECK("k_lk_boxsum");
         }
         // windows up to 9 x 9: blocks of iterations per launch (k_lk_iters_blocked)
+        const LkShape shape = blocked ? lk_block_shape(wc, w, h, iters) : LkShape{0, 0};
         for (int it = 0; it < iters && blocked;) {
-            const int kb = lk_block_iters(wc, (long long)w * h);
-            const int kk = iters - it < kb ? iters - it : kb;
-            const int O = kLkBlockEdge - 2 * kk * wc;
-            const dim3 bgrid(cdiv(w, O), cdiv(h, O));
+            const int kk = iters - it < shape.iters ? iters - it : shape.iters;
+            const dim3 bgrid(cdiv(w, 64 - 2 * kk * wc), cdiv(h, 16 * shape.rows - 2 * kk * wc));
+            const bool zero = zero_start && l == levels - 1 && it == 0;
             if (direct && l == 0 && it + kk == iters) {
                 nu = du;
                 nv = dv;
             }
-            if (wc == 1) hipLaunchKernelGGL((k_lk_iters_blocked<1>), bgrid, dim3(1024), 0, st, p0, p1, Ix, Iy, GT, u, v, w, h, det_eps, kk, nu, nv);
-            if (wc == 2) hipLaunchKernelGGL((k_lk_iters_blocked<2>), bgrid, dim3(1024), 0, st, p0, p1, Ix, Iy, GT, u, v, w, h, det_eps, kk, nu, nv);
-            if (wc == 3) hipLaunchKernelGGL((k_lk_iters_blocked<3>), bgrid, dim3(1024), 0, st, p0, p1, Ix, Iy, GT, u, v, w, h, det_eps, kk, nu, nv);
-            if (wc == 4) hipLaunchKernelGGL((k_lk_iters_blocked<4>), bgrid, dim3(1024), 0, st, p0, p1, Ix, Iy, GT, u, v, w, h, det_eps, kk, nu, nv);
+#define LK_ITERS(WC, NP)                                                                           \
+    if (wc == WC && shape.rows == NP)                                                              \
+    hipLaunchKernelGGL((k_lk_iters_blocked<WC, NP>), bgrid, dim3(1024), 0, st, p0, p1, lix, liy, lgt, \
+                       zero ? nullptr : u, zero ? nullptr : v, w, h, det_eps, kk, nu, nv)
+            LK_ITERS(1, 1); LK_ITERS(1, 2); LK_ITERS(1, 4);
+            LK_ITERS(2, 1); LK_ITERS(2, 2); LK_ITERS(2, 4);
+            LK_ITERS(3, 1); LK_ITERS(3, 2); LK_ITERS(3, 4);
+            LK_ITERS(4, 1); LK_ITERS(4, 2); LK_ITERS(4, 4);
+#undef LK_ITERS
             LK_CHECK("k_lk_iters_blocked");
             float* t = u; u = nu; nu = t;
             t = v; v = nv; nv = t;

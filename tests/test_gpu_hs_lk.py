@@ -164,6 +164,36 @@ def test_lk_pyramidal_blocked_levels_match_oracle(w, h, win, iters):
     assert np.array_equal(u, ou) and np.array_equal(v, ov)
 
 
+# Rows per thread and iterations per launch follow the level's size and window:
+# 1, 2 and 4 rows with a shorter last launch, levels one pixel beyond a tile's
+# centre, frames lower or narrower than one tile.  Zoom factors 1/2 and 0.6
+# sample in pairs of lanes in part of the waves or none; at 0.8 the levels'
+# tensors do not fit one buffer and are formed level by level.  The arithmetic
+# is the oracle's: no difference.
+@pytest.mark.parametrize("w,h,win,iters,levels,zf", [(40, 30, 5, 4, 1, 0.5), (53, 13, 3, 3, 1, 0.5),
+                                                     (105, 65, 3, 8, 2, 0.5), (161, 121, 9, 4, 2, 0.5),
+                                                     (333, 251, 7, 5, 3, 0.5), (643, 361, 5, 4, 2, 0.5),
+                                                     (1283, 701, 3, 3, 2, 0.5), (901, 701, 9, 3, 1, 0.5),
+                                                     (200, 150, 5, 2, 3, 0.8), (211, 157, 3, 4, 3, 0.6)])
+def test_lk_pyramidal_shapes_by_size_match_oracle(w, h, win, iters, levels, zf):
+    I0, I1, _, _ = synth.make_pair(w, h, 3.0, 51 + w + win)
+    u, v = lk_pyramidal(I0, I1, levels=levels, zf=zf, sigma=1.0, window=win, iters=iters, det_eps=1e-6)
+    ou, ov = O.lk_pyr(I0, I1, levels=levels, zf=zf, sigma=1.0, win=win, iters=iters, det_eps=1e-6)
+    assert np.array_equal(u, ou) and np.array_equal(v, ov)
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, 3e38])
+def test_lk_pyramidal_non_finite_frames_match_oracle(bad):
+    """A frame value that makes flows non-finite or huge: such waves take the
+    clamped taps, the others the paired ones."""
+    I0, I1, _, _ = synth.make_pair(150, 120, 3.0, 53)
+    I1 = I1.copy()
+    I1[60, 70] = bad
+    u, v = lk_pyramidal(I0, I1, levels=1, zf=0.5, sigma=1.0, window=5, iters=4, det_eps=1e-6)
+    ou, ov = O.lk_pyr(I0, I1, levels=1, zf=0.5, sigma=1.0, win=5, iters=4, det_eps=1e-6)
+    assert np.array_equal(u, ou, equal_nan=True) and np.array_equal(v, ov, equal_nan=True)
+
+
 def test_lk_pyramidal_1280x720_matches_oracle():
     """The LK workload: 1280x720, |flow| <= 8 px, 3 levels, 7x7, 5 iterations/level."""
     cfg = synth.CONFIGS["lk_1280x720"]
