@@ -187,6 +187,7 @@ void release(of_tvl1* h)
     dev_free(h->ctl);
     dev_free(h->partials);
     dev_free(h->tile_flags);
+    dev_free(h->halo);
     dev_free(h->energy);
     dev_free(h->d_iters);
     host_free(h->hflow);
@@ -302,6 +303,18 @@ int run_warping(of_tvl1* h, int s, int w, hipStream_t st)
         h->scale_P[s] = 0;
     }
     if (persistent) {
+        // tags of the warping's chunks (at least one iteration each); when they
+        // run out, the words are cleared and the tags start again
+        if (persistent == kPersistNeighbour) {
+            const unsigned tags = (unsigned)h->run_max + 1u;
+            if (h->halo_tag > 0xFFFFFFFFu - tags) {
+                OF_TRY(launch_fill((float*)h->halo, 2 * halo_words((size_t)h->W * h->H), 0.0f, st));
+                h->halo_tag = 0;
+            }
+            a.halo = h->halo;
+            a.tag0 = h->halo_tag;
+            h->halo_tag += tags;
+        }
         // the whole warping in one launch: no host involvement
         if (h->profiling) return timed_launch(h, K, R, persistent, a, st);
         h->launches_issued++;
@@ -739,6 +752,7 @@ int of_tvl1_create(const of_tvl1_params* params, int width, int height, of_tvl1*
         // x2: the persistent kernel double-buffers its partials by chunk parity
         if (!st) st = dev_alloc(&h->partials, 2 * maxpart);
         if (!st) st = dev_alloc(&h->tile_flags, maxtiles);
+        if (!st) st = dev_alloc(&h->halo, halo_words(N0));
         if (!st) st = dev_alloc(&h->energy, 2 * kEnergyBlocks + 3);
         if (!st) st = dev_alloc(&h->d_iters, (size_t)ns * p.warps);
         if (!st) st = host_alloc(&h->hflow, 2 * N0, hipHostMallocDefault);
@@ -753,7 +767,8 @@ int of_tvl1_create(const of_tvl1_params* params, int width, int height, of_tvl1*
         h->h_iters.assign((size_t)ns * p.warps, 0);
         // flags carry the warping's seq (from 1): zero means never set
         if (hipMemset(h->d_iters, 0, sizeof(int) * (size_t)ns * p.warps) != hipSuccess ||
-            hipMemset(h->tile_flags, 0, sizeof(unsigned long long) * maxtiles) != hipSuccess) {
+            hipMemset(h->tile_flags, 0, sizeof(unsigned long long) * maxtiles) != hipSuccess ||
+            hipMemset(h->halo, 0, sizeof(unsigned long long) * halo_words(N0)) != hipSuccess) {
             release(h);
             return OF_ERR_HIP;
         }

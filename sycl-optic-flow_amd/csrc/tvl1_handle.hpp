@@ -61,6 +61,8 @@ struct of_tvl1 {
     amdflow::TvCtl* ctl = nullptr;
     double* partials = nullptr;
     unsigned long long* tile_flags = nullptr;   // one word per tile (neighbour-synchronised warpings)
+    unsigned long long* halo = nullptr;         // halo_words(W*H): IterArgs::halo
+    unsigned halo_tag = 0;                      // tags up to this one have been used in it
     double* energy = nullptr;   // 2*kEnergyBlocks partials, then (E, data, TV)
     bool prepared = false;      // pyramids hold the last prepared pair
     bool solved = false;        // per-scale flows hold the last solve

@@ -1276,6 +1276,253 @@ __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist_nbr(IterArgs a, unsigned ti
 }
 
 // ---------------------------------------------------------------------------
+// neighbour-synchronised driver with tagged values
+// ---------------------------------------------------------------------------
+
+// The state of one pixel.
+struct SqState {
+    float u1, u2, p11, p12, p21, p22;
+    __device__ __forceinline__ void get(const SqPixel& q)
+    {
+        u1 = q.u1, u2 = q.u2, p11 = q.p11, p12 = q.p12, p21 = q.p21, p22 = q.p22;
+    }
+    __device__ __forceinline__ void put(SqPixel& q) const
+    {
+        q.u1 = u1, q.u2 = u2, q.p11 = p11, q.p12 = p12, q.p21 = p21, q.p22 = p22;
+    }
+};
+
+// A 32-bit value and its tag in one word: whoever reads the tag has the value.
+__device__ __forceinline__ void st_tagged(unsigned long long* w, unsigned tag, unsigned v)
+{
+    __hip_atomic_store(w, ((unsigned long long)tag << 32) | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Bounded wait of one wave until the N words at w, w + stride, .. of every lane
+// with `need` carry `tag`; v receives their values.  The bounds are wave_wait's;
+// false after flagging an error or once another workgroup has flagged one.
+template <int N>
+__device__ __forceinline__ bool wait_tagged(const IterArgs& a, const unsigned long long* w, size_t stride, int n,
+                                            bool need, unsigned tag, unsigned (&v)[N], const FirstBound& fb)
+{
+    TvCtl* ctl = a.ctl;
+    if (fb.force) {
+        __hip_atomic_store(&ctl->error, kBarNotResident, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return false;
+    }
+    const unsigned long long t_end = fb.ticks ? (unsigned long long)wall_clock64() + fb.ticks : 0ull;
+    unsigned spins = 0;
+    while (true) {
+        bool there = true;
+        if (need) {
+            unsigned long long x[N];
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                if (i < n) x[i] = __hip_atomic_load(w + i * stride, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int i = 0; i < N; i++)
+                if (i < n) {
+                    there &= (unsigned)(x[i] >> 32) == tag;
+                    v[i] = (unsigned)x[i];
+                }
+        }
+        if (__all(there)) return true;
+        __builtin_amdgcn_s_sleep(1);
+        if (++spins > (1u << 21)) {
+            __hip_atomic_store(&ctl->error, kBarTimeout, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            return false;
+        }
+        if (past_first_bound(fb, t_end, spins, ctl)) return false;
+        if ((spins & 1023u) == 0 &&
+            __hip_atomic_load(&ctl->error, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            return false;
+    }
+}
+
+// A whole warping on square tiles that all have a workgroup of their own
+// (blockIdx = tile, the last block is the referee).  The protocol and the
+// decisions are k_tvl1_persist_nbr's, the synchronisation is in the data: a
+// tile keeps its pixels in registers and stores only the ring that its
+// neighbours read, each value in one word with the tag tag0 + chunk + 1; they
+// wait for the words themselves.  No store is waited for and no flag follows
+// it.  Error partials go to the referee the same way.
+// Both parities of a word are safe to reuse: a tile stores chunk c after it has
+// read its neighbours' chunk c-1, which they stored after reading its chunk
+// c-2; partials and decisions likewise, since a tile sees decision c-2 before
+// it iterates chunk c.  By then it has chunk c-1's output in registers, and
+// keeps the inputs of chunks c-1 and c-2: "continue" goes on, "stop after keep
+// iterations of chunk c-2" takes chunk c-1's input or re-runs keep iterations
+// from chunk c-2's.  A tile never waits on work that waits on it, so no order of
+// the workgroups deadlocks, and the waits are bounded all the same.
+// Bound by the chain of an iteration and the exchange, about 3 us per chunk
+// where stores, flag and loads one after the other took 4.5.  Whole scales, ms:
+// 480x270 0.515 -> 0.464, 240x135 0.386 -> 0.349, 120x68 0.292 -> 0.257, 40x30 0.360
+// -> 0.307.  Four iterations per chunk instead of five, and polling without
+// sleeps, change no scale by more than 3%.
+template <int T, int K>
+__global__ OF_ITER_BOUNDS(T * T / 64, K) void k_tvl1_persist_tag(IterArgs a, unsigned tiles_x, unsigned ntiles)
+{
+    constexpr int NW = T * T / 64, C = T - 2 * K;
+    static_assert(C >= K, "the halo of a tile must lie within its neighbours");
+    static_assert(T * T > kSqOnePerCu && K <= kSqMaxIters, "the referee has a lane per tile");
+    __shared__ SqShared<T> sh;
+    __shared__ double sh_err[NW][K];
+    __shared__ double sh_tot[K];
+    __shared__ int sh_keep[2], sh_fail[2];
+
+    TvCtl* ctl = a.ctl;
+    const size_t plane = (size_t)a.plane;
+    unsigned long long* const parts = a.halo + 12 * plane;   // [parity][iteration][half][tile]
+    const int cur0 = uniform(ctl->cur[a.level]);
+    const int nchunks = (a.max_iter + K - 1) / K;
+
+    if (blockIdx.x == ntiles) {   // referee
+        int n = 0, c = 0;
+        while (c < nchunks) {
+            const int kk = min(K, a.max_iter - n);
+            const bool mine = threadIdx.x < ntiles;
+            unsigned v[2 * K] = {};
+            const bool ok = wait_tagged<2 * K>(a, parts + (size_t)(c & 1) * 2 * K * ntiles + threadIdx.x, ntiles,
+                                               2 * kk, mine, a.tag0 + (unsigned)c + 1u, v, FirstBound{0ull, 0});
+            if (!uniform(__syncthreads_and(ok))) return;
+            double s[K];
+#pragma unroll
+            for (int t = 0; t < K; t++)
+                s[t] = mine && t < kk ? __hiloint2double((int)v[2 * t + 1], (int)v[2 * t]) : 0.0;
+            const double tot = block_sum<K, NW>(s, sh_err, threadIdx.x);
+            if (threadIdx.x < (unsigned)K) sh_tot[threadIdx.x] = tot;
+            __syncthreads();
+            const int keep = uniform(stop_after(sh_tot, kk, n, a));
+            if (a.err_log && threadIdx.x < (unsigned)kk) a.err_log[n + threadIdx.x] = sh_tot[threadIdx.x];
+            if (threadIdx.x == 0)
+                __hip_atomic_store(&ctl->decision[c & 1].v,
+                                   (a.seq << 24) | ((unsigned long long)(c + 1) << 4) |
+                                       (unsigned long long)keep,
+                                   __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            n += keep ? keep : kk;
+            c++;
+            if (keep) break;
+            __syncthreads();   // sh_tot is rewritten next chunk
+        }
+        if (threadIdx.x == 0) {
+            ctl->cur[a.level] = cur0 ^ 1;
+            ctl->n = n;
+            ctl->stop = 1;
+            *a.iters_slot = n;
+        }
+        return;
+    }
+
+    const int bx = (int)(blockIdx.x % tiles_x), by = (int)(blockIdx.x / tiles_x);
+    const int lx = threadIdx.x % T, ly = threadIdx.x / T;
+    const int x = bx * C - K + lx, y = by * C - K + ly;
+    const bool in = x >= 0 && x < a.nx && y >= 0 && y < a.ny;
+    const bool centre = lx >= K && lx < K + C && ly >= K && ly < K + C;
+    // neighbours read the K outermost pixels of the centre
+    const bool ring = in && centre && (lx < 2 * K || lx >= C || ly < 2 * K || ly >= C);
+    const size_t idx = (size_t)y * a.nx + x;
+    SqPixel q;
+    q.fc = x == 0;
+    q.lc = x == a.nx - 1;
+    q.fr = y == 0;
+    q.lr = y == a.ny - 1;
+    q.mine = in && centre;
+    if (threadIdx.x < 2) sh_fail[threadIdx.x] = 0;
+    sq_load_constants<false>(a, q, in, idx);
+    sq_load_state<false>(a, q, in, idx, cur0);
+    __syncthreads();
+
+    // decision of chunk d, in wave 0: keep, or -1 if the wait failed
+    FirstBound fb{a.resident_ticks, a.force_not_resident};
+    auto decision = [&](int d) -> int {
+        const unsigned long long* w = &ctl->decision[d & 1].v;
+        const unsigned long long want = (a.seq << 24) | ((unsigned long long)(d + 1) << 4);
+        if (!wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, fb)) return -1;
+        return uniform((int)(__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFull));
+    };
+    SqState in0{}, in1{};   // inputs of the chunks before the last and last iterated
+    double acc[K];
+    int c = 0, keep = 0, full = 0;   // the warping stops after `keep` of the `full` iterations of a chunk
+    while (true) {
+        if (c > 0) {
+            bool ok = true;
+            if (c < nchunks) {
+                const size_t par = (size_t)((c - 1) & 1) * 6 * plane;
+                unsigned v[6] = {};
+                const bool need = in && !centre;
+                ok = wait_tagged<6>(a, a.halo + par + (need ? idx : 0), plane, 6, need, a.tag0 + (unsigned)c, v, fb);
+                if (need) {
+                    q.u1 = __uint_as_float(v[0]);
+                    q.u2 = __uint_as_float(v[1]);
+                    q.p11 = __uint_as_float(v[2]);
+                    q.p12 = __uint_as_float(v[3]);
+                    q.p21 = __uint_as_float(v[4]);
+                    q.p22 = __uint_as_float(v[5]);
+                }
+            }
+            if (threadIdx.x < 64) {
+                int r = 0;
+                if (ok && c > 1) r = decision(c - 2);
+                if (threadIdx.x == 0) sh_keep[c & 1] = r;
+                ok &= r >= 0;
+            }
+            if (!ok) sh_fail[c & 1] = 1;
+            if (c < nchunks) fb = FirstBound{0ull, 0};   // the first wait was it
+            __syncthreads();
+            if (uniform(sh_fail[c & 1])) return;
+            keep = uniform(sh_keep[c & 1]);
+            if (keep) {   // chunk c-2: in0 is its input, in1 its output
+                full = min(K, a.max_iter - (c - 2) * K);
+                break;
+            }
+            if (c == nchunks) break;
+        }
+        in0 = in1;
+        in1.get(q);
+        const int kk = min(K, a.max_iter - c * K);
+#pragma unroll
+        for (int t = 0; t < K; t++) acc[t] = 0.0;
+        sq_iterations<T, K>(a, q, kk, T, acc, sh);
+        const unsigned tag = a.tag0 + (unsigned)c + 1u;
+        if (ring && c + 1 < nchunks) {
+            unsigned long long* w = a.halo + (size_t)(c & 1) * 6 * plane + idx;
+            st_tagged(w, tag, __float_as_uint(q.u1));
+            st_tagged(w + plane, tag, __float_as_uint(q.u2));
+            st_tagged(w + 2 * plane, tag, __float_as_uint(q.p11));
+            st_tagged(w + 3 * plane, tag, __float_as_uint(q.p12));
+            st_tagged(w + 4 * plane, tag, __float_as_uint(q.p21));
+            st_tagged(w + 5 * plane, tag, __float_as_uint(q.p22));
+        }
+        const double part = block_sum<K, NW>(acc, sh_err, threadIdx.x);
+        if (threadIdx.x < (unsigned)kk) {
+            unsigned long long* w = parts + ((size_t)(c & 1) * 2 * K + 2 * threadIdx.x) * ntiles + blockIdx.x;
+            st_tagged(w, tag, (unsigned)__double2loint(part));
+            st_tagged(w + ntiles, tag, (unsigned)__double2hiint(part));
+        }
+        c++;
+    }
+    if (!keep) {   // the last chunk's decision: in1 is its input, q holds its output
+        if (threadIdx.x < 64) {
+            const int r = decision(nchunks - 1);
+            if (threadIdx.x == 0) sh_keep[(c + 1) & 1] = r;
+        }
+        __syncthreads();
+        keep = uniform(sh_keep[(c + 1) & 1]);
+        if (keep < 0) return;
+        full = a.max_iter - (nchunks - 1) * K;
+        in0 = in1;
+        in1.get(q);
+    }
+    if (keep < full) {
+        in0.put(q);
+        sq_iterations<T, K>(a, q, keep, T, acc, sh);
+    } else {
+        in1.put(q);
+    }
+    if (q.mine) sq_store_state<false>(a, q, idx, cur0 ^ 1);
+}
+
+// ---------------------------------------------------------------------------
 // one-workgroup driver
 // ---------------------------------------------------------------------------
 
@@ -1646,8 +1893,10 @@ unsigned long long next_warp_seq() { return g_warp_seq.fetch_add(1) + 1; }
 // nbr: the neighbour-synchronised kernel with K iterations per chunk, whose
 // grid is the tile workgroups plus one referee workgroup.  `resident` caches
 // the kernel's co-resident workgroups on the device (-1: not known yet).
+// tile_each: every tile needs a workgroup of its own.
 static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, unsigned gx, unsigned gy,
-                               const IterArgs& a, int nblocks, int* resident, hipStream_t s)
+                               const IterArgs& a, int nblocks, int* resident, hipStream_t s,
+                               bool tile_each = false)
 {
     static unsigned long long bound_ticks = 0;
     if (*resident < 0) {
@@ -1675,6 +1924,7 @@ static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, uns
     unsigned nb = nblocks > 0 ? (unsigned)nblocks : ntiles;
     if (nb > ntiles) nb = ntiles;
     if (nb > (unsigned)*resident - (nbr ? 1u : 0u)) nb = (unsigned)*resident - (nbr ? 1u : 0u);
+    if (tile_each && nb < ntiles) return OF_ERR_UNSUPPORTED;
     if (nbr) {
         if (!a.tile_flags || a.seq == 0 || a.seq >= kNbrMaxSeq) return OF_ERR_ARG;
         if ((long long)a.max_iter / K + 1 >= kNbrMaxChunks) return OF_ERR_UNSUPPORTED;
@@ -1715,6 +1965,18 @@ static int launch_persist_sq(const IterArgs& a, int nblocks, hipStream_t s)
                                nblocks, &resident, s);
 }
 
+// The same with tagged values; OF_ERR_UNSUPPORTED where the tiles do not all
+// have a workgroup, or without the words for them.
+template <int T, int K>
+static int launch_persist_tagged(const IterArgs& a, int nblocks, hipStream_t s)
+{
+    static int resident = -1;
+    const unsigned gx = cdiv((size_t)a.nx, (size_t)(T - 2 * K)), gy = cdiv((size_t)a.ny, (size_t)(T - 2 * K));
+    if (!a.halo || nblocks > 0) return OF_ERR_UNSUPPORTED;
+    return launch_persist_grid((const void*)k_tvl1_persist_tag<T, K>, T * T, K, true, gx, gy, a, (int)(gx * gy),
+                               &resident, s, true);
+}
+
 // The shape (4, 0) with neighbour flags: square tiles of a size chosen by the
 // scale's.  A chunk costs its iterations (one tile per CU: 0.5 us each at 16 x
 // 16, 0.74 at 24 x 24, 0.9 at 32 x 32, the chain of an iteration and its two
@@ -1732,7 +1994,8 @@ static int launch_persist_sq(const IterArgs& a, int nblocks, hipStream_t s)
 //    480x270       0.78       1.03                  0.73       0.52       0.61
 //    641x479       0.70       1.10                  0.60       0.58       0.44
 //    1024x436      0.90       1.40                  0.66       0.66       0.52
-// Scales with more 32 x 32 tiles than CUs take three iterations per chunk, whose
+// Where every tile has a CU, tagged values take another 3 to 15% off.  Scales
+// with more 32 x 32 tiles than CUs take three iterations per chunk, whose
 // registers let two tiles share a CU.  A scale that fits one workgroup needs no
 // exchange at all (30x17: 0.15 against 0.20 ms, 20x15: 0.29 against 0.33).
 static bool one_per_cu(const IterArgs& a, int centre)
@@ -1752,12 +2015,14 @@ static int launch_persist_square(const IterArgs& a, int nblocks, hipStream_t s)
         }
         return OF_OK;
     }
-    if (one_per_cu(a, 6)) return launch_persist_sq<16, 5>(a, nblocks, s);
-    if (one_per_cu(a, 14)) return launch_persist_sq<24, 5>(a, nblocks, s);
-    if (one_per_cu(a, 22)) return launch_persist_sq<32, 5>(a, nblocks, s);
+    int st = OF_ERR_UNSUPPORTED;
+    if (one_per_cu(a, 6)) st = launch_persist_tagged<16, 5>(a, nblocks, s);
+    else if (one_per_cu(a, 14)) st = launch_persist_tagged<24, 5>(a, nblocks, s);
+    else if (one_per_cu(a, 22)) st = launch_persist_tagged<32, 5>(a, nblocks, s);
+    else if (one_per_cu(a, 24)) st = launch_persist_tagged<32, 4>(a, nblocks, s);
+    if (st != OF_ERR_UNSUPPORTED) return st;
     // a flag counts the chunks of 4 iterations of any accepted limit, not those of 3
-    if (one_per_cu(a, 24) || (long long)a.max_iter / 3 + 1 >= kNbrMaxChunks)
-        return launch_persist_sq<32, 4>(a, nblocks, s);
+    if ((long long)a.max_iter / 3 + 1 >= kNbrMaxChunks) return launch_persist_sq<32, 4>(a, nblocks, s);
     return launch_persist_sq<32, 3>(a, nblocks, s);
 }
 

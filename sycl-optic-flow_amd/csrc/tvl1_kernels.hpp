@@ -84,6 +84,11 @@ struct IterArgs {
     // always compare below the current warping's
     unsigned long long* tile_flags;
     unsigned long long seq;
+    // warpings whose tiles exchange tagged values (k_tvl1_persist_tag): the
+    // words of halo_words(), zero or written by earlier warpings of the
+    // handle, whose tags lie at or below tag0 (null: not available)
+    unsigned long long* halo;
+    unsigned tag0;
 };
 
 // Launch modes of a warping (LaunchRule::persistent, of_tvl1_set_launch_rule).
@@ -104,6 +109,14 @@ void iter_grid(int K, int R, int nx, int ny, unsigned* gx, unsigned* gy);
 // iter_grid's: at most kSqOnePerCu then (a CU each, one left for the referee),
 // with up to kSqMaxIters iterations per chunk.
 constexpr int kSqOnePerCu = 255, kSqMaxIters = 5;
+// Pixels of the largest scale whose tiles have a CU each (centres of 24 x 24),
+// and the words of IterArgs::halo for frames of up to n pixels: 6 values of 2
+// parities per pixel, then 2 halves of each error partial of 2 parities.
+constexpr size_t kSqMaxPixels = (size_t)kSqOnePerCu * 24 * 24;
+constexpr size_t halo_words(size_t n)
+{
+    return 12 * (n < kSqMaxPixels ? n : kSqMaxPixels) + (size_t)4 * kSqMaxIters * kSqOnePerCu;
+}
 // Whole warping in one launch of a grid that fits the device at once;
 // `nblocks` = 0 picks the largest such grid not above the tile count.  Its
 // first grid barrier reports kBarNotResident if the grid did not fully start.
