@@ -2005,6 +2005,8 @@ static bool one_per_cu(const IterArgs& a, int centre)
 
 static int launch_persist_square(const IterArgs& a, int nblocks, hipStream_t s)
 {
+    // the limit of the shape's own 4 iterations per chunk, whichever tile it takes
+    if ((long long)a.max_iter / 4 + 1 >= kNbrMaxChunks) return OF_ERR_UNSUPPORTED;
     if (a.nx <= kSingleCols && a.ny <= kSingleCols) {
         const unsigned threads = 64 * cdiv((size_t)a.ny * kSingleCols, 64);
         hipLaunchKernelGGL(k_tvl1_single<4>, dim3(1), dim3(threads), 0, s, a);
