@@ -1,13 +1,20 @@
 // tvl1_iter.hip -- the TV-L1 primal-dual iterations (tvl1.cpp:214-292).
 //
-// Two drivers share one tile core:
-//   k_tvl1_iter<K,R>     one launch = K iterations; the last workgroup to
-//                        finish evaluates the stopping rule; the host keeps a
-//                        few launches queued (large scales);
-//   k_tvl1_persist<K,R>  one launch of a co-resident grid = a whole warping;
-//                        chunks of K iterations separated by a grid barrier, every
-//                        workgroup evaluating the stopping rule on the same
-//                        data (small, launch-latency-bound scales).
+// Drivers of the tile cores:
+//   k_tvl1_iter<K,R>         one launch = K iterations; the last workgroup to
+//                            finish evaluates the stopping rule; the host keeps
+//                            a few launches queued;
+//   k_tvl1_persist<K,R>      one launch of a co-resident grid = a whole
+//                            warping; chunks of K iterations separated by a
+//                            grid barrier, every workgroup evaluating the
+//                            stopping rule on the same data;
+//   k_tvl1_persist_nbr<K,R>  the same without grid barriers: tiles wait for
+//                            their neighbours' flags, a referee workgroup
+//                            decides;
+//   k_tvl1_persist_tag<T,K>  square tiles with a CU each, state in registers,
+//                            tagged values in place of flags;
+//   k_tvl1_single<K>         scales of at most 32 x 32 in one workgroup;
+//   k_ls_iter<K,R>           one launch = K iterations of many pairs.
 // Arithmetic follows the reference operation by operation; the library is
 // built with -ffp-contract=off.
 #include <algorithm>
