@@ -58,12 +58,9 @@ __device__ __forceinline__ f32x4 mfma32(bf16x8 a, bf16x8 b, f32x4 c)
 // fp32 -> bf16, round to nearest even (v_cvt_pk_bf16_f32 on gfx950).
 __device__ __forceinline__ bf16x8 to_bf16x8(f32x8 v) { return __builtin_convertvector(v, bf16x8); }
 
-// GEMM-k layout of the packed weights: tap t, channel c at k = t*CP + c, with
-// the channel count padded to CP (a multiple of 8, so that the 8 consecutive
-// k of one MFMA lane are channels of one tap: one 16-byte LDS read), the
-// whole padded to a multiple of 32.
-__host__ __device__ constexpr int pad_channels(int c) { return (c + 7) / 8 * 8; }
-__host__ __device__ constexpr int pad_k(int c) { return (9 * pad_channels(c) + 31) / 32 * 32; }
+// GEMM-k layout of the packed weights: tap t, channel c at k = t*C + c, zero
+// from 9*C on, the whole padded to a multiple of 32.
+__host__ __device__ constexpr int pad_k(int c) { return (9 * c + 31) / 32 * 32; }
 
 // Eight consecutive channels c8 .. c8+7 (zero past CX) of an NHWC pixel.
 template <int CX>
@@ -98,6 +95,12 @@ __device__ __forceinline__ f32x8 load_channels(const float* __restrict__ X, long
 // the first is used: with branches around the loads they had gone out one by
 // one (26.7 us; one image 9 us, now 3.8).  LDS rows are padded by 16 B so that
 // 8 lanes' 16-byte reads fall on distinct banks.
+//
+// The 8 consecutive k of an MFMA lane are channels of one tap where CX is a
+// multiple of 8: one 16-byte LDS read.  The 5- and 2-channel layers read them
+// one by one: padding a tap to 8 channels instead would group the fp32 sums
+// differently and, past 9*CX, multiply zero weights with pixels, which an
+// infinite one turns into NaN.
 template <int CX, int NT, int TR>
 __global__ __launch_bounds__(256) void k_conv_lds(const float* __restrict__ X, int B, int H, int W,
                                                   const short* __restrict__ Wp, int N,
@@ -105,7 +108,8 @@ __global__ __launch_bounds__(256) void k_conv_lds(const float* __restrict__ X, i
                                                   const float* __restrict__ mask,
                                                   float* __restrict__ Y)
 {
-    constexpr int CP = pad_channels(CX), KP = pad_k(CX), MB = TR / 4;
+    constexpr int CP = (CX + 7) / 8 * 8, KP = pad_k(CX), MB = TR / 4;
+    constexpr bool kWhole = CX % 8 == 0;   // a lane's 8 k lie in one tap
     constexpr int PW = 18, PP = PW * (TR + 2), PS = CP + 8, WS = KP + 8;
     __shared__ __align__(16) short patch[PP * PS];
     __shared__ __align__(16) short wts[NT * 16 * WS];
@@ -150,15 +154,31 @@ __global__ __launch_bounds__(256) void k_conv_lds(const float* __restrict__ X, i
 #pragma unroll
     for (int k0 = 0; k0 < KP; k0 += 32) {
         const int k = k0 + 8 * kg;
-        const int tap = CP % 32 == 0 ? k0 / CP : (k / CP < 9 ? k / CP : 8);   // past 9: zero weights
-        const int c = CP % 32 == 0 ? k0 % CP + 8 * kg : k % CP;
-        const int off = sgn * ((tap / 3 - 1) * PW + (tap % 3 - 1)) * PS + c;
+        // patch offsets of the lane's k; past the last tap a channel that pads
+        // the pixel with zero, or zeros in its place
+        int off[kWhole ? 1 : 8];
+#pragma unroll
+        for (int j = 0; j < (kWhole ? 1 : 8); j++) {
+            const int kj = k + j, tap = kj / CX, c = kj - tap * CX;
+            off[j] = sgn * ((tap / 3 - 1) * PW + (tap % 3 - 1)) * PS + c;
+            if (kj >= 9 * CX) off[j] = kWhole ? 0 : CX;
+        }
         bf16x8 w[NT];
 #pragma unroll
         for (int t = 0; t < NT; t++) w[t] = *reinterpret_cast<const bf16x8*>(wts + (t * 16 + row) * WS + k);
 #pragma unroll
         for (int m = 0; m < MB; m++) {
-            const bf16x8 a = *reinterpret_cast<const bf16x8*>(pbase + m * PW * PS + off);
+            const short* p = pbase + m * PW * PS;
+            bf16x8 a;
+            if constexpr (kWhole) {
+                a = *reinterpret_cast<const bf16x8*>(p + off[0]);
+                if (9 * CX % 32 != 0 && k >= 9 * CX) a = bf16x8{};
+            } else {
+                s16x8 v8;
+#pragma unroll
+                for (int j = 0; j < 8; j++) v8[j] = p[off[j]];
+                a = __builtin_bit_cast(bf16x8, v8);
+            }
 #pragma unroll
             for (int t = 0; t < NT; t++) acc[m][t] = mfma32(a, w[t], acc[m][t]);
         }
@@ -454,8 +474,8 @@ __global__ __launch_bounds__(256) void k_adam(float* __restrict__ w, const float
 
 // bf16 packs of one layer's weights Wm[n][t][c] (N outputs, C inputs), zero
 // in the padding:
-//   fwd [Npad][pad_k(C)]: row n, k = t*pad_channels(C) + c
-//   bwd [Cpad][pad_k(N)]: row c, k = t*pad_channels(N) + n
+//   fwd [Npad][pad_k(C)]: row n, k = t*C + c
+//   bwd [Cpad][pad_k(N)]: row c, k = t*N + n
 __global__ __launch_bounds__(256) void k_pack(const float* __restrict__ Wm, int N, int C, int Npad,
                                               int Cpad, short* __restrict__ fwd,
                                               short* __restrict__ bwd)
@@ -464,13 +484,12 @@ __global__ __launch_bounds__(256) void k_pack(const float* __restrict__ Wm, int 
     const int idx = blockIdx.x * blockDim.x + threadIdx.x;
     if (idx < Npad * Kf) {
         const int n = idx / Kf, k = idx - n * Kf;
-        const int t = k / pad_channels(C), c = k - t * pad_channels(C);
-        fwd[idx] = (n < N && t < 9 && c < C) ? to_bf16(Wm[(n * 9 + t) * C + c]) : (short)0;
+        fwd[idx] = (n < N && k < 9 * C) ? to_bf16(Wm[n * 9 * C + k]) : (short)0;
     }
     if (idx < Cpad * Kb) {
         const int c = idx / Kb, k = idx - c * Kb;
-        const int t = k / pad_channels(N), n = k - t * pad_channels(N);
-        bwd[idx] = (c < C && t < 9 && n < N) ? to_bf16(Wm[(n * 9 + t) * C + c]) : (short)0;
+        const int t = k / N, n = k - t * N;
+        bwd[idx] = (c < C && t < 9) ? to_bf16(Wm[(n * 9 + t) * C + c]) : (short)0;
     }
 }
 

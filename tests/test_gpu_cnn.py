@@ -81,6 +81,54 @@ def test_forward_matches_oracle(hidden, B, H, W):
     assert _rel(got, exact) <= 3e-2
 
 
+def test_forward_keeps_the_order_of_its_sums():
+    """Bits of one 68x120 image through the whole network, as its first
+    convolution kernel gave them: GEMM-k runs tap by tap over the layer's own
+    channels, 32 at a time.  Another grouping of a layer's fp32 sums flips
+    bfloat16 roundings of the layers behind it."""
+    import hashlib
+    torch = _torch()
+    X = np.random.default_rng(1109).normal(size=(16, 68, 120, 5)).astype(np.float32)[0]
+    from amdflow.cnn import WarmStartNet
+    with WarmStartNet(hidden=5, seed=0) as net:
+        net.set_params(NO.init_params(5, seed=7))
+        dX = torch.from_numpy(X.reshape(-1)).cuda()
+        dY = torch.empty(68 * 120 * 2, dtype=torch.float32, device="cuda")
+        net.forward(dX.data_ptr(), 1, 68, 120, dY.data_ptr())
+        torch.cuda.synchronize()
+    assert hashlib.sha256(dY.cpu().numpy().tobytes()).hexdigest() == FORWARD_SHA256
+
+
+FORWARD_SHA256 = "fe4f04a3ce601a9cbe057dda30f4f7fbf3c8779250848a9dbe60c21cb2931e32"
+
+
+@pytest.mark.parametrize("x,y", [(0, 0), (7, 5), (16, 8), (39, 19)])
+def test_forward_infinite_input_stays_in_its_window(x, y):
+    """With positive weights an infinite input makes every output whose 5x5
+    window (two layers) holds it infinite, and no other: a GEMM entry past
+    the last tap must not bring it in (0 * inf is NaN, which the ReLU turns
+    into 0)."""
+    torch = _torch()
+    H, W = 20, 40
+    rng = np.random.default_rng(5)
+    X = rng.random((1, H, W, 5)).astype(np.float32)
+    X[0, y, x, 0] = np.inf
+    net, p = _net(0)
+    p = (np.abs(p) + 0.01).astype(np.float32)
+    net.set_params(p)
+    dX = torch.from_numpy(X.reshape(-1)).cuda()
+    dY = torch.empty(H * W * 2, dtype=torch.float32, device="cuda")
+    net.forward(dX.data_ptr(), 1, H, W, dY.data_ptr())
+    torch.cuda.synchronize()
+    got = dY.cpu().numpy().reshape(1, H, W, 2)
+    emu = NO.forward(p, X, 0, bf16=True)[-1]
+    inf = np.isinf(emu)
+    assert inf.sum() == 2 * (min(x + 3, W) - max(x - 2, 0)) * (min(y + 3, H) - max(y - 2, 0))
+    assert np.array_equal(got[inf], emu[inf])
+    assert np.isfinite(got[~inf]).all()
+    assert _rel(got[~inf], emu[~inf]) <= 2e-3
+
+
 @pytest.mark.parametrize("hidden,B,H,W", [(0, 1, 6, 5), (1, 2, 9, 13), (5, 2, 20, 17)])
 def test_gradients_match_oracle(hidden, B, H, W):
     torch = _torch()
