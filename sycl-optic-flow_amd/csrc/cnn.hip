@@ -235,6 +235,10 @@ __global__ __launch_bounds__(256) void k_conv_lds(const float* __restrict__ X, i
 // an MFMA operand holds; X^T three times, shifted by the taps' dx, so that
 // every tap reads aligned.  part: [blocks][NT*16][Kpad] with k = t*CX + c.
 // The bias gradient is the fp32 sum of dY, taken on the way to LDS.
+// Positions of a tile outside the image have dY = 0 and X = 0: a pixel inside
+// that such a position's taps would reach must not count even where it is
+// infinite (0 * inf is NaN), so the operand that such a position multiplies is
+// zero by the position of dY, not of X.
 //
 // Bound by reading dY and X once (fp32; 67 MB per 32->32 layer at 32 x 68 x
 // 120 pixels).  The earlier kernel formed one 16x16
@@ -258,13 +262,16 @@ __global__ __launch_bounds__(256) void k_wgrad(const float* __restrict__ dY,
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int row = lane & 15, kg = lane >> 4;
     const int tiles_x = (W + 7) / 8, tiles_y = (H + T - 1) / T;
-    // LDS offset of this lane's column of each of the wave's column tiles
-    int xoff[CW];
+    // LDS offset of this lane's column of each of the wave's column tiles, and
+    // that for the first row past the image, whose upper taps reach the last
+    // row inside: they read the row of zeros after it
+    int xoff[CW], xbelow[CW];
 #pragma unroll
     for (int i = 0; i < CW; i++) {
         const int k = min((wave + 4 * i) * 16 + row, 9 * CX - 1);   // past the end: computed, not read back
         const int t = k / CX, c = k - t * CX;
         xoff[i] = ((t % 3) * CX + c) * XR * 8 + (t / 3) * 8;
+        xbelow[i] = xoff[i] + (t / 3 == 0 ? 8 : 0);
     }
     f32x4 acc[CW][NT];
 #pragma unroll
@@ -328,6 +335,11 @@ __global__ __launch_bounds__(256) void k_wgrad(const float* __restrict__ dY,
                     f32x8 v;
 #pragma unroll
                     for (int j = 0; j < 8; j++) v[j] = xv[i][d + j];
+                    if (xedge) {
+#pragma unroll
+                        for (int j = 0; j < 8; j++)
+                            if (x0 + j >= W) v[j] = 0.0f;
+                    }
                     *reinterpret_cast<bf16x8*>(&xs[d][c][pr][0]) = xin[i] ? to_bf16x8(v) : bf16x8{};
                 }
             }
@@ -349,13 +361,15 @@ __global__ __launch_bounds__(256) void k_wgrad(const float* __restrict__ dY,
 #pragma unroll
         for (int ks = 0; ks < T / 4; ks++) {   // 32 pixels: 4 rows of 8
             const int pr = ks * 4 + kg;
+            const bool below = pr == H - y0;   // the first row past the image
             bf16x8 a[NT];
 #pragma unroll
             for (int t = 0; t < NT; t++) a[t] = *reinterpret_cast<const bf16x8*>(&ys[t * 16 + row][pr][0]);
 #pragma unroll
             for (int i = 0; i < CW; i++) {
                 if (wave + 4 * i >= COLS) break;   // wave-uniform
-                const bf16x8 x = *reinterpret_cast<const bf16x8*>(&xs[0][0][0][0] + xoff[i] + pr * 8);
+                const int off = below ? xbelow[i] : xoff[i];
+                const bf16x8 x = *reinterpret_cast<const bf16x8*>(&xs[0][0][0][0] + off + pr * 8);
 #pragma unroll
                 for (int t = 0; t < NT; t++) acc[i][t] = mfma32(a[t], x, acc[i][t]);
             }

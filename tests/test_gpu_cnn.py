@@ -153,6 +153,32 @@ def test_gradients_match_oracle(hidden, B, H, W):
     assert _rel(g, g_ex) <= 5e-2
 
 
+@pytest.mark.parametrize("H,W,y,x", [(17, 9, 16, 8), (19, 21, 18, 3), (20, 12, 7, 11), (16, 8, 15, 7),
+                                     (21, 10, 20, 9), (30, 24, 29, 23)])
+def test_gradients_infinite_input_counts_inside_the_image_only(H, W, y, x):
+    """An infinite input at the image's last row or column, behind weights
+    that make its features -inf and so 0: the loss stays finite, and the weight
+    gradient holds 0 * inf only for the taps through which a pixel of the image
+    sees it, not for those of tile positions outside the image."""
+    torch = _torch()
+    rng = np.random.default_rng(H + W)
+    X = rng.normal(size=(1, H, W, 5)).astype(np.float32)
+    X[0, y, x, 0] = np.inf
+    T = rng.normal(size=(1, 2, H, W)).astype(np.float32)
+    net, p = _net(0)
+    p[0:32 * 45:5] = -np.abs(p[0:32 * 45:5]) - 0.01   # input channel 0 of the first layer
+    net.set_params(p)
+    dX, dT = torch.from_numpy(X.reshape(-1)).cuda(), torch.from_numpy(T.reshape(-1)).cuda()
+    loss, g = net.gradients(dX.data_ptr(), dT.data_ptr(), 1, H, W)
+    with np.errstate(invalid="ignore"):
+        l_emu, g_emu = NO.loss_and_grads(p, X, T, 0, bf16=True)
+    assert np.isfinite(l_emu) and abs(loss - l_emu) <= 1e-4 * l_emu
+    nan = np.isnan(g_emu)
+    assert 0 < nan.sum() < 32 * 9 and nan[:32 * 45:5].sum() == nan.sum()
+    assert np.array_equal(np.isnan(g), nan)
+    assert _rel(g[~nan], g_emu[~nan]) <= 5e-3
+
+
 @pytest.mark.parametrize("B,H,W", [(1, 1, 1), (1, 3, 17), (2, 16, 8), (1, 17, 9), (3, 33, 31), (1, 2, 130),
                                    (64, 9, 50)])
 def test_tile_edges_match_oracle(B, H, W):
