@@ -77,6 +77,10 @@ int of_dbg_cnn_mfma(const float *A, const float *B, float *D);
  * workgroup arrives, then all end), so the solve takes its host-paced
  * repeat; a test of that path. */
 int of_dbg_persist_force_not_resident(int on);
+/* While `on` is nonzero, the pyramidal Lucas-Kanade runs its iterations on
+ * frames of any size with the kernels of those too large for the blocked one
+ * (a side of 2^24 or more than 2^30 pixels); a test of that path. */
+int of_dbg_lk_force_unblocked(int on);
 /* Allocation failure injection: after this call the first `n` device or
  * pinned host allocations of the library succeed and every later one fails
  * with OF_ERR_ALLOC, as a real failure would (n < 0: none fails).  The call

@@ -20,6 +20,7 @@ _SIGS = {
                                            C.c_int, C.c_int, C.c_int, _vp],
     "of_dbg_hypot": [_vp, _vp, _vp, C.c_size_t],
     "of_dbg_persist_force_not_resident": [C.c_int],
+    "of_dbg_lk_force_unblocked": [C.c_int],
     "of_dbg_fail_alloc_after": [C.c_longlong],
 }
 for _n, _a in _SIGS.items():
@@ -178,6 +179,12 @@ def persist_force_not_resident(on: bool) -> None:
     """While on, launches of the persistent warping kernel report that their
     grid was not co-resident, so solves take their host-paced repeat."""
     _check(_lib.of_dbg_persist_force_not_resident(1 if on else 0), "dbg_persist_force_not_resident")
+
+
+def lk_force_unblocked(on: bool) -> None:
+    """Pyramidal LK takes the iterations of frames beyond the blocked kernel's
+    limits at any size while on (test aid)."""
+    _check(_lib.of_dbg_lk_force_unblocked(1 if on else 0), "dbg_lk_force_unblocked")
 
 
 _lib.of_dbg_alloc_attempts.restype = C.c_longlong

@@ -14,6 +14,7 @@
 // u -= G^-1 b where det G > det_eps), flow carried up with zoom_in x 1/zf.
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdint>
 #include <cstring>
 #include <mutex>
@@ -765,6 +766,10 @@ LkBufs lk_carve(float* base, const LkPlan& P)
     return B;
 }
 
+// Test hook: frames of any size take the iterations of those beyond the
+// blocked kernel's limits.
+static std::atomic<int> g_unblocked{0};
+
 // The solve proper: pyramid, then coarse to fine the structure tensor and
 // `iters` iterations per level, zoom_in between levels.  Every buffer of B
 // is written before it is read (u, v are cleared at the coarsest level), so
@@ -833,7 +838,7 @@ int lk_pyr_run(const LkPlan& P, const LkBufs& B, const float* dI0, const float* 
     // the blocked iterations index planes with 32-bit byte offsets and
     // 24-bit row products; level 0 is the largest level
     const bool blocked = wc >= 1 && wc <= 4 && nx[0] < (1 << 24) && ny[0] < (1 << 24) &&
-                         n0 <= ((size_t)1 << 30);
+                         n0 <= ((size_t)1 << 30) && !g_unblocked.load(std::memory_order_relaxed);
     const bool direct = blocked && iters >= 1 && !overlaps(du, dv, n0) &&
                         !overlaps(du, dI0, n0) && !overlaps(du, dI1, n0) &&
                         !overlaps(dv, dI0, n0) && !overlaps(dv, dI1, n0);
@@ -867,9 +872,10 @@ int lk_pyr_run(const LkPlan& P, const LkBufs& B, const float* dI0, const float* 
     };
     // The coarser levels' tensors take the blur buffers, free by now, where
     // five planes of every level fit one (at a zoom factor of 1/2: 5/3 of the
-    // 3 planes); otherwise each level's are formed when it is its turn.
+    // 3 planes); otherwise each level's are formed when it is its turn, as
+    // also for the unblocked iterations, which need those buffers themselves.
     const bool fused = wc >= 1 && wc <= 4;
-    const bool together = fused && 5 * P.pyr <= 3 * n0;
+    const bool together = blocked && 5 * P.pyr <= 3 * n0;
     auto level_planes = [&](int l, float** ix, float** iy, float** gt) {
         const bool own = l > 0 && together;
         const size_t m = (size_t)nx[l] * ny[l];
@@ -888,13 +894,13 @@ int lk_pyr_run(const LkPlan& P, const LkBufs& B, const float* dI0, const float* 
         if (fused) {
             if (!together) OF_TRY(tensors(l, l, level_planes));
         } else {
-            hipLaunchKernelGGL(k_lk_tensor_products, grid2d(w, h), dim3(256), 0, st, p0, w, h, Ix,
-                               Iy, PROD);
+            hipLaunchKernelGGL(k_lk_tensor_products, grid2d(w, h), dim3(256), 0, st, p0, w, h, lix,
+                               liy, PROD);
             LK_CHECK("k_lk_tensor_products");
             hipLaunchKernelGGL(k_lk_boxsum, grid2d(w, h), dim3(256), 0, st, PROD, ROWS, w, h, 3, wc,
                                0);
             LK_CHECK("k_lk_boxsum");
-            hipLaunchKernelGGL(k_lk_boxsum, grid2d(w, h), dim3(256), 0, st, ROWS, GT, w, h, 3, wc,
+            hipLaunchKernelGGL(k_lk_boxsum, grid2d(w, h), dim3(256), 0, st, ROWS, lgt, w, h, 3, wc,
                                1);
             LK_CHECK("k_lk_boxsum");
         }
@@ -923,12 +929,12 @@ int lk_pyr_run(const LkPlan& P, const LkBufs& B, const float* dI0, const float* 
             it += kk;
         }
         for (int it = 0; it < iters && !blocked; it++) {
-            hipLaunchKernelGGL(k_lk_it_products, grid2d(w, h), dim3(256), 0, st, p0, p1, Ix, Iy,
+            hipLaunchKernelGGL(k_lk_it_products, grid2d(w, h), dim3(256), 0, st, p0, p1, lix, liy,
                                u, v, w, h, PROD);
             LK_CHECK("k_lk_it_products");
             hipLaunchKernelGGL(k_lk_boxsum, grid2d(w, h), dim3(256), 0, st, PROD, ROWS, w, h, 2, wc, 0);
             LK_CHECK("k_lk_boxsum");
-            hipLaunchKernelGGL(k_lk_update, grid2d(w, h), dim3(256), 0, st, ROWS, GT, w, h, wc,
+            hipLaunchKernelGGL(k_lk_update, grid2d(w, h), dim3(256), 0, st, ROWS, lgt, w, h, wc,
                                det_eps, u, v);
             LK_CHECK("k_lk_update");
         }
@@ -1195,6 +1201,12 @@ int of_lk_pyr_compute_device_noalloc(const float* dI0, const float* dI1, int wid
         (void)hipGetLastError();
     }
     return status;
+}
+
+int of_dbg_lk_force_unblocked(int on)
+{
+    g_unblocked.store(on != 0);
+    return OF_OK;
 }
 
 int of_lk_pyr_compute(const float* I0, const float* I1, int width, int height, int levels, float zf,

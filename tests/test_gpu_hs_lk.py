@@ -182,6 +182,26 @@ def test_lk_pyramidal_shapes_by_size_match_oracle(w, h, win, iters, levels, zf):
     assert np.array_equal(u, ou) and np.array_equal(v, ov)
 
 
+@pytest.fixture
+def unblocked():
+    D.lk_force_unblocked(True)
+    yield
+    D.lk_force_unblocked(False)
+
+
+@pytest.mark.parametrize("w,h,win,iters,levels,zf", [(64, 48, 3, 3, 1, 0.5), (161, 121, 5, 3, 2, 0.5),
+                                                     (333, 251, 9, 4, 3, 0.5), (105, 165, 7, 2, 2, 0.8),
+                                                     (120, 90, 11, 3, 2, 0.5), (120, 90, 1, 3, 2, 0.5)])
+def test_lk_pyramidal_unblocked_matches_oracle(w, h, win, iters, levels, zf, unblocked):
+    """Frames beyond the blocked kernel's limits (a side of 2^24, more than 2^30
+    pixels) iterate with one launch per step: here at small sizes, windows of
+    the fused tensor (3 to 9) and others."""
+    I0, I1, _, _ = synth.make_pair(w, h, 3.0, 57 + w + win)
+    u, v = lk_pyramidal(I0, I1, levels=levels, zf=zf, sigma=1.0, window=win, iters=iters, det_eps=1e-6)
+    ou, ov = O.lk_pyr(I0, I1, levels=levels, zf=zf, sigma=1.0, win=win, iters=iters, det_eps=1e-6)
+    assert np.array_equal(u, ou) and np.array_equal(v, ov)
+
+
 @pytest.mark.parametrize("bad", [np.nan, np.inf, 3e38])
 def test_lk_pyramidal_non_finite_frames_match_oracle(bad):
     """A frame value that makes flows non-finite or huge: such waves take the
