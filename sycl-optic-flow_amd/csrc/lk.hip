@@ -14,6 +14,7 @@
 // u -= G^-1 b where det G > det_eps), flow carried up with zoom_in x 1/zf.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cstdint>
 #include <cstring>
@@ -195,9 +196,13 @@ constexpr int kLkCUs = 256;
 // columns (windows clipped to the image, ascending order).  The tensors do not
 // depend on the flow, so one launch takes all levels: the coarse ones, too
 // small to fill the device, run beside the finest instead of before it, and
-// their launches go.
+// their launches go.  Blocks are numbered along x and then y: a frame of few
+// columns and 2^27 rows has more of them than one dimension of a grid takes
+// (below 2^32 threads).
+constexpr unsigned kLkTensorGridX = 1u << 20;
 struct LkTensorLevels {
     int n;
+    int blocks;                // of all levels
     int first[kLkMaxLevels];   // first block of each level
     int w[kLkMaxLevels], h[kLkMaxLevels];
     const float* p0[kLkMaxLevels];
@@ -207,14 +212,16 @@ struct LkTensorLevels {
 template <int WC, int TH = kLkTileRows>
 __global__ __launch_bounds__(256) void k_lk_tensor_fused(LkTensorLevels L)
 {
+    const int block = (int)(blockIdx.y * kLkTensorGridX + blockIdx.x);
+    if (block >= L.blocks) return;
     int l = 0;
-    while (l + 1 < L.n && (int)blockIdx.x >= L.first[l + 1]) l++;
+    while (l + 1 < L.n && block >= L.first[l + 1]) l++;
     const float* __restrict__ P0 = L.p0[l];
     float* __restrict__ Ix = L.Ix[l];
     float* __restrict__ Iy = L.Iy[l];
     float* __restrict__ G = L.G[l];
     const int w = L.w[l], h = L.h[l];
-    const int tiles_x = (w + 63) / 64, tile = (int)blockIdx.x - L.first[l];
+    const int tiles_x = (w + 63) / 64, tile = block - L.first[l];
     const int bx = tile % tiles_x, by = tile / tiles_x;
     constexpr int TW = 64, EW = TW + 2 * WC, EH = TH + 2 * WC;
     constexpr int NE = (EW * EH + 255) / 256;
@@ -862,7 +869,8 @@ int lk_pyr_run(const LkPlan& P, const LkBufs& B, const float* dI0, const float* 
             planes(l, &T.Ix[i], &T.Iy[i], &T.G[i]);
             blocks += (size_t)cdiv(nx[l], 64) * cdiv(ny[l], kLkTileRows);
         }
-        const dim3 tgrid((unsigned)blocks);
+        T.blocks = (int)blocks;
+        const dim3 tgrid((unsigned)std::min(blocks, (size_t)kLkTensorGridX), cdiv(blocks, kLkTensorGridX));
         if (wc == 1) hipLaunchKernelGGL((k_lk_tensor_fused<1>), tgrid, dim3(256), 0, st, T);
         if (wc == 2) hipLaunchKernelGGL((k_lk_tensor_fused<2>), tgrid, dim3(256), 0, st, T);
         if (wc == 3) hipLaunchKernelGGL((k_lk_tensor_fused<3>), tgrid, dim3(256), 0, st, T);

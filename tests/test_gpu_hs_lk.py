@@ -202,6 +202,26 @@ def test_lk_pyramidal_unblocked_matches_oracle(w, h, win, iters, levels, zf, unb
     assert np.array_equal(u, ou) and np.array_equal(v, ov)
 
 
+def test_lk_pyramidal_many_rows_of_two_columns():
+    """2^27 rows make 2^24 tensor tiles, more than one grid dimension takes.
+    The flow of the first rows does not see the others: it has the bits of a
+    frame that ends earlier."""
+    import torch
+    from amdflow.lk import lk_pyramidal_device
+    H, N, K = 1 << 27, 4096, 1024
+    y = np.arange(N, dtype=np.float32)[:, None] + np.float32([0.0, 0.3])
+    I0 = (127 + 90 * np.sin(0.4 * y)).astype(np.float32)
+    I1 = (127 + 90 * np.sin(0.4 * (y - 0.7))).astype(np.float32)
+    d0, d1 = (torch.from_numpy(a).cuda().reshape(-1).repeat(H // N) for a in (I0, I1))
+    u, v = (torch.full((2 * H,), np.nan, dtype=torch.float32, device="cuda") for _ in range(2))
+    lk_pyramidal_device(d0.data_ptr(), d1.data_ptr(), 2, H, u.data_ptr(), v.data_ptr(), levels=1, zf=0.5,
+                        sigma=1.0, window=3, iters=1, det_eps=1e-6)
+    ou, ov = O.lk_pyr(I0, I1, levels=1, zf=0.5, sigma=1.0, win=3, iters=1, det_eps=1e-6)
+    for got, want in ((u, ou), (v, ov)):
+        assert np.array_equal(got[:2 * K].cpu().numpy().reshape(K, 2), want[:K])
+        assert bool(torch.isfinite(got).all())
+
+
 @pytest.mark.parametrize("bad", [np.nan, np.inf, 3e38])
 def test_lk_pyramidal_non_finite_frames_match_oracle(bad):
     """A frame value that makes flows non-finite or huge: such waves take the
