@@ -916,19 +916,24 @@ int orc_hs_compute(const float *I0, const float *I1, int width, int height, int 
         orc_hs_downscale(pI1[L], pW[L], pH[L], pS[L], pI1[L - 1], nw, nh, ns);
         pW[L - 1] = nw; pH[L - 1] = nh; pS[L - 1] = ns;
     }
-    float *du0 = (float *)calloc(fsize, sizeof(float)), *dv0 = (float *)calloc(fsize, sizeof(float));
-    float *du1 = (float *)calloc(fsize, sizeof(float)), *dv1 = (float *)calloc(fsize, sizeof(float));
-    float *Ix = (float *)calloc(fsize, sizeof(float)), *Iy = (float *)calloc(fsize, sizeof(float));
-    float *Iz = (float *)calloc(fsize, sizeof(float)), *tmp = (float *)calloc(fsize, sizeof(float));
-    float *cu = (float *)calloc(fsize, sizeof(float)), *cv = (float *)calloc(fsize, sizeof(float));
-    float *nu = (float *)calloc(fsize, sizeof(float)), *nv = (float *)calloc(fsize, sizeof(float));
+    /* the shared planes hold the largest level: coarse pitches are whole 32
+     * columns, more than a narrow frame's own */
+    size_t plane = 0;
+    for (L = 0; L < nLevels; ++L)
+        if ((size_t)pS[L] * pH[L] > plane) plane = (size_t)pS[L] * pH[L];
+    float *du0 = (float *)calloc(plane, sizeof(float)), *dv0 = (float *)calloc(plane, sizeof(float));
+    float *du1 = (float *)calloc(plane, sizeof(float)), *dv1 = (float *)calloc(plane, sizeof(float));
+    float *Ix = (float *)calloc(plane, sizeof(float)), *Iy = (float *)calloc(plane, sizeof(float));
+    float *Iz = (float *)calloc(plane, sizeof(float)), *tmp = (float *)calloc(plane, sizeof(float));
+    float *cu = (float *)calloc(plane, sizeof(float)), *cv = (float *)calloc(plane, sizeof(float));
+    float *nu = (float *)calloc(plane, sizeof(float)), *nv = (float *)calloc(plane, sizeof(float));
     for (L = 0; L < nLevels; ++L) {
         const int w = pW[L], h = pH[L], s = pS[L];
         for (int wi = 0; wi < nWarpIters; ++wi) {
-            memset(du0, 0, sizeof(float) * fsize);
-            memset(dv0, 0, sizeof(float) * fsize);
-            memset(du1, 0, sizeof(float) * fsize);
-            memset(dv1, 0, sizeof(float) * fsize);
+            memset(du0, 0, sizeof(float) * plane);
+            memset(dv0, 0, sizeof(float) * plane);
+            memset(du1, 0, sizeof(float) * plane);
+            memset(dv1, 0, sizeof(float) * plane);
             orc_hs_warp(pI1[L], w, h, s, cu, cv, tmp);
             orc_hs_derivatives(pI0[L], tmp, w, h, s, Ix, Iy, Iz);
             for (int it = 0; it < nSolverIters; ++it) {

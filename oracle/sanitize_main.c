@@ -168,6 +168,7 @@ int main(void)
     tvl1_case(80, 60, 4, 1);
     tvl1_case(80, 60, 4, 2);
     hs_lk_case(72, 40, 1);
+    hs_lk_case(8, 300, 0);    /* coarse HS planes larger than the finest one */
     orc_set_error_mode(ORC_ERROR_FLOAT_SEQUENTIAL);
     tvl1_case(48, 40, 2, 0);
     orc_set_error_mode(ORC_ERROR_DOUBLE_ROWS);
