@@ -290,17 +290,18 @@ __global__ __launch_bounds__(64 * NW) void k_hs_jacobi(JacobiArgs a)
     else jacobi_tile<R, NW, true>(a, sh);
 }
 
-// Frames in and flow cleared, or flow out: two planes copied (a1 may be
-// null: that pair is not copied) and two cleared, in one launch.
+// Frames in and flow cleared, or flow out: two planes of n floats copied and
+// two of nz cleared, in one launch.
 __global__ __launch_bounds__(256) void k_hs_copy2(const float* a0, float* a1, const float* b0, float* b1,
-                                                  float* z0, float* z1, size_t n)
+                                                  size_t n, float* z0, float* z1, size_t nz)
 {
-    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n;
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n || i < nz;
          i += (size_t)gridDim.x * blockDim.x) {
-        if (a1) a1[i] = a0[i];
-        if (b1) b1[i] = b0[i];
-        if (z0) z0[i] = 0.0f;
-        if (z1) z1[i] = 0.0f;
+        if (i < n) {
+            a1[i] = a0[i];
+            b1[i] = b0[i];
+        }
+        if (i < nz) z0[i] = z1[i] = 0.0f;
     }
 }
 
@@ -387,6 +388,7 @@ struct of_hs {
     float** pI0 = nullptr;
     float** pI1 = nullptr;
     int pW[32]{}, pH[32]{}, pS[32]{};
+    size_t plane = 0;   // floats of the largest level's plane: of each buffer from u to Iz
     float *u = nullptr, *v = nullptr, *nu = nullptr, *nv = nullptr;
     float *du[2]{}, *dv[2]{};
     float *Ix = nullptr, *Iy = nullptr, *Iz = nullptr;
@@ -452,9 +454,11 @@ int hs_solve(of_hs* h, const float* dI0, const float* dI1, int width, int height
     if (nWarpIters < 0 || nSolverIters < 0) return OF_ERR_ARG;
     const size_t fsize = (size_t)stride * height;
     int L = nLevels - 1;
-    const unsigned blocks = cdiv(fsize, 256) > 2048 ? 2048 : cdiv(fsize, 256);
-    hipLaunchKernelGGL(k_hs_copy2, dim3(blocks), dim3(256), 0, st, dI0, h->pI0[L], dI1, h->pI1[L], h->u,
-                       h->v, fsize);
+    const unsigned blocks = std::min(cdiv(fsize, 256), 2048u);
+    // the initial flow is read at the coarsest level, the padding columns of
+    // the result are those of the finest
+    hipLaunchKernelGGL(k_hs_copy2, dim3(blocks), dim3(256), 0, st, dI0, h->pI0[L], dI1, h->pI1[L], fsize,
+                       h->u, h->v, std::max(fsize, (size_t)h->pS[0] * h->pH[0]));
     HS_CHECK("k_hs_copy2");
     for (; L > 0; --L) {
         hipLaunchKernelGGL(k_hs_downscale, grid2d(h->pW[L - 1], h->pH[L - 1]), dim3(256), 0, st,
@@ -498,8 +502,8 @@ int hs_solve(of_hs* h, const float* dI0, const float* dI1, int width, int height
     }
     // the result is in h->u/h->v, which the level loop swaps with nu/nv
     if (du_out && dv_out) {
-        hipLaunchKernelGGL(k_hs_copy2, dim3(blocks), dim3(256), 0, st, h->u, du_out, h->v, dv_out,
-                           (float*)nullptr, (float*)nullptr, fsize);
+        hipLaunchKernelGGL(k_hs_copy2, dim3(blocks), dim3(256), 0, st, h->u, du_out, h->v, dv_out, fsize,
+                           (float*)nullptr, (float*)nullptr, (size_t)0);
         HS_CHECK("k_hs_copy2");
     }
     OF_HIP(hipStreamSynchronize(st));
@@ -539,6 +543,9 @@ int of_hs_create(int nLevels, int stride, int width, int height, of_hs** out)
     h->pI1 = new (std::nothrow) float*[nLevels]();
     if (!h->pI0 || !h->pI1) { hs_release(h); return OF_ERR_ALLOC; }
     const size_t fsize = (size_t)stride * height;
+    // coarse levels have pitches of whole 32 columns: on frames narrower than
+    // 16 columns their planes are larger than the finest one's
+    for (int L = 0; L < nLevels; L++) h->plane = std::max(h->plane, (size_t)h->pS[L] * h->pH[L]);
     int st = OF_OK;
     for (int L = 0; L < nLevels && !st; L++) {
         const size_t n = (size_t)h->pS[L] * h->pH[L];
@@ -546,13 +553,18 @@ int of_hs_create(int nLevels, int stride, int width, int height, of_hs** out)
         if (!st) st = dev_alloc(&h->pI1[L], n);
     }
     float** bufs[] = {&h->u, &h->v, &h->nu, &h->nv, &h->du[0], &h->du[1], &h->dv[0], &h->dv[1],
-                      &h->Ix, &h->Iy, &h->Iz, &h->hin0, &h->hin1};
+                      &h->Ix, &h->Iy, &h->Iz};
+    float** staging[] = {&h->hin0, &h->hin1};
     for (float** b : bufs)
+        if (!st) st = dev_alloc(b, h->plane);
+    for (float** b : staging)
         if (!st) st = dev_alloc(b, fsize);
     if (st) { hs_release(h); return st; }
     // padding columns of strided buffers are never read by the kernels;
     // clear everything once so downloads are deterministic
     for (float** b : bufs)
+        if (hipMemsetAsync(*b, 0, h->plane * sizeof(float), h->stream) != hipSuccess) st = OF_ERR_HIP;
+    for (float** b : staging)
         if (hipMemsetAsync(*b, 0, fsize * sizeof(float), h->stream) != hipSuccess) st = OF_ERR_HIP;
     for (int L = 0; L < nLevels; L++) {
         const size_t n = (size_t)h->pS[L] * h->pH[L];

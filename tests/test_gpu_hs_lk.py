@@ -110,6 +110,23 @@ def test_hs_shape_by_size_matches_oracle(w, h, sweeps):
     assert np.array_equal(u, ou) and np.array_equal(v, ov)
 
 
+@pytest.mark.parametrize("w,stride,h,levels", [(8, 8, 4096, 2), (12, 12, 2000, 2), (8, 15, 1000, 3),
+                                               (15, 16, 700, 3), (31, 33, 400, 4)])
+def test_hs_narrow_levels_match_oracle(w, stride, h, levels):
+    """Coarse levels have pitches of whole 32 columns: on narrow frames their
+    planes are larger than the finest level's, and so are the buffers that all
+    levels share.  Two calls, as the second finds the first one's values."""
+    rng = np.random.default_rng(w + h)
+    I0 = (rng.random((h, stride)) * 255).astype(np.float32)
+    I1 = (rng.random((h, stride)) * 255).astype(np.float32)
+    ou, ov = O.hs_compute(np.ascontiguousarray(I0[:, :w]), np.ascontiguousarray(I1[:, :w]), alpha=15.0,
+                          nLevels=levels, nWarpIters=2, nSolverIters=9)
+    with HornSchunck(levels, stride, w, h) as hs:
+        for _ in range(2):
+            u, v = hs.ComputeFlow(I0, I1, w, h, stride, 15.0, levels, 2, 9)
+            assert np.array_equal(u[:, :w], ou) and np.array_equal(v[:, :w], ov)
+
+
 @pytest.mark.parametrize("scale", [1e-37, 1e-41, 3e-45])
 def test_hs_jacobi_subnormal_increments_bitexact(scale):
     """Quotients that land on and between subnormal floats (a diffusion front
