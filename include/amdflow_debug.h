@@ -77,6 +77,11 @@ int of_dbg_cnn_mfma(const float *A, const float *B, float *D);
  * workgroup arrives, then all end), so the solve takes its host-paced
  * repeat; a test of that path. */
 int of_dbg_persist_force_not_resident(int on);
+/* While `on` is nonzero, the referee workgroup of neighbour-synchronised
+ * warpings ends at once, as if it had not started: every tile's wait for its
+ * first decision ends at the residency bound, and the solve takes its
+ * host-paced repeat. */
+int of_dbg_persist_referee_absent(int on);
 /* While `on` is nonzero, the pyramidal Lucas-Kanade runs its iterations on
  * frames of any size with the kernels of those too large for the blocked one
  * (a side of 2^24 or more than 2^30 pixels); a test of that path. */

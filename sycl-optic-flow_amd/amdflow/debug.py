@@ -20,6 +20,7 @@ _SIGS = {
                                            C.c_int, C.c_int, C.c_int, _vp],
     "of_dbg_hypot": [_vp, _vp, _vp, C.c_size_t],
     "of_dbg_persist_force_not_resident": [C.c_int],
+    "of_dbg_persist_referee_absent": [C.c_int],
     "of_dbg_lk_force_unblocked": [C.c_int],
     "of_dbg_fail_alloc_after": [C.c_longlong],
 }
@@ -179,6 +180,12 @@ def persist_force_not_resident(on: bool) -> None:
     """While on, launches of the persistent warping kernel report that their
     grid was not co-resident, so solves take their host-paced repeat."""
     _check(_lib.of_dbg_persist_force_not_resident(1 if on else 0), "dbg_persist_force_not_resident")
+
+
+def persist_referee_absent(on: bool) -> None:
+    """While on, the referee workgroup of neighbour-synchronised warpings ends
+    at once, so solves take their host-paced repeat."""
+    _check(_lib.of_dbg_persist_referee_absent(1 if on else 0), "dbg_persist_referee_absent")
 
 
 def lk_force_unblocked(on: bool) -> None:

@@ -258,6 +258,12 @@ int of_dbg_persist_force_not_resident(int on)
     return OF_OK;
 }
 
+int of_dbg_persist_referee_absent(int on)
+{
+    set_persist_referee_absent(on != 0);
+    return OF_OK;
+}
+
 int of_dbg_hypot(const float* a, const float* b, float* out, size_t n)
 {
     if (!a || !b || !out) return OF_ERR_ARG;

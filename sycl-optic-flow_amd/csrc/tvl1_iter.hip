@@ -1049,7 +1049,9 @@ __device__ __forceinline__ int wave_wait(const IterArgs& a, const unsigned long 
 // stop_keep iterations of chunk stop_chunk.  Members are uniform.
 struct NbrSync {
     const IterArgs& a;
-    FirstBound fb;   // the first wait of a plain launch also checks that the grid is resident
+    // a plain launch also checks that the grid is resident: the first wait for
+    // the neighbours, and the first for a decision, which the referee makes
+    FirstBound fb, fb_referee;
     int* sh;         // LDS word for results of wave 0
     unsigned tiles_x, tiles_y, tile;
     int c;           // chunk of the current tile
@@ -1065,13 +1067,14 @@ struct NbrSync {
         __syncthreads();
         if (threadIdx.x == 0) *sh = r;
         __syncthreads();
-        fb = FirstBound{0ull, 0};
         return uniform(*sh);
     }
 
     __device__ __forceinline__ int wait(const unsigned long long* w, unsigned long long want)
     {
-        return share(threadIdx.x < 64 ? wave_wait(a, w, want, fb) : 0);
+        const int r = share(threadIdx.x < 64 ? wave_wait(a, w, want, fb) : 0);
+        fb = FirstBound{0ull, 0};
+        return r;
     }
 
     // Decision of chunk q once published: keep, or -1 if the wait failed.
@@ -1081,9 +1084,10 @@ struct NbrSync {
         if (threadIdx.x < 64) {
             const unsigned long long* w = &a.ctl->decision[q & 1].v;
             const unsigned long long want = (a.seq << 24) | ((unsigned long long)(q + 1) << 4);
-            if (wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, fb))
+            if (wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, fb_referee))
                 r = (int)(__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFull);
         }
+        fb_referee = FirstBound{0ull, 0};
         return share(r);
     }
 
@@ -1186,6 +1190,7 @@ __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist_nbr(IterArgs a, unsigned ti
     const int nchunks = (a.max_iter + K - 1) / K;
 
     if (blockIdx.x == nbw) {   // referee
+        if (a.referee_absent) return;
         int n = 0, c = 0;
         while (c < nchunks) {
             const int kk = min(K, a.max_iter - n);
@@ -1234,8 +1239,8 @@ __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist_nbr(IterArgs a, unsigned ti
         return;
     }
 
-    NbrSync sync{a, FirstBound{a.resident_ticks, a.force_not_resident}, &sh_word, tiles_x, ntiles / tiles_x,
-                 0, 0, -1, 0, 0, false, false};
+    NbrSync sync{a, FirstBound{a.resident_ticks, a.force_not_resident},
+                 FirstBound{a.referee_ticks, a.force_not_resident}, &sh_word, tiles_x, ntiles / tiles_x, 0, 0, -1, 0, 0, false, false};
     double acc[K];
     // chunk after chunk; the last pass re-runs part of the chunk that stopped
     while (true) {
@@ -1384,6 +1389,7 @@ __global__ OF_ITER_BOUNDS(T * T / 64, K) void k_tvl1_persist_tag(IterArgs a, uns
     const int nchunks = (a.max_iter + K - 1) / K;
 
     if (blockIdx.x == ntiles) {   // referee
+        if (a.referee_absent) return;
         int n = 0, c = 0;
         while (c < nchunks) {
             const int kk = min(K, a.max_iter - n);
@@ -1439,12 +1445,16 @@ __global__ OF_ITER_BOUNDS(T * T / 64, K) void k_tvl1_persist_tag(IterArgs a, uns
     sq_load_state<false>(a, q, in, idx, cur0);
     __syncthreads();
 
-    // decision of chunk d, in wave 0: keep, or -1 if the wait failed
-    FirstBound fb{a.resident_ticks, a.force_not_resident};
+    // decision of chunk d, in wave 0: keep, or -1 if the wait failed.  The
+    // first wait for the neighbours and the first for the referee check that
+    // the grid is resident
+    FirstBound fb{a.resident_ticks, a.force_not_resident}, fb_referee{a.referee_ticks, a.force_not_resident};
     auto decision = [&](int d) -> int {
         const unsigned long long* w = &ctl->decision[d & 1].v;
         const unsigned long long want = (a.seq << 24) | ((unsigned long long)(d + 1) << 4);
-        if (!wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, fb)) return -1;
+        const int r = wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, fb_referee);
+        fb_referee = FirstBound{0ull, 0};
+        if (!r) return -1;
         return uniform((int)(__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFull));
     };
     SqState in0{}, in1{};   // inputs of the chunks before the last and last iterated
@@ -1474,7 +1484,7 @@ __global__ OF_ITER_BOUNDS(T * T / 64, K) void k_tvl1_persist_tag(IterArgs a, uns
                 ok &= r >= 0;
             }
             if (!ok) sh_fail[c & 1] = 1;
-            if (c < nchunks) fb = FirstBound{0ull, 0};   // the first wait was it
+            fb = FirstBound{0ull, 0};   // the first wait was it
             __syncthreads();
             if (uniform(sh_fail[c & 1])) return;
             keep = uniform(sh_keep[c & 1]);
@@ -1866,14 +1876,16 @@ static constexpr int persist_threads()
 // guarantee co-residency, but the runtime brackets it with about 11 us of
 // idle device time on each side (kernel trace of the 1920x1080 solve, 20
 // such launches per solve: 6.07 vs 5.67 ms per solve).  Instead the first
-// grid barrier of each launch checks residency with a wall-clock bound: if
-// the grid did not fully start (another persistent kernel on another stream
-// or process holding CUs, a CU-masked stream), the kernel ends with
-// kBarNotResident, the host switches the process to host-paced launches for
-// the warpings that would be persistent, and repeats the solve.  Host-paced
-// launches need no co-residency and give the same bits.
+// grid barrier of each launch (with neighbour flags: each workgroup's first
+// wait for its neighbours and its first for the referee, the last workgroup of
+// the grid) checks residency with a wall-clock bound: if the grid did not
+// fully start (another persistent kernel on another stream or process holding
+// CUs, a CU-masked stream), the kernel ends with kBarNotResident, the host
+// switches the process to host-paced launches for the warpings that would be
+// persistent, and repeats the solve.  Host-paced launches need no
+// co-residency and give the same bits.
 static std::atomic<int> g_host_paced{-1};   // -1: not read from the environment yet
-static std::atomic<int> g_force_not_resident{0};
+static std::atomic<int> g_force_not_resident{0}, g_referee_absent{0};
 constexpr double kResidentBoundUs = 2000.0;   // first-barrier wait of a launch
 
 bool persist_host_paced()
@@ -1891,6 +1903,8 @@ bool persist_host_paced()
 void set_persist_host_paced(bool on) { g_host_paced.store(on ? 1 : 0); }
 
 void set_persist_force_not_resident(bool on) { g_force_not_resident.store(on ? 1 : 0); }
+
+void set_persist_referee_absent(bool on) { g_referee_absent.store(on ? 1 : 0); }
 
 static std::atomic<unsigned long long> g_warp_seq{0};
 
@@ -1939,7 +1953,11 @@ static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, uns
     }
     IterArgs args = a;
     args.resident_ticks = bound_ticks;
+    // the referee decides once the slowest workgroup has completed the chunk:
+    // another 2 ms per 2^24 pixels, which take a chunk 0.3 ms
+    args.referee_ticks = bound_ticks + (bound_ticks * (unsigned long long)a.plane >> 24);
     args.force_not_resident = g_force_not_resident.load(std::memory_order_relaxed);
+    args.referee_absent = g_referee_absent.load(std::memory_order_relaxed);
     unsigned tx = gx, nt = ntiles;
     void* kargs[] = {(void*)&args, (void*)&tx, (void*)&nt};
     const hipError_t e = hipLaunchKernel(fn, dim3(nb), dim3(threads), kargs, 0, s);

@@ -76,7 +76,10 @@ struct IterArgs {
     // persistent kernel: wall-clock ticks that the first grid barrier waits
     // for all workgroups before it reports kBarNotResident (0: no bound)
     unsigned long long resident_ticks;
+    // the same for the first decision of a neighbour-synchronised warping
+    unsigned long long referee_ticks;
     int force_not_resident;   // test hook: the first barrier reports kBarNotResident
+    int referee_absent;       // test hook: the referee workgroup ends at once, as if it had not started
     // neighbour-synchronised warping kernel: per tile, (seq << 20) | chunks
     // completed.  `seq` numbers the warpings of the process from 1 (never
     // reused, below 2^40): it tags a warping's flags and decisions, so words
@@ -133,5 +136,8 @@ void set_persist_host_paced(bool on);
 // Test hook: persistent launches report kBarNotResident at their first
 // barrier while set.
 void set_persist_force_not_resident(bool on);
+// Test hook: the referee of neighbour-synchronised warpings ends at once while
+// set, and the tiles have to report kBarNotResident.
+void set_persist_referee_absent(bool on);
 
 }  // namespace amdflow

@@ -22,6 +22,7 @@ pytestmark = pytest.mark.gpu
 def restore_mode():
     yield
     D.persist_force_not_resident(False)
+    D.persist_referee_absent(False)
     set_persist_launch_mode(PERSIST_PLAIN)
 
 
@@ -54,6 +55,33 @@ def test_not_resident_takes_the_host_paced_repeat(K, R, restore_mode):
     D.persist_force_not_resident(True)
     u, it, uo, ito = _solve(320, 240, K, R, 42)
     assert persist_launch_mode() == PERSIST_HOST_PACED
+    assert np.array_equal(it, ito)
+    assert np.array_equal(u, uo)
+
+
+# The referee is the last workgroup of a neighbour-synchronised grid, so the one
+# that finds no place where the tiles just fit.  Tagged tiles of each size, tiles
+# that share CUs, 64-column tiles; one, two and many chunks.
+REFEREE_CASES = [(96, 70, 4, 0, 300), (200, 150, 4, 0, 9), (374, 330, 4, 0, 300), (100, 60, 4, 0, 4),
+                 (641, 479, 4, 0, 40), (320, 240, 2, 8, 300), (320, 240, 4, 4, 3), (150, 100, 2, 0, 4)]
+
+
+@pytest.mark.parametrize("w,h,K,R,cap,builtin", [c + (False,) for c in REFEREE_CASES] +
+                         [c + (True,) for c in REFEREE_CASES[:5]])
+def test_absent_referee_takes_the_host_paced_repeat(w, h, K, R, cap, builtin, restore_mode):
+    print("referee", w, h, K, R, cap, builtin, flush=True)
+    set_persist_launch_mode(PERSIST_PLAIN)
+    I0, I1, _, _ = synth.make_pair(w, h, 4.0, 45, bumps=True)
+    q0, q1 = synth.quantize(I0), synth.quantize(I1)
+    prm = dict(nscales=1, warps=2, max_iterations=cap)
+    D.persist_referee_absent(True)
+    with TV_L1(w, h, **prm) as tv:
+        if not builtin:
+            tv.set_launch_rule(0, K, R, 2)
+        tv.runDualTVL1Multiscale(q0, q1)
+        u, it = tv.getU().copy(), tv.iterations()
+    assert persist_launch_mode() == (PERSIST_PLAIN if builtin else PERSIST_HOST_PACED)
+    uo, ito = O.tvl1(q0, q1, O.default_params(**prm))
     assert np.array_equal(it, ito)
     assert np.array_equal(u, uo)
 
