@@ -151,6 +151,11 @@ public:
         h->paced_solves = h->paced_next;
         h->paced_next = std::min(2 * h->paced_next, kPacedMost);
     }
+    // A persistent solve went through: the next miss is a first one again.
+    void succeeded(of_tvl1* h) const
+    {
+        if (unique_.owns_lock() || shared_.owns_lock()) h->paced_next = kPacedFirst;
+    }
     bool builtin() const { return unique_.owns_lock(); }   // the built-in persistent rules apply
     bool own_rules() const { return own_rules_; }          // some scale's own rule is persistent
 
@@ -524,7 +529,7 @@ int solve_levels_once(of_tvl1* h, const float* init, int first, const int* warps
 // solve_levels_once, repeated once with host-paced launches if a persistent
 // launch was not co-resident: from then on, for the whole process, where the
 // handle's own rules asked for persistent launches; for a number of solves of
-// the handle, doubled each time, where only the built-in ones did.  The repeat
+// the handle (PersistTurn::pace) where only the built-in ones did.  The repeat
 // starts from the same pyramids and `init`, which a solve does not write.
 int solve_levels_schedule(of_tvl1* h, const float* init, int first, const int* warps_s,
                           const int* max_s, float* dst, hipStream_t st)
@@ -532,6 +537,7 @@ int solve_levels_schedule(of_tvl1* h, const float* init, int first, const int* w
     const PersistTurn turn(h, first);
     h->run_persist = turn.builtin();
     const int rc = solve_levels_once(h, init, first, warps_s, max_s, dst, st);
+    if (rc == OF_OK) turn.succeeded(h);
     if (rc != kRetryHostPaced) return rc;
     if (turn.own_rules()) set_persist_host_paced(true);
     else PersistTurn::pace(h);

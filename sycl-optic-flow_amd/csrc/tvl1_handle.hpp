@@ -15,7 +15,11 @@ namespace amdflow {
 
 constexpr int kInFlight = 3;   // iteration launches kept queued ahead of the device
 
-constexpr int kPacedMost = 4096;   // host-paced solves after a launch that was not co-resident, at most
+// Host-paced solves of a handle after a launch that was not co-resident or a
+// turn that did not come: the first time and, doubled each time without a
+// persistent solve between, at most.  A miss costs up to 20 ms, so at 256 solves
+// of 2 ms and more it adds 4% to a handle that never gets its turn.
+constexpr int kPacedFirst = 16, kPacedMost = 256;
 
 // Launch shape for scales of at least `min_pixels` pixels.
 struct LaunchRule {
@@ -78,7 +82,7 @@ struct of_tvl1 {
     std::vector<amdflow::LaunchRule> rules;
     bool run_persist = false;   // the built-in persistent rules apply to this solve
     int paced_solves = 0;       // solves that still take the host-paced ones
-    int paced_next = 16;        // how many after the next launch that is not co-resident
+    int paced_next = amdflow::kPacedFirst;   // how many after the next miss
     long long launches_issued = 0;
     int inflight = amdflow::kInFlight;
     double host_launch_s = 0.0, host_wait_s = 0.0;

@@ -80,6 +80,27 @@ def test_not_resident_keeps_the_process_and_paces_the_handle(restore_mode):
         _check(got, q0, q1, nscales=3)
 
 
+def test_back_off_starts_again_after_a_persistent_solve(restore_mode):
+    """Two misses with persistent solves between pace 16 solves each; misses one
+    after the other pace 16, 32, .. up to 256."""
+    q0, q1 = _pair(80, 60, 65)
+
+    def paced_after_a_miss(tv, missed):
+        D.persist_force_not_resident(True)
+        tv.runDualTVL1Multiscale(q0, q1)
+        D.persist_force_not_resident(False)
+        for n in range(missed):   # these do not try
+            assert _solve(tv, q0, q1)[2] == {0}
+
+    with TV_L1(80, 60, nscales=2, max_iterations=8) as tv:
+        for _ in range(3):
+            paced_after_a_miss(tv, 16)
+            assert _solve(tv, q0, q1)[2] == {2}
+        for missed in (16, 32, 64, 128, 256, 256):
+            paced_after_a_miss(tv, missed)
+        assert _solve(tv, q0, q1)[2] == {2}
+
+
 def test_host_paced_process_takes_host_paced_rules(restore_mode):
     q0, q1 = _pair(160, 120, 64)
     set_persist_launch_mode(PERSIST_HOST_PACED)
