@@ -108,9 +108,8 @@ void pick_rule(const of_tvl1* h, long long npx, int* K, int* R, int* persistent)
 // threads at 640x480: 1.54, 1.58, 1.28; at 1024x436: 1.92, 1.92, 1.38; at
 // 1920x1080: 4.11, 3.96, 2.81).  A solve whose own rules are persistent runs next
 // to others of its kind, as it asks for, and waits for one on built-in rules to
-// end.  No wait is longer than kTurnWait, since the other solve may itself wait
-// for work on its stream; a handle that waited in vain does not wait again for a
-// number of solves.  (Other processes are not seen: the residency check covers
+// end.  No wait is longer than kTurnWait, the time of a long solve; a handle that
+// waited in vain does not wait again for a number of solves.  (Other processes are not seen: the residency check covers
 // them.)
 constexpr int kTurnDevices = 64;
 constexpr long long kTurnPixels = 200000;
@@ -118,7 +117,10 @@ constexpr std::chrono::milliseconds kTurnWait{20};
 
 class PersistTurn {
 public:
-    PersistTurn(of_tvl1* h, int first)
+    // Takes the turn, or does without.  `earlier`, if not null, is an event on
+    // the solve's stream after the work that was there before the solve: a
+    // turn is not held through that, when nothing persistent runs.
+    PersistTurn(of_tvl1* h, int first, hipEvent_t earlier)
     {
         const bool back_off = h->paced_solves > 0;
         if (back_off) h->paced_solves--;
@@ -132,6 +134,8 @@ public:
         if (persist_host_paced() || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kTurnDevices)
             return;
         own_rules_ = own;
+        if (!own && (!builtin || back_off)) return;
+        if (earlier && hipEventSynchronize(earlier) != hipSuccess) return;   // the solve will see the error
         std::shared_timed_mutex& m = turns()[dev];
         if (builtin && !back_off) {
             const bool wait = (long long)h->nx[0] * h->ny[0] >= kTurnPixels;
@@ -198,6 +202,7 @@ void release(of_tvl1* h)
     host_free(h->hflow);
     host_free(h->hstatus);
     host_free(h->hreport);
+    if (h->earlier) (void)hipEventDestroy(h->earlier);
     for (hipEvent_t e : h->ev_pool) (void)hipEventDestroy(e);
     for (hipEvent_t e : h->scale_ev) (void)hipEventDestroy(e);
     if (h->stream) (void)hipStreamDestroy(h->stream);
@@ -532,9 +537,9 @@ int solve_levels_once(of_tvl1* h, const float* init, int first, const int* warps
 // the handle (PersistTurn::pace) where only the built-in ones did.  The repeat
 // starts from the same pyramids and `init`, which a solve does not write.
 int solve_levels_schedule(of_tvl1* h, const float* init, int first, const int* warps_s,
-                          const int* max_s, float* dst, hipStream_t st)
+                          const int* max_s, float* dst, hipStream_t st, hipEvent_t earlier)
 {
-    const PersistTurn turn(h, first);
+    const PersistTurn turn(h, first, earlier);
     h->run_persist = turn.builtin();
     const int rc = solve_levels_once(h, init, first, warps_s, max_s, dst, st);
     if (rc == OF_OK) turn.succeeded(h);
@@ -553,26 +558,47 @@ int solve_levels_schedule(of_tvl1* h, const float* init, int first, const int* w
 
 // The same limits at every scale.
 int solve_levels(of_tvl1* h, const float* init, int first, int warps, int max_iter, float* dst,
-                 hipStream_t st)
+                 hipStream_t st, hipEvent_t earlier = nullptr)
 {
     int w[kMaxScales], m[kMaxScales];
     for (int s = 0; s < kMaxScales; s++) {
         w[s] = warps;
         m[s] = max_iter;
     }
-    return solve_levels_schedule(h, init, first, w, m, dst, st);
+    return solve_levels_schedule(h, init, first, w, m, dst, st, earlier);
+}
+
+// An event after the work that `st`, a caller's stream, still has to do, or null
+// if it is idle (or the query fails: the solve's own calls then report it).
+int earlier_work(of_tvl1* h, hipStream_t st, hipEvent_t* out)
+{
+    *out = nullptr;
+    const hipError_t q = hipStreamQuery(st);
+    if (q == hipSuccess) return OF_OK;
+    if (q != hipErrorNotReady) {
+        (void)hipGetLastError();
+        return OF_OK;
+    }
+    (void)hipGetLastError();
+    if (!h->earlier) OF_HIP(hipEventCreateWithFlags(&h->earlier, hipEventDisableTiming));
+    OF_HIP(hipEventRecord(h->earlier, st));
+    *out = h->earlier;
+    return OF_OK;
 }
 
 // One full multiscale solve with the handle's parameters and zero initial flow.
 int solve(of_tvl1* h, const void* src0, const void* src1, bool is_u8, float* dst, hipStream_t st)
 {
+    // (the handle's own stream holds at most its copies of the frames)
+    hipEvent_t earlier = nullptr;
+    if (!st || st != h->stream) OF_TRY(earlier_work(h, st, &earlier));
     OF_TRY(tvl1_prepare(h, src0, src1, is_u8, st));
     if (h->init_level >= 0) {   // one-shot initial flow of of_tvl1_set_init_flow
         const int first = h->init_level;
         h->init_level = -1;
-        return solve_levels(h, h->init, first, h->prm.warps, h->prm.max_iterations, dst, st);
+        return solve_levels(h, h->init, first, h->prm.warps, h->prm.max_iterations, dst, st, earlier);
     }
-    return solve_levels(h, nullptr, h->ns - 1, h->prm.warps, h->prm.max_iterations, dst, st);
+    return solve_levels(h, nullptr, h->ns - 1, h->prm.warps, h->prm.max_iterations, dst, st, earlier);
 }
 
 // Launch-shape autotuner: every supported (iterations per launch, rows per
@@ -861,7 +887,9 @@ int of_tvl1_solve_prepared(of_tvl1* h, const float* dUinit, int first_scale, int
         if (first_scale < 0) first_scale = h->ns - 1;
         if (warps == 0) warps = h->prm.warps;
         if (max_iterations == 0) max_iterations = h->prm.max_iterations;
-        return solve_levels(h, dUinit, first_scale, warps, max_iterations, dU, st);
+        hipEvent_t earlier = nullptr;
+        OF_TRY(earlier_work(h, st, &earlier));
+        return solve_levels(h, dUinit, first_scale, warps, max_iterations, dU, st, earlier);
     });
 }
 
@@ -880,7 +908,9 @@ int of_tvl1_solve_prepared_schedule(of_tvl1* h, const float* dUinit, int first_s
             w[s] = warps[s] ? warps[s] : h->prm.warps;
             m[s] = max_iterations[s] ? max_iterations[s] : h->prm.max_iterations;
         }
-        return solve_levels_schedule(h, dUinit, first_scale, w, m, dU, (hipStream_t)stream);
+        hipEvent_t earlier = nullptr;
+        OF_TRY(earlier_work(h, (hipStream_t)stream, &earlier));
+        return solve_levels_schedule(h, dUinit, first_scale, w, m, dU, (hipStream_t)stream, earlier);
     });
 }
 

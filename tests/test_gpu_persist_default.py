@@ -110,6 +110,41 @@ def test_host_paced_process_takes_host_paced_rules(restore_mode):
     _check(got, q0, q1, nscales=3)
 
 
+def test_a_solve_behind_other_work_does_not_hold_the_turn(restore_mode):
+    """A solve whose stream still has a tenth of a second of other work to do
+    runs nothing persistent yet: another handle's solve takes the turn
+    meanwhile instead of waiting in vain and running host-paced."""
+    import time
+
+    import torch
+    W, H = 640, 480
+    q0, q1 = _pair(W, H, 66)
+    prm = dict(nscales=3, max_iterations=60)
+    d0, d1 = torch.from_numpy(q0).cuda(), torch.from_numpy(q1).cuda()
+    dU = torch.empty(2 * W * H, dtype=torch.float32, device="cuda")
+    st = torch.cuda.Stream()
+    with TV_L1(W, H, **prm) as a, TV_L1(W, H, **prm) as b:
+        _solve(b, q0, q1)
+        a.run_device_u8(d0.data_ptr(), d1.data_ptr(), dU.data_ptr(), st.cuda_stream)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(st):
+            torch.cuda._sleep(300_000_000)
+        t = threading.Thread(target=a.run_device_u8,
+                             args=(d0.data_ptr(), d1.data_ptr(), dU.data_ptr(), st.cuda_stream))
+        t.start()
+        time.sleep(0.02)
+        behind = not st.query()
+        got = _solve(b, q0, q1)
+        behind &= not st.query()
+        t.join()
+        torch.cuda.synchronize()
+        first = (dU.cpu().numpy(), a.iterations())
+    assert behind, "the other work ended too early to show anything"
+    assert got[2] == {2}
+    _check(got, q0, q1, **prm)
+    _check(first, q0, q1, **prm)
+
+
 def test_solves_from_several_threads(restore_mode):
     """One solve at a time takes the persistent rules, the others run host-paced
     beside it."""
