@@ -108,9 +108,11 @@ void pick_rule(const of_tvl1* h, long long npx, int* K, int* R, int* persistent)
 // threads at 640x480: 1.54, 1.58, 1.28; at 1024x436: 1.92, 1.92, 1.38; at
 // 1920x1080: 4.11, 3.96, 2.81).  A solve whose own rules are persistent runs next
 // to others of its kind, as it asks for, and waits for one on built-in rules to
-// end.  No wait is longer than kTurnWait, the time of a long solve; a handle that
-// waited in vain does not wait again for a number of solves.  (Other processes are not seen: the residency check covers
-// them.)
+// end; without its turn it runs host-paced too, since a launch of its own rules
+// that is not co-resident makes the whole process host-paced.  No wait is longer
+// than kTurnWait, the time of a long solve; a handle that waited in vain does not
+// wait again for a number of solves.  (Other processes are not seen: the residency
+// check covers them.)
 constexpr int kTurnDevices = 64;
 constexpr long long kTurnPixels = 200000;
 constexpr std::chrono::milliseconds kTurnWait{20};
@@ -130,22 +132,24 @@ public:
             if (!r) builtin = true;
             else if (r->persistent) own = true;
         }
+        own_rules_ = own;
         int dev = 0;
         if (persist_host_paced() || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kTurnDevices)
             return;
-        own_rules_ = own;
+        unlocked_ = false;
         if (!own && (!builtin || back_off)) return;
         if (earlier && hipEventSynchronize(earlier) != hipSuccess) return;   // the solve will see the error
         std::shared_timed_mutex& m = turns()[dev];
+        bool waited = back_off;
         if (builtin && !back_off) {
-            const bool wait = (long long)h->nx[0] * h->ny[0] >= kTurnPixels;
+            waited = (long long)h->nx[0] * h->ny[0] >= kTurnPixels;
             unique_ = std::unique_lock<std::shared_timed_mutex>(m, std::defer_lock);
-            if (wait ? unique_.try_lock_for(kTurnWait) : unique_.try_lock()) return;
-            if (wait) pace(h);
+            if (waited ? unique_.try_lock_for(kTurnWait) : unique_.try_lock()) return;
+            if (waited) pace(h);
         }
         if (own) {
             shared_ = std::shared_lock<std::shared_timed_mutex>(m, std::defer_lock);
-            if (!(back_off ? shared_.try_lock() : shared_.try_lock_for(kTurnWait))) pace(h);
+            if (!(waited ? shared_.try_lock() : shared_.try_lock_for(kTurnWait))) pace(h);
         }
     }
     // The handle's next solves neither take the built-in persistent rules nor wait.
@@ -161,7 +165,8 @@ public:
         if (unique_.owns_lock() || shared_.owns_lock()) h->paced_next = kPacedFirst;
     }
     bool builtin() const { return unique_.owns_lock(); }   // the built-in persistent rules apply
-    bool own_rules() const { return own_rules_; }          // some scale's own rule is persistent
+    // the handle's own persistent rules apply, and some scale has one
+    bool own() const { return own_rules_ && (unique_.owns_lock() || shared_.owns_lock() || unlocked_); }
 
 private:
     // never destroyed: a solve may run while the process ends
@@ -173,6 +178,7 @@ private:
     std::unique_lock<std::shared_timed_mutex> unique_;
     std::shared_lock<std::shared_timed_mutex> shared_;
     bool own_rules_ = false;
+    bool unlocked_ = true;   // no turns are kept: own rules apply as they are
 };
 
 void release(of_tvl1* h)
@@ -301,8 +307,8 @@ int run_warping(of_tvl1* h, int s, int w, hipStream_t st)
     a.tile_flags = h->tile_flags;
     a.seq = next_warp_seq();
 
-    if (persistent && persist_host_paced()) {
-        persistent = 0;   // the process gave up persistent launches
+    if (persistent && (persist_host_paced() || !(h->run_persist || h->run_own))) {
+        persistent = 0;   // the process gave up persistent launches, or this solve has no turn
         // (4, 0) with neighbour flags picks its tiles by size (launch_persist);
         // 16 x 16 ones host-paced are the slower choice from about 20 000
         // pixels on (1920x1080 pyramid, ms: 120x68 0.64 against 0.78 of (4, 4);
@@ -541,12 +547,13 @@ int solve_levels_schedule(of_tvl1* h, const float* init, int first, const int* w
 {
     const PersistTurn turn(h, first, earlier);
     h->run_persist = turn.builtin();
+    h->run_own = turn.own();
     const int rc = solve_levels_once(h, init, first, warps_s, max_s, dst, st);
     if (rc == OF_OK) turn.succeeded(h);
     if (rc != kRetryHostPaced) return rc;
-    if (turn.own_rules()) set_persist_host_paced(true);
+    if (turn.own()) set_persist_host_paced(true);
     else PersistTurn::pace(h);
-    h->run_persist = false;
+    h->run_persist = h->run_own = false;
     h->timed.clear();   // launch events of the abandoned solve
     const int rc2 = solve_levels_once(h, init, first, warps_s, max_s, dst, st);
     if (rc2 == kRetryHostPaced) {   // the mode was set back to persistent meanwhile

@@ -81,6 +81,7 @@ struct of_tvl1 {
     amdflow::GaussTaps g_pre{}, g_zoom{};
     std::vector<amdflow::LaunchRule> rules;
     bool run_persist = false;   // the built-in persistent rules apply to this solve
+    bool run_own = false;       // the handle's own persistent rules do
     hipEvent_t earlier = nullptr;   // the work on a caller's stream ahead of a solve
     int paced_solves = 0;       // solves that still take the host-paced ones
     int paced_next = amdflow::kPacedFirst;   // how many after the next miss

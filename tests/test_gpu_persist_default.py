@@ -145,6 +145,30 @@ def test_a_solve_behind_other_work_does_not_hold_the_turn(restore_mode):
     _check(first, q0, q1, **prm)
 
 
+def test_own_rules_do_not_run_beside_a_builtin_solve(restore_mode):
+    """While a long solve on the built-in rules has the device, a handle with
+    persistent rules of its own waits 20 ms for it and then runs host-paced:
+    beside it, either grid may not be resident, and the process would become
+    host-paced for good."""
+    import time
+    q0, q1 = _pair(320, 240, 67)
+    L0, L1 = _pair(1280, 720, 68)
+    prm = dict(nscales=3, max_iterations=60)
+    with TV_L1(1280, 720, nscales=1, warps=60, epsilon=0.0) as a, TV_L1(320, 240, **prm) as b:
+        b.set_launch_rule(0, 4, 0, 2)
+        t = threading.Thread(target=a.runDualTVL1Multiscale, args=(L0, L1))
+        t0 = time.monotonic()
+        t.start()
+        time.sleep(0.01)
+        got = _solve(b, q0, q1)
+        t.join()
+        took = time.monotonic() - t0
+    assert took > 0.06, "the long solve ended too early to show anything"
+    assert persist_launch_mode() == PERSIST_PLAIN
+    assert got[2] == {0}
+    _check(got, q0, q1, **prm)
+
+
 def test_solves_from_several_threads(restore_mode):
     """One solve at a time takes the persistent rules, the others run host-paced
     beside it."""
@@ -173,3 +197,29 @@ def test_solves_from_several_threads(restore_mode):
         for u, it in results[k]:
             assert np.array_equal(it, ito)
             assert np.array_equal(u, uo)
+
+
+def test_threads_take_turns_at_persistent_solves(restore_mode):
+    """From 200000 pixels on a solve waits for the device's turn: solves
+    of two threads are persistent one after the other."""
+    q0, q1 = _pair(640, 480, 69)
+    prm = dict(nscales=3, max_iterations=40)
+    got, errors = [], []
+
+    def worker():
+        try:
+            with TV_L1(640, 480, **prm) as tv:
+                for _ in range(4):
+                    got.append(_solve(tv, q0, q1))
+        except Exception as e:   # reported by the main thread
+            errors.append(e)
+
+    th = [threading.Thread(target=worker) for _ in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not errors, errors
+    assert len(got) == 8 and sum(g[2] == {2} for g in got) >= 1
+    for g in got:
+        _check(g, q0, q1, **prm)
