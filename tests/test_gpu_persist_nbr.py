@@ -165,3 +165,32 @@ def test_handles_created_after_destroyed_ones():
         u, it = _solve(q0, q1, [(0, (1, 2, 4, 1)[k], (4, 0, 8, 0)[k], NBR)], nscales=4)
         assert np.array_equal(it, ito), k
         assert np.array_equal(u, uo), k
+
+
+def test_tagged_words_past_the_last_tag():
+    """A warping takes as many of a handle's 2^32 tags as its iteration limit
+    allows chunks: with a limit of 2^20 they run out in the 4096th warping,
+    where the words are cleared and the tags start again.  Every solve before,
+    at and after that gives the oracle's bits, here on three sizes of tagged
+    tiles."""
+    q0, q1 = _pair(300, 250, 3.0, 77)
+    prm = dict(nscales=3, warps=40, max_iterations=1 << 20, epsilon=0.03)
+    uo, ito = _oracle(q0, q1, **prm)
+    assert ito.max() < 300
+    solves = 4096 // (3 * 40) + 4
+    with TV_L1(300, 250, **prm) as tv:
+        for n in range(solves):
+            tv.runDualTVL1Multiscale(q0, q1)
+            assert np.array_equal(tv.iterations(), ito), n
+            assert np.array_equal(tv.getU(), uo), n
+
+
+def test_limits_past_the_flags_of_three_iterations_per_chunk():
+    """Tiles that share CUs take 3 iterations per chunk, and 4 where the
+    iteration limit has more than 2^20 chunks of 3."""
+    q0, q1 = _pair(500, 420, 3.0, 78)
+    prm = dict(nscales=1, warps=2, max_iterations=3_200_000)
+    u, it = _solve(q0, q1, [(0, 4, 0, NBR)], **prm)
+    uo, ito = _oracle(q0, q1, **prm)
+    assert np.array_equal(it, ito)
+    assert np.array_equal(u, uo)
