@@ -139,8 +139,10 @@ __device__ __forceinline__ void bicubic_sample_pairs(const float* __restrict__ a
 {
     bool same = t.fy == __int_as_float(lane_partner(__float_as_int(t.fy)));
 #pragma unroll
-    for (int c = 0; c < 4; c++)
-        same &= (t.cols[c] == lane_partner(t.cols[c])) & (t.rows[c] == lane_partner(t.rows[c]));
+    for (int c = 0; c < 4; c++) {
+        same &= t.cols[c] == lane_partner(t.cols[c]);
+        same &= t.rows[c] == lane_partner(t.rows[c]);
+    }
     if (!__all(same)) {
         ra = bicubic_sample(a, nx, t);
         rb = bicubic_sample(b, nx, t);

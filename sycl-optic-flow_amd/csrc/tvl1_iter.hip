@@ -506,7 +506,6 @@ __device__ __forceinline__ void sq_iterations(const IterArgs& a, SqPixel& q, int
     }
 }
 
-template <bool COH>
 __device__ __forceinline__ void sq_load_constants(const IterArgs& a, SqPixel& q, bool in, size_t idx)
 {
     q.gx = q.gy = q.rc = 0.0f;
@@ -567,7 +566,7 @@ __device__ __forceinline__ void tile_iterate_sq(const IterArgs& a, int bx, int b
     q.fr = y == 0;
     q.lr = y == ny - 1;
     q.mine = in && lx >= K && lx < K + C && ly >= K && ly < K + C;
-    sq_load_constants<COH>(a, q, in, idx);
+    sq_load_constants(a, q, in, idx);
     if (!sync.ready()) return;
     sq_load_state<COH>(a, q, in, idx, cur);
     sq_iterations<T, K>(a, q, kk, T, acc, sh);
@@ -1441,7 +1440,7 @@ __global__ OF_ITER_BOUNDS(T * T / 64, K) void k_tvl1_persist_tag(IterArgs a, uns
     q.lr = y == a.ny - 1;
     q.mine = in && centre;
     if (threadIdx.x < 2) sh_fail[threadIdx.x] = 0;
-    sq_load_constants<false>(a, q, in, idx);
+    sq_load_constants(a, q, in, idx);
     sq_load_state<false>(a, q, in, idx, cur0);
     __syncthreads();
 
@@ -1569,7 +1568,7 @@ __global__ __launch_bounds__(1024) void k_tvl1_single(IterArgs a)
     q.fr = ly == 0;
     q.lr = ly == ny - 1;
     q.mine = in;
-    sq_load_constants<false>(a, q, in, idx);
+    sq_load_constants(a, q, in, idx);
     sq_load_state<false>(a, q, in, idx, cur);
     int n = 0;
     while (n < a.max_iter) {
