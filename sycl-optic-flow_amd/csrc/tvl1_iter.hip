@@ -1911,15 +1911,17 @@ unsigned long long next_warp_seq() { return g_warp_seq.fetch_add(1) + 1; }
 
 // Launches the persistent kernel `fn` of `threads` threads over gx x gy tiles.
 // nbr: the neighbour-synchronised kernel with K iterations per chunk, whose
-// grid is the tile workgroups plus one referee workgroup.  `resident` caches
-// the kernel's co-resident workgroups on the device (-1: not known yet).
+// grid is the tile workgroups plus one referee workgroup.  `cache` holds the
+// kernel's co-resident workgroups on the device (-1: not known yet); solves of
+// several threads may find it so at once, and then each asks.
 // tile_each: every tile needs a workgroup of its own.
 static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, unsigned gx, unsigned gy,
-                               const IterArgs& a, int nblocks, int* resident, hipStream_t s,
+                               const IterArgs& a, int nblocks, std::atomic<int>& cache, hipStream_t s,
                                bool tile_each = false)
 {
-    static unsigned long long bound_ticks = 0;
-    if (*resident < 0) {
+    static std::atomic<unsigned long long> bound{0};   // written before any cache
+    int resident = cache.load(std::memory_order_acquire);
+    if (resident < 0) {
         int dev = 0, per_cu = 0, cus = 0, clock_khz = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
@@ -1929,7 +1931,8 @@ static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, uns
             return OF_ERR_HIP;
         }
         // the residency bound in wall-clock ticks (at least 1 ms at any rate)
-        bound_ticks = (unsigned long long)(kResidentBoundUs * 1e-3 * std::max(clock_khz, 1000));
+        bound.store((unsigned long long)(kResidentBoundUs * 1e-3 * std::max(clock_khz, 1000)),
+                    std::memory_order_relaxed);
         // at most 4 workgroups per CU: 1024 arrivals on one counter and
         // pollers of one word per barrier are already plenty (the compiled
         // bound allows 2 of 8 waves)
@@ -1937,13 +1940,14 @@ static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, uns
         // 9 waves puts 3 on one SIMD, which the occupancy query does not see
         const int waves = threads / 64, per_simd = (waves + 3) / 4;
         per_cu = std::min(per_cu, per_cu * waves / 4 / per_simd);
-        *resident = std::min(per_cu, 4) * cus;
+        resident = std::min(per_cu, 4) * cus;
+        cache.store(resident, std::memory_order_release);
     }
-    if (*resident <= (nbr ? 1 : 0)) return OF_ERR_UNSUPPORTED;
+    if (resident <= (nbr ? 1 : 0)) return OF_ERR_UNSUPPORTED;
     const unsigned ntiles = gx * gy;
     unsigned nb = nblocks > 0 ? (unsigned)nblocks : ntiles;
     if (nb > ntiles) nb = ntiles;
-    if (nb > (unsigned)*resident - (nbr ? 1u : 0u)) nb = (unsigned)*resident - (nbr ? 1u : 0u);
+    if (nb > (unsigned)resident - (nbr ? 1u : 0u)) nb = (unsigned)resident - (nbr ? 1u : 0u);
     if (tile_each && nb < ntiles) return OF_ERR_UNSUPPORTED;
     if (nbr) {
         if (!a.tile_flags || a.seq == 0 || a.seq >= kNbrMaxSeq) return OF_ERR_ARG;
@@ -1951,6 +1955,7 @@ static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, uns
         nb += 1;   // the referee
     }
     IterArgs args = a;
+    const unsigned long long bound_ticks = bound.load(std::memory_order_relaxed);
     args.resident_ticks = bound_ticks;
     // the referee decides once the slowest workgroup has completed the chunk:
     // another 2 ms per 2^24 pixels, which take a chunk 0.3 ms
@@ -1970,23 +1975,23 @@ static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, uns
 template <int K, int R, bool NBR>
 static int launch_persist_kr(const IterArgs& a, int nblocks, hipStream_t s)
 {
-    static int resident = -1;
+    static std::atomic<int> resident{-1};
     unsigned gx, gy;
     iter_grid(K, R, a.nx, a.ny, &gx, &gy);
     return launch_persist_grid(persist_kernel<K, R, NBR>(), persist_threads<R>(), K, NBR, gx, gy, a, nblocks,
-                               &resident, s);
+                               resident, s);
 }
 
 // Square tiles of T x T pixels with K iterations per chunk.
 template <int T, int K>
 static int launch_persist_sq(const IterArgs& a, int nblocks, hipStream_t s)
 {
-    static int resident = -1;
+    static std::atomic<int> resident{-1};
     static_assert(T * T % 64 == 0 && T * T <= 1024, "whole waves");
     static_assert(K <= kSqMaxIters, "room for the partials");
     const unsigned gx = cdiv((size_t)a.nx, (size_t)(T - 2 * K)), gy = cdiv((size_t)a.ny, (size_t)(T - 2 * K));
     return launch_persist_grid((const void*)k_tvl1_persist_nbr<K, 0, T * T / 64, T>, T * T, K, true, gx, gy, a,
-                               nblocks, &resident, s);
+                               nblocks, resident, s);
 }
 
 // The same with tagged values; OF_ERR_UNSUPPORTED where the tiles do not all
@@ -1994,11 +1999,11 @@ static int launch_persist_sq(const IterArgs& a, int nblocks, hipStream_t s)
 template <int T, int K>
 static int launch_persist_tagged(const IterArgs& a, int nblocks, hipStream_t s)
 {
-    static int resident = -1;
+    static std::atomic<int> resident{-1};
     const unsigned gx = cdiv((size_t)a.nx, (size_t)(T - 2 * K)), gy = cdiv((size_t)a.ny, (size_t)(T - 2 * K));
     if (!a.halo || nblocks > 0) return OF_ERR_UNSUPPORTED;
     return launch_persist_grid((const void*)k_tvl1_persist_tag<T, K>, T * T, K, true, gx, gy, a, (int)(gx * gy),
-                               &resident, s, true);
+                               resident, s, true);
 }
 
 // The shape (4, 0) with neighbour flags: square tiles of a size chosen by the
