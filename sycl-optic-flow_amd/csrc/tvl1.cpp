@@ -201,10 +201,8 @@ void release(of_tvl1* h)
     dev_free(h->init);
     dev_free(h->ctl);
     dev_free(h->partials);
-    dev_free(h->tile_flags);
-    dev_free(h->halo);
+    dev_free(h->zeroed);
     dev_free(h->energy);
-    dev_free(h->d_iters);
     host_free(h->hflow);
     host_free(h->hstatus);
     host_free(h->hreport);
@@ -790,10 +788,11 @@ int of_tvl1_create(const of_tvl1_params* params, int width, int height, of_tvl1*
         if (!st) st = dev_alloc(&h->ctl, 1);
         // x2: the persistent kernel double-buffers its partials by chunk parity
         if (!st) st = dev_alloc(&h->partials, 2 * maxpart);
-        if (!st) st = dev_alloc(&h->tile_flags, maxtiles);
-        if (!st) st = dev_alloc(&h->halo, halo_words(N0));
+        // what starts as zeros, in one block and one fill: the flags carry the
+        // warping's seq and the halo words a tag, both from 1 on
+        const size_t nhalo = halo_words(N0), nzero = maxtiles + nhalo + ((size_t)ns * p.warps + 1) / 2;
+        if (!st) st = dev_alloc(&h->zeroed, nzero);
         if (!st) st = dev_alloc(&h->energy, 2 * kEnergyBlocks + 3);
-        if (!st) st = dev_alloc(&h->d_iters, (size_t)ns * p.warps);
         if (!st) st = host_alloc(&h->hflow, 2 * N0, hipHostMallocDefault);
         if (!st) st = host_alloc(&h->hstatus, 1, hipHostMallocMapped | hipHostMallocCoherent);
         if (!st)
@@ -804,10 +803,10 @@ int of_tvl1_create(const of_tvl1_params* params, int width, int height, of_tvl1*
         std::memset(h->hreport, 0, sizeof(int) * ((size_t)ns * p.warps + 1));
         std::memset(h->hflow, 0, sizeof(float) * 2 * N0);
         h->h_iters.assign((size_t)ns * p.warps, 0);
-        // flags carry the warping's seq (from 1): zero means never set
-        if (hipMemset(h->d_iters, 0, sizeof(int) * (size_t)ns * p.warps) != hipSuccess ||
-            hipMemset(h->tile_flags, 0, sizeof(unsigned long long) * maxtiles) != hipSuccess ||
-            hipMemset(h->halo, 0, sizeof(unsigned long long) * halo_words(N0)) != hipSuccess) {
+        h->tile_flags = h->zeroed;
+        h->halo = h->zeroed + maxtiles;
+        h->d_iters = (int*)(h->halo + nhalo);
+        if (hipMemset(h->zeroed, 0, sizeof(unsigned long long) * nzero) != hipSuccess) {
             release(h);
             return OF_ERR_HIP;
         }

@@ -64,6 +64,7 @@ struct of_tvl1 {
     float* hflow = nullptr;     // pinned host copy returned by of_tvl1_flow
     amdflow::TvCtl* ctl = nullptr;
     double* partials = nullptr;
+    unsigned long long* zeroed = nullptr;       // the block of the next two and d_iters
     unsigned long long* tile_flags = nullptr;   // one word per tile (neighbour-synchronised warpings)
     unsigned long long* halo = nullptr;         // halo_words(W*H): IterArgs::halo
     unsigned halo_tag = 0;                      // tags up to this one have been used in it
