@@ -1043,14 +1043,23 @@ __device__ __forceinline__ int wave_wait(const IterArgs& a, const unsigned long 
     }
 }
 
+// Bound of the wait for decision q: the first one checks that the referee is
+// resident.  It decides once the slowest workgroup has completed the chunk:
+// another 2 ms per 2^24 pixels, which take a chunk 0.3 ms.
+__device__ __forceinline__ FirstBound referee_bound(const IterArgs& a, int q)
+{
+    if (q != 0) return FirstBound{0ull, 0};
+    return FirstBound{a.resident_ticks + (a.resident_ticks * (unsigned long long)a.plane >> 24), a.force_not_resident};
+}
+
 // Synchronisation of one workgroup of k_tvl1_persist_nbr with the others.
 // `stop_chunk`/`stop_keep`: set once the warping is known to stop after
 // stop_keep iterations of chunk stop_chunk.  Members are uniform.
 struct NbrSync {
     const IterArgs& a;
     // a plain launch also checks that the grid is resident: the first wait for
-    // the neighbours, and the first for a decision, which the referee makes
-    FirstBound fb, fb_referee;
+    // the neighbours (fb), and the one for the referee's first decision
+    FirstBound fb;
     int* sh;         // LDS word for results of wave 0
     unsigned tiles_x, tiles_y, tile;
     int c;           // chunk of the current tile
@@ -1083,10 +1092,9 @@ struct NbrSync {
         if (threadIdx.x < 64) {
             const unsigned long long* w = &a.ctl->decision[q & 1].v;
             const unsigned long long want = (a.seq << 24) | ((unsigned long long)(q + 1) << 4);
-            if (wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, fb_referee))
+            if (wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, referee_bound(a, q)))
                 r = (int)(__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFull);
         }
-        fb_referee = FirstBound{0ull, 0};
         return share(r);
     }
 
@@ -1238,8 +1246,8 @@ __global__ OF_ITER_BOUNDS(NW, K) void k_tvl1_persist_nbr(IterArgs a, unsigned ti
         return;
     }
 
-    NbrSync sync{a, FirstBound{a.resident_ticks, a.force_not_resident},
-                 FirstBound{a.referee_ticks, a.force_not_resident}, &sh_word, tiles_x, ntiles / tiles_x, 0, 0, -1, 0, 0, false, false};
+    NbrSync sync{a, FirstBound{a.resident_ticks, a.force_not_resident}, &sh_word, tiles_x, ntiles / tiles_x,
+                 0, 0, -1, 0, 0, false, false};
     double acc[K];
     // chunk after chunk; the last pass re-runs part of the chunk that stopped
     while (true) {
@@ -1445,15 +1453,13 @@ __global__ OF_ITER_BOUNDS(T * T / 64, K) void k_tvl1_persist_tag(IterArgs a, uns
     __syncthreads();
 
     // decision of chunk d, in wave 0: keep, or -1 if the wait failed.  The
-    // first wait for the neighbours and the first for the referee check that
-    // the grid is resident
-    FirstBound fb{a.resident_ticks, a.force_not_resident}, fb_referee{a.referee_ticks, a.force_not_resident};
+    // first wait for the neighbours (fb) and the one for the first decision
+    // check that the grid is resident
+    FirstBound fb{a.resident_ticks, a.force_not_resident};
     auto decision = [&](int d) -> int {
         const unsigned long long* w = &ctl->decision[d & 1].v;
         const unsigned long long want = (a.seq << 24) | ((unsigned long long)(d + 1) << 4);
-        const int r = wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, fb_referee);
-        fb_referee = FirstBound{0ull, 0};
-        if (!r) return -1;
+        if (!wave_wait(a, threadIdx.x == 0 ? w : nullptr, want, referee_bound(a, d))) return -1;
         return uniform((int)(__hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 0xFull));
     };
     SqState in0{}, in1{};   // inputs of the chunks before the last and last iterated
@@ -1955,11 +1961,7 @@ static int launch_persist_grid(const void* fn, int threads, int K, bool nbr, uns
         nb += 1;   // the referee
     }
     IterArgs args = a;
-    const unsigned long long bound_ticks = bound.load(std::memory_order_relaxed);
-    args.resident_ticks = bound_ticks;
-    // the referee decides once the slowest workgroup has completed the chunk:
-    // another 2 ms per 2^24 pixels, which take a chunk 0.3 ms
-    args.referee_ticks = bound_ticks + (bound_ticks * (unsigned long long)a.plane >> 24);
+    args.resident_ticks = bound.load(std::memory_order_relaxed);
     args.force_not_resident = g_force_not_resident.load(std::memory_order_relaxed);
     args.referee_absent = g_referee_absent.load(std::memory_order_relaxed);
     unsigned tx = gx, nt = ntiles;

@@ -76,8 +76,6 @@ struct IterArgs {
     // persistent kernel: wall-clock ticks that the first grid barrier waits
     // for all workgroups before it reports kBarNotResident (0: no bound)
     unsigned long long resident_ticks;
-    // the same for the first decision of a neighbour-synchronised warping
-    unsigned long long referee_ticks;
     int force_not_resident;   // test hook: the first barrier reports kBarNotResident
     int referee_absent;       // test hook: the referee workgroup ends at once, as if it had not started
     // neighbour-synchronised warping kernel: per tile, (seq << 20) | chunks
