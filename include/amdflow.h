@@ -150,7 +150,9 @@ int of_tvl1_set_launch_rule(of_tvl1 *h, long long min_pixels, int iters_per_laun
  * 16 x 16 ones, or 64 x 16 from 20000 pixels on), which needs no
  * co-residency.  AMDFLOW_HOST_PACED=1 in the environment starts a process in
  * host-paced mode.  Where only the built-in rules made a warping persistent,
- * the process keeps its mode and the handle's next solves run host-paced.
+ * the process keeps its mode and the handle's next solves run host-paced.  A
+ * solve with persistent rules of its own waits up to 20 ms for one on the
+ * built-in rules to end, and runs host-paced if it does not.
  * Results are the same bits in both modes. */
 enum { OF_PERSIST_PLAIN = 0, OF_PERSIST_HOST_PACED = 1 };
 int of_persist_launch_mode(void);

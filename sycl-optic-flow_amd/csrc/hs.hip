@@ -416,10 +416,11 @@ void hs_release(of_hs* h)
 }
 
 // The launch shape of a level: the caller's, or the cheapest of 64x32 and
-// 64x48 tiles with 1..14 sweeps per launch.  A sweep is bound by VALU issue
-// (26 instructions per pixel of the tile, halo included), a launch adds its ramp and, per round of 256 workgroups, the loads and
-// stores; deep blocks amortise those, small halos save work, and the grid
-// quantises to rounds of the 256 CUs.  The model (us): 1.5 per launch, per
+// 64x48 tiles with 1..14 sweeps per launch.  A sweep is its chain, barrier and
+// 26 VALU instructions per pixel of the tile, halo included (VALU busy a third
+// of the time at 640x480); a launch adds its ramp and, per round of 256
+// workgroups, the loads and stores; deep blocks amortise those, small halos save
+// work, and the grid quantises to rounds of the 256 CUs.  The model (us): 1.5 per launch, per
 // round 1.5 + 0.010 per tile row and sweep.  Over 79x44 .. 1920x1080 it
 // picks within 8% of the fastest of 46 measured shapes (64x64 and 8-wave
 // tiles among them), e.g. 120 sweeps (us; 64x32 tiles with 4 sweeps per

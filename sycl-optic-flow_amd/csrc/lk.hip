@@ -394,7 +394,9 @@ __global__ __launch_bounds__(256) void k_lk_update(const float* __restrict__ row
 // the three-kernel iteration k_lk_it_products / k_lk_boxsum / k_lk_update (the
 // windows clipped to the image), so the flow is the same bits as kk rounds of
 // it.  A null u starts from zero flow.
-// Bound by VALU issue: 0.95 us per iteration and row of each wave.  Row sums as
+// Bound by the rounds of one 16-wave workgroup per CU, 0.95 us per iteration and
+// row of each wave, whose loads, iterations and stores follow one another (VALU
+// busy 34% of a launch at 1280 x 720).  Row sums as
 // shifted adds and tap pairs from one address took a 1280 x 720 solve (3 levels,
 // 7 x 7, 5 iterations) from 172 to 157 us.  Tried and slower: 512 threads of 8
 // rows (172 us), a cap of 64 registers so that two workgroups share a CU (204

@@ -33,8 +33,9 @@ namespace {
 // million pixels on (whole scales, ms: 1280x720 1.01 / 1.08, 1536x864 0.99 / 1.07,
 // 1664x936 1.31 / 1.45, 1760x990 1.38 / 1.34, 1920x1080 2.50 / 2.09).  They save
 // the host's part in every chunk, 9 to 14 us at the small scales where a chunk's
-// work is 2 to 4 (320x240, five scales: 2.92 -> 1.31 ms per solve; 1024x436: 3.27 ->
-// 1.52; 1920x1080: 5.82 -> 3.30).
+// work is 2 to 4 (ms per solve against kPacedRules, five scales, u8 host frames of
+// a synthetic pair with flows up to 6 px: 320x240 2.69 -> 1.23, 640x480 2.67 ->
+// 1.34, 1024x436 3.24 -> 1.45, 1920x1080 5.78 -> 3.19).
 const LaunchRule kDefaultRules[] = {
     {1600000, 2, 8, kPersistNeighbour},
     {0, 4, 0, kPersistNeighbour},
