@@ -33,6 +33,7 @@ namespace amdflow {
 namespace {
 
 typedef short s16x8 __attribute__((ext_vector_type(8)));
+typedef short s16x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -98,7 +99,8 @@ __device__ __forceinline__ f32x8 load_channels(const float* __restrict__ X, long
 //
 // The 8 consecutive k of an MFMA lane are channels of one tap where CX is a
 // multiple of 8: one 16-byte LDS read.  The 5- and 2-channel layers read them
-// one by one: padding a tap to 8 channels instead would group the fp32 sums
+// one by one, by a table of offsets (16 images of 68x120: the whole forward 82.1
+// us, 84.4 with the offsets computed per lane): padding a tap to 8 channels instead would group the fp32 sums
 // differently and, past 9*CX, multiply zero weights with pixels, which an
 // infinite one turns into NaN.
 template <int CX, int NT, int TR>
@@ -110,9 +112,12 @@ __global__ __launch_bounds__(256) void k_conv_lds(const float* __restrict__ X, i
 {
     constexpr int CP = (CX + 7) / 8 * 8, KP = pad_k(CX), MB = TR / 4;
     constexpr bool kWhole = CX % 8 == 0;   // a lane's 8 k lie in one tap
-    constexpr int PW = 18, PP = PW * (TR + 2), PS = CP + 8, WS = KP + 8;
+    // shorts per pixel: rows of whole 16 bytes, or the channels and a zero in an
+    // odd number of dwords (5 channels) or two (2 channels)
+    constexpr int PW = 18, PP = PW * (TR + 2), PS = kWhole ? CP + 8 : CX / 2 * 2 + 2, WS = KP + 8;
     __shared__ __align__(16) short patch[PP * PS];
     __shared__ __align__(16) short wts[NT * 16 * WS];
+    __shared__ __align__(16) short koff[kWhole ? 8 : KP];   // patch offset of every k
     const int tiles_x = (W + 15) / 16, tiles_y = (H + TR - 1) / TR;
     const int tile = blockIdx.x;
     const int b = tile / (tiles_x * tiles_y);
@@ -140,7 +145,19 @@ __global__ __launch_bounds__(256) void k_conv_lds(const float* __restrict__ X, i
     for (int i = 0; i < NI; i++) {
         const int e = (int)threadIdx.x + 256 * i;
         const int pix = e / (CP / 8), c8 = (e - pix * (CP / 8)) * 8;
-        if (e < ITEMS) *reinterpret_cast<bf16x8*>(patch + pix * PS + c8) = in[i] ? to_bf16x8(v[i]) : bf16x8{};
+        const bf16x8 q = in[i] ? to_bf16x8(v[i]) : bf16x8{};
+        if (e >= ITEMS) continue;
+        if constexpr (kWhole) *reinterpret_cast<bf16x8*>(patch + pix * PS + c8) = q;
+        else {
+            const s16x8 w = __builtin_bit_cast(s16x8, q);
+#pragma unroll
+            for (int d = 0; d < PS; d += 2) *reinterpret_cast<s16x2*>(patch + pix * PS + d) = s16x2{w[d], w[d + 1]};
+        }
+    }
+    if constexpr (!kWhole) {   // past the last tap the zero behind the channels
+        static_assert(KP <= 256, "one entry per thread");
+        const int k = threadIdx.x, tap = k / CX, c = k - tap * CX;
+        if (k < KP) koff[k] = k < 9 * CX ? sgn * ((tap / 3 - 1) * PW + (tap % 3 - 1)) * PS + c : CX;
     }
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -154,15 +171,11 @@ __global__ __launch_bounds__(256) void k_conv_lds(const float* __restrict__ X, i
 #pragma unroll
     for (int k0 = 0; k0 < KP; k0 += 32) {
         const int k = k0 + 8 * kg;
-        // patch offsets of the lane's k; past the last tap a channel that pads
-        // the pixel with zero, or zeros in its place
-        int off[kWhole ? 1 : 8];
-#pragma unroll
-        for (int j = 0; j < (kWhole ? 1 : 8); j++) {
-            const int kj = k + j, tap = kj / CX, c = kj - tap * CX;
-            off[j] = sgn * ((tap / 3 - 1) * PW + (tap % 3 - 1)) * PS + c;
-            if (kj >= 9 * CX) off[j] = kWhole ? 0 : CX;
-        }
+        // (the 16-channel layer of the test entry point has k past its taps)
+        const int tap = CX % 32 == 0 ? k0 / CX : k / CX, c = CX % 32 == 0 ? k0 % CX + 8 * kg : k % CX;
+        const int off = kWhole && k < 9 * CX ? sgn * ((tap / 3 - 1) * PW + (tap % 3 - 1)) * PS + c : 0;
+        s16x8 offs{};
+        if constexpr (!kWhole) offs = *reinterpret_cast<const s16x8*>(koff + k);
         bf16x8 w[NT];
 #pragma unroll
         for (int t = 0; t < NT; t++) w[t] = *reinterpret_cast<const bf16x8*>(wts + (t * 16 + row) * WS + k);
@@ -171,12 +184,12 @@ __global__ __launch_bounds__(256) void k_conv_lds(const float* __restrict__ X, i
             const short* p = pbase + m * PW * PS;
             bf16x8 a;
             if constexpr (kWhole) {
-                a = *reinterpret_cast<const bf16x8*>(p + off[0]);
+                a = *reinterpret_cast<const bf16x8*>(p + off);
                 if (9 * CX % 32 != 0 && k >= 9 * CX) a = bf16x8{};
             } else {
                 s16x8 v8;
 #pragma unroll
-                for (int j = 0; j < 8; j++) v8[j] = p[off[j]];
+                for (int j = 0; j < 8; j++) v8[j] = p[offs[j]];
                 a = __builtin_bit_cast(bf16x8, v8);
             }
 #pragma unroll
@@ -335,10 +348,11 @@ __global__ __launch_bounds__(256) void k_wgrad(const float* __restrict__ dY,
                     f32x8 v;
 #pragma unroll
                     for (int j = 0; j < 8; j++) v[j] = xv[i][d + j];
-                    if (xedge) {
+                    // dY past the last column: X there is zero by now but for
+                    // its left taps
+                    if (d == 0 && x0 + 8 > W) {   // uniform
 #pragma unroll
-                        for (int j = 0; j < 8; j++)
-                            if (x0 + j >= W) v[j] = 0.0f;
+                        for (int j = 1; j < 8; j++) v[j] = x0 + j < W ? v[j] : 0.0f;
                     }
                     *reinterpret_cast<bf16x8*>(&xs[d][c][pr][0]) = xin[i] ? to_bf16x8(v) : bf16x8{};
                 }
